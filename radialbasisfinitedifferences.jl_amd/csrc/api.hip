@@ -33,7 +33,7 @@ struct rbffd_buf {
 // Workspace slots of one neighbour search and the per-set buffers of a batch.
 enum ArenaSlot {
     A_PART, A_BOX, A_GRID, A_COUNTS, A_START, A_CELL_OF, A_SLOT, A_CELL_XY, A_CELL_IDX, A_CELL_GRP,
-    A_SCAN_TMP, A_STENCILS, A_STATUS, A_REDO, A_REDO_TAU, A_REDO2, A_GEN_SCRATCH, A_NSLOT
+    A_SCAN_TMP, A_STENCILS, A_STATUS, A_REDO, A_REDO_TAU, A_REDO2, A_GEN_SCRATCH, A_NS_REDO, A_NSLOT
 };
 
 struct rbffd_arena {
@@ -104,7 +104,7 @@ enum Slot {
     S_H_PTR64, S_H_ROW64, S_SCAN_TMP2, S_BATCH_FLAGS, S_MORTON_KEY, S_MORTON_IDX, S_CSC_PERM_IN, S_LSQ_ROWOF, S_LSQ_TCOL, S_LSQ_TPTR, S_LSQ_F64,
     S_LSQ_COUNT, S_LSQ_DENSE, S_LSQ_INFO, S_CLOSURE_T,
     S_CLOSURE_PART, S_GRP_COUNTS, S_GRP_YSTART, S_GRP_FILL, S_GRP_NTASK, S_GRP_TSTART, S_GRP_YLIST, S_GRP_TASKS,
-    S_GRP_TMP, S_GEN_SCRATCH, S_NSLOT
+    S_GRP_TMP, S_GEN_SCRATCH, S_NS_REDO, S_NSLOT
 };
 
 struct rbffd_context {
@@ -541,9 +541,10 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
                     const int *stencils, int n, const int *y2x, const int *rows, long nrows, int p, int polydeg,
                     int method, int nops, const int *ops, const int *opk, int precision, int *colidx,
                     double *const *vals, int *status, hipStream_t s, bool may_tune, rbffd_buf &scratch,
-                    const int **ntasks_dev = nullptr)
+                    rbffd_buf &redo_buf, const int **ntasks_dev = nullptr)
 {
     const int P = n_monomials(polydeg);
+    const bool ns = precision == RBFFD_PREC_FP64 && rbffd::ns_applies(n, polydeg, p, nops, ops);
     const int cmax = std::min(rbffd::kMaxRhs, nops);
     if (ntasks_dev) *ntasks_dev = nullptr;
     // ---- group the Y rows by their X node
@@ -555,16 +556,20 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
         fill = (int *)w.get(S_GRP_FILL, sizeof(int) * N);
         int *flag = (int *)w.get(S_FLAG, sizeof(int) * 8);
         rbffd::launch_group_count(y2x, M, N, counts, fill, s);
-        rbffd::launch_fill_i32(flag, 1, 0, s);
-        max_kernel<<<(unsigned)std::min<long>(2048, nblk(N)), 256, 0, s>>>(counts, N, flag);
-        RBFFD_HIP(hipGetLastError());
-        const int maxrows = read_flag(c, flag);
+        // the null-space kernel's tasks hold any number of rows: no need to know the largest group
+        int maxrows = rbffd::kNsRows;
+        if (!ns) {
+            rbffd::launch_fill_i32(flag, 1, 0, s);
+            max_kernel<<<(unsigned)std::min<long>(2048, nblk(N)), 256, 0, s>>>(counts, N, flag);
+            RBFFD_HIP(hipGetLastError());
+            maxrows = read_flag(c, flag);
+        }
         // calls below the tuning size keep one factorisation per X node: in
         // the specialised kernel while an X node's rows fit its 24-column
         // block, else in the generic kernel (blocks up to 72 columns)
         const bool small = M < kGroupTuneRows;
         if (grp_tuned && maxrows * cmax > rbffd::kLuGrpMaxRhs && small) grp_tuned = false;
-        ky = grp_tuned ? lu_rows_per_task(cmax, maxrows, (double)M / (double)N, small)
+        ky = ns ? rbffd::kNsRows : grp_tuned ? lu_rows_per_task(cmax, maxrows, (double)M / (double)N, small)
                        : rbffd::gen_rows_per_task(n, P, cmax, maxrows, (double)M / (double)N);
     }
     const int *grp_x = nullptr, *grp_start = nullptr, *grp_count = nullptr, *ylist = nullptr, *ntd = nullptr;
@@ -598,6 +603,7 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
         if (mem_tasks < 1) mem_tasks = 1;  // w.get reports a static array too small for one system
         mem = (double *)w.get(scratch, per * mem_tasks);
     }
+    int *redo = ns ? (int *)w.get(redo_buf, sizeof(int) * (1 + (rows ? nrows : M))) : nullptr;
     // every operator chunk, with tasks of kyv rows (1: one row per task)
     auto launch_all = [&](int kyv) {
         const bool grouped = kyv > 1;
@@ -625,7 +631,7 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
             }
             // right-hand-side columns of the generic kernel: row-major over
             // (output row of the task, operator)
-            a.gen_cols = kyv * cnt;
+            a.gen_cols = ns ? cnt : kyv * cnt;  // the null-space kernel walks its rows itself
             for (int cc = 0; cc < a.gen_cols; ++cc) {
                 const int o = cc % cnt;
                 a.col_sub[cc] = (int8_t)(cc / cnt);
@@ -649,6 +655,26 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
             a.status_accumulate = o0 > 0;
             a.max_iter = 8;
             a.tol = 4e-16;
+            if (ns) {
+                rbffd::NsArgs b{};
+                static_cast<rbffd::SolveArgs &>(b) = a;
+                b.redo = redo;
+                for (int o = 0; o < cnt; ++o)
+                    if (a.op_kind[o] == RBFFD_OP_XK || a.op_kind[o] == RBFFD_OP_YK)
+                        rbffd::ns_deriv_constants(p, a.op_k[o], b.xk_c[o]);
+                if (o0 == 0) c->last_group = 16;
+                rbffd::launch_fill_i32(redo, 1, 0, s);
+                rbffd::launch_ns(b, s);
+                // what it handed back, one row per task
+                a.grp_x = nullptr;
+                a.rows = redo + 1;
+                a.ntasks = rows ? nrows : M;
+                a.ntasks_dev = redo;
+                a.redo_pass = 1;
+                rbffd::launch_solve(a, RBFFD_PREC_FP64, s);
+                RBFFD_HIP(hipGetLastError());
+                continue;
+            }
             if (tuned && precision == RBFFD_PREC_FP64) {
                 a.group = choose_group(c, a, may_tune);
             } else if (tuned) {
@@ -672,7 +698,7 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
     // both and keeps the faster; smaller calls group.  RBFFD_GROUP_ROWS=1
     // forces grouping.
     bool group = ky > 1;
-    if (group && rbffd::solve_tuned(n, P, precision)) {
+    if (group && !ns && rbffd::solve_tuned(n, P, precision)) {
         const char *env = std::getenv("RBFFD_GROUP_ROWS");
         const bool forced = env && env[0] == '1';
         auto key = std::make_tuple(n, P, cmax, grp_tuned);
@@ -717,7 +743,7 @@ long weights_impl(rbffd_context *c, const double *X, long N, const double *Y, lo
     // the static array admits no autotuning (its events are allocations)
     return solves_enqueue(c, w, N, X, Y, M, stencils, n, y2x, rows, nrows, p, polydeg, method, nops, ops, opk,
                           precision, colidx, vals, status, c->stream, wsp == nullptr, c->bufs[S_GEN_SCRATCH],
-                          ntasks_dev);
+                          c->bufs[S_NS_REDO], ntasks_dev);
 }
 
 // group ids that restate calculateneighbors' masks (src/calculateneighbors.jl:16-42, 83-87)
@@ -1132,7 +1158,7 @@ void batch_enqueue(rbffd_context *c, const rbffd_batch_set *sets, int nsets, con
         Workspace w{c};
         w.may_alloc = !capture;
         solves_enqueue(c, w, S.N, S.X, S.X, S.N, st, S.n, nullptr, nullptr, 0, S.p, S.polydeg, 1, nops, ops, opk,
-                       RBFFD_PREC_FP64, S.colidx, S.vals, status, s, !capture, A.b[A_GEN_SCRATCH]);
+                       RBFFD_PREC_FP64, S.colidx, S.vals, status, s, !capture, A.b[A_GEN_SCRATCH], A.b[A_NS_REDO]);
         status_count_kernel<<<nblk(S.N), 256, 0, s>>>(status, S.N, f + 2);
         RBFFD_HIP(hipGetLastError());
     }

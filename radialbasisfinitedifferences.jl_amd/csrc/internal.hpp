@@ -91,6 +91,7 @@ struct SolveArgs {
     int max_iter;
     double tol;
     int group;              // lanes per stencil of the FP64 kernel (0: default)
+    int redo_pass;          // rows handed back by the null-space kernel: a small fixed grid walks them
     // ---- the generic kernel (stencil_gen.hpp): any (n, P), and output rows
     // sharing one stencil.  Tasks of several rows: task -> X node grp_x, its
     // rows ylist[grp_start .. grp_start + grp_count); NULL: one row per task.
@@ -109,6 +110,12 @@ struct SolveArgs {
     long mem_ld, mem_tasks;
 };
 
+// Arguments of the null-space kernel (stencil_ns.hpp).
+struct NsArgs : SolveArgs {
+    int *redo;               // redo[0]: rows for the pivoting kernel, which follow (at most one per output row)
+    double xk_c[kMaxRhs][7]; // constants of the pure k-th derivatives (OP_XK, OP_YK)
+};
+
 // Shapes the library solves: stencils of 1..128 nodes (the neighbour
 // search's limit) and systems of at most 512 equations.
 bool solve_supported(int n, int P);
@@ -119,6 +126,29 @@ bool solve_tuned(int n, int P, int precision);
 // several rows (a.grp_x) and shapes without a specialised kernel run the
 // generic kernel.  a.nops <= kMaxRhs.
 void launch_solve(const SolveArgs &a, int precision, hipStream_t s);
+// The null-space kernel (stencil_ns.hpp): whether it takes stencils of n nodes
+// with polynomials of degree polydeg, PHS power m and these operators, the
+// launch, and the host's constants of the pure k-th derivatives.  Stencils it
+// cannot solve are listed in a.redo for the pivoting kernel.
+bool ns_applies(int n, int polydeg, int m, int nops, const int *ops);
+void launch_ns(const NsArgs &a, hipStream_t s);
+void ns_deriv_constants(int m, int k, double *c);
+#define RBFFD_NS_SHAPES(X) X(20, 10) X(21, 10) X(31, 15)
+#define RBFFD_DECLARE_NS(nn, pp) void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s);
+RBFFD_NS_SHAPES(RBFFD_DECLARE_NS)
+#undef RBFFD_DECLARE_NS
+constexpr bool ns_shape(int n, int P)
+{
+#define RBFFD_CASE(nn, pp) \
+    if (n == nn && P == pp) return true;
+    RBFFD_NS_SHAPES(RBFFD_CASE)
+#undef RBFFD_CASE
+    return false;
+}
+// blocks of the pivoting kernel's pass over the rows handed back
+constexpr unsigned kRedoBlocks = 1024;
+// rows per grouped task of the null-space kernel
+constexpr int kNsRows = 16;
 // Compiled lane-group sizes for a shape: groups[0] default, groups[1..kMaxGroups-1]
 // alternatives or 0.
 constexpr int kMaxGroups = 3;

@@ -3,6 +3,7 @@
 // generic kernel (stencil_gen<NSB>.hip, stencil_genmem.hip) for every other
 // shape and for output rows that share a stencil.  Also the grouping of Y
 // rows by their stencil.
+#include <cmath>
 #include <cstdlib>
 #include <string>
 
@@ -43,6 +44,51 @@ bool solve_tuned(int n, int P, int precision)
     RBFFD_SHAPES(RBFFD_CASE)
 #undef RBFFD_CASE
     return false;
+}
+
+// The null-space kernel needs the form definite on the polynomials' complement:
+// odd PHS powers with polynomials of at least degree (m - 1) / 2.  Laplacian^k
+// (per-axis scales inside a double sum) stays with the pivoting kernels, and
+// so do calls that pick one of those with RBFFD_LU_GROUP, RBFFD_GROUP_ROWS=1,
+// RBFFD_TUNED_GROUPS or RBFFD_SPECIALISED=0; RBFFD_NULLSPACE=0 turns it off.
+bool ns_applies(int n, int polydeg, int m, int nops, const int *ops)
+{
+    if (!(m & 1) || polydeg < (m - 1) / 2) return false;
+    for (int o = 0; o < nops; ++o)
+        if (ops[o] < 0 || ops[o] > 8) return false;
+    const char *g = std::getenv("RBFFD_GROUP_ROWS");
+    if (env_off("RBFFD_NULLSPACE") || env_off("RBFFD_SPECIALISED") || std::getenv("RBFFD_LU_GROUP") ||
+        std::getenv("RBFFD_TUNED_GROUPS") || (g && g[0] == '1'))
+        return false;
+    const int P = (polydeg + 1) * (polydeg + 2) / 2;
+#define RBFFD_CASE(nn, pp) \
+    if (n == nn && P == pp) return true;
+    RBFFD_NS_SHAPES(RBFFD_CASE)
+#undef RBFFD_CASE
+    return false;
+}
+
+void launch_ns(const NsArgs &a, hipStream_t s)
+{
+    if (a.ntasks <= 0) return;
+#define RBFFD_CASE(nn, pp) \
+    if (a.n == nn && a.P == pp) { launch_ns_##nn##_##pp(a, s); return; }
+    RBFFD_NS_SHAPES(RBFFD_CASE)
+#undef RBFFD_CASE
+    throw Error{3, "null-space solve: no kernel for this shape"};
+}
+
+// d^k/dt^k (t^2 + y^2)^(m/2) = sum_i c[i] t^(k-2i) r^(m-2(k-i)):
+// c[i] = k! / (i! (k-2i)!) 2^(k-2i) s (s-1) .. (s-k+i+1), s = m / 2
+void ns_deriv_constants(int m, int k, double *c)
+{
+    for (int i = 0; i <= k / 2; ++i) {
+        double v = 1.0;
+        for (int j = k - 2 * i + 1; j <= k; ++j) v *= (double)j;
+        for (int j = 2; j <= i; ++j) v /= (double)j;
+        for (int j = 0; j < k - i; ++j) v *= 0.5 * (double)m - (double)j;
+        c[i] = std::ldexp(v, k - 2 * i);
+    }
 }
 
 int gen_rows_per_task(int n, int P, int nops, int maxrows, double mean_rows)

@@ -391,6 +391,21 @@ constexpr int lu_min_waves()
     return T::ROWS * T::WIDTH * 2 + head <= 168 ? 3 : 1;
 }
 
+// Lane-group sizes compiled for a stencil size: g0 is the default, the others
+// (0 = none) are candidates for the autotuner.  A lane holds ceil(n / G) row
+// slots of n + P + r doubles; a layout is compiled where those stay within
+// 200 registers at r = 3 (no spill with the rest of the kernel) and where at
+// least half of a group's lanes hold a node.  g0 is the smallest such G
+// (most stencils per wavefront), 64 when none fits.
+template <int NN, int NS>
+struct LuGroups {
+    static constexpr bool fits(int g) { return ((NN + g - 1) / g) * (NS + 3) * 2 <= 200; }
+    static constexpr bool used(int g) { return fits(g) && 2 * NN > g; }
+    static constexpr int g0 = used(16) ? 16 : (used(32) ? 32 : 64);
+    static constexpr int g1 = g0 < 32 && used(32) ? 32 : (g0 < 64 && used(64) ? 64 : 0);
+    static constexpr int g2 = g0 < 32 && g1 == 32 && used(64) ? 64 : 0;
+};
+
 // FP64 Gauss-Jordan kernel: G lanes per stencil.
 template <int NN, int NP, int R, int G>
 void launch_lu(const SolveArgs &a, hipStream_t s)
@@ -402,6 +417,13 @@ void launch_lu(const SolveArgs &a, hipStream_t s)
     constexpr int wpb = G == 16 ? 1 : lu_wpb(bytes);
     constexpr int per_block = wpb * (64 / G);
     const unsigned blocks = (unsigned)((a.ntasks + per_block - 1) / per_block);
+    if constexpr (ns_shape(NN, NP) && G == LuGroups<NN, NN + NP>::g0) {
+        if (a.redo_pass) {
+            solve_lu_kernel<NN, NP, R, G, wpb, lu_min_waves<NN, NP, R, G>(), false, true>
+                <<<blocks < kRedoBlocks ? blocks : kRedoBlocks, 64 * wpb, 0, s>>>(a);
+            return;
+        }
+    }
     solve_lu_kernel<NN, NP, R, G, wpb, lu_min_waves<NN, NP, R, G>()><<<blocks, 64 * wpb, 0, s>>>(a);
 }
 
@@ -427,21 +449,6 @@ void launch_shape_grp(const SolveArgs &a, hipStream_t s)
     else if (a.gen_cols <= 24) launch_lu_grp<NN, NP, 24>(a, s);
     else throw Error{2, "grouped tasks of at most 24 right-hand-side columns in a specialised kernel"};
 }
-
-// Lane-group sizes compiled for a stencil size: g0 is the default, the others
-// (0 = none) are candidates for the autotuner.  A lane holds ceil(n / G) row
-// slots of n + P + r doubles; a layout is compiled where those stay within
-// 200 registers at r = 3 (no spill with the rest of the kernel) and where at
-// least half of a group's lanes hold a node.  g0 is the smallest such G
-// (most stencils per wavefront), 64 when none fits.
-template <int NN, int NS>
-struct LuGroups {
-    static constexpr bool fits(int g) { return ((NN + g - 1) / g) * (NS + 3) * 2 <= 200; }
-    static constexpr bool used(int g) { return fits(g) && 2 * NN > g; }
-    static constexpr int g0 = used(16) ? 16 : (used(32) ? 32 : 64);
-    static constexpr int g1 = g0 < 32 && used(32) ? 32 : (g0 < 64 && used(64) ? 64 : 0);
-    static constexpr int g2 = g0 < 32 && g1 == 32 && used(64) ? 64 : 0;
-};
 
 template <int NN, int NP, int R>
 void launch_prec(const SolveArgs &a, int precision, hipStream_t s)

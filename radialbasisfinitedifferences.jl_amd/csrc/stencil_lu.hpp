@@ -359,27 +359,21 @@ struct LuRows {
 // output row a.col_sub[cc] of the task and operator a.col_op[cc], and every
 // column sees the same operations wherever it sits, so a row's weights are
 // those of a task of its own, bit for bit.  Else one output row per task.
-template <int NN, int NP, int R, int G, int WPB, int MINW, bool GRP = false>
-__global__ __launch_bounds__(64 * WPB, MINW) void solve_lu_kernel(const SolveArgs a)
+template <int NN, int NP, int R, int G, int WPB, bool GRP>
+__device__ __forceinline__ void solve_lu_tasks(const SolveArgs &a, long task0, long ntasks, LuLDS<NN, NP, R, G> *lds_all,
+                                               LuRows<R, 64 / G> *rows_all)
 {
     using T = LuShape<NN, NP, R, G>;
     constexpr int NS = T::NS, ROWS = T::ROWS, WIDTH = T::WIDTH, S = T::S, NODES = T::NODES;
     static_assert(NS <= 128, "system size above 128");
     static_assert(!GRP || R <= 64, "one status bit per output row of a task");
-    __shared__ LuLDS<NN, NP, R, G> lds_all[WPB];
-    __shared__ LuRows<R, S> rows_all[GRP ? WPB : 1];
-
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int grp = lane / G;
     const int t = lane % G;
     auto &L = lds_all[w];
-    long ntasks = a.ntasks;
-    if (GRP && a.ntasks_dev) ntasks = min(ntasks, (long)*a.ntasks_dev);
     // every lane of the wavefront stays until the end (shuffles span the wave);
     // a group without a task works on a copy of task 0 and stores nothing
-    const long task0 = ((long)blockIdx.x * WPB + w) * S;
-    if (task0 >= ntasks) return;  // whole wavefront
     long task = task0 + grp;
     const bool live = task < ntasks;
     if (!live) task = task0;
@@ -1002,6 +996,29 @@ __global__ __launch_bounds__(64 * WPB, MINW) void solve_lu_kernel(const SolveArg
         const int st = (sflag & 2u) ? 1 : ((sflag & 1u) ? 2 : 0);
         if (a.status_accumulate) a.status[yk] = max(a.status[yk], st);
         else a.status[yk] = st;
+    }
+}
+
+// LOOP: the tasks are the rows the null-space kernel handed back, few and of a
+// number known on the device only (a.ntasks_dev), so a small fixed grid walks
+// them.  The loop costs the other launches registers (9.8 against 6.9 ms for
+// 1M stencils of n = 31), which run one pass per wavefront.
+template <int NN, int NP, int R, int G, int WPB, int MINW, bool GRP = false, bool LOOP = false>
+__global__ __launch_bounds__(64 * WPB, MINW) void solve_lu_kernel(const SolveArgs a)
+{
+    constexpr int S = 64 / G;
+    __shared__ LuLDS<NN, NP, R, G> lds_all[WPB];
+    __shared__ LuRows<R, S> rows_all[GRP ? WPB : 1];
+    long ntasks = a.ntasks;
+    if ((GRP || LOOP) && a.ntasks_dev) ntasks = min(ntasks, (long)*a.ntasks_dev);
+    long task0 = ((long)blockIdx.x * WPB + (threadIdx.x >> 6)) * S;
+    if constexpr (LOOP) {
+        for (; task0 < ntasks; task0 += (long)gridDim.x * (WPB * S)) {
+            solve_lu_tasks<NN, NP, R, G, WPB, GRP>(a, task0, ntasks, lds_all, rows_all);
+            __builtin_amdgcn_wave_barrier();
+        }
+    } else {
+        if (task0 < ntasks) solve_lu_tasks<NN, NP, R, G, WPB, GRP>(a, task0, ntasks, lds_all, rows_all);
     }
 }
 

@@ -1,0 +1,1291 @@
+// stencil_ns.hpp -- K2, FP64 null-space path: batched local RBF-FD solves for
+// conditionally positive definite splines, 16 lanes per stencil.
+//
+// Replaces the same hot loops as stencil_lu.hpp (src/generate_operator.jl:55-65,
+// :89-166, method 3 at :388-467; src/hyperviscosity_operator.jl:66-161).
+//
+// The system  [Phi P; P^T 0] [w; lambda] = [b; p]  needs only w.  Gauss-Jordan
+// on the n x NP block P alone, with row pivoting, picks NP nodes (positions
+// 0..NP-1 from here on, the others follow) and leaves
+//     T = P2 P1^-1   (the other nodes' rows against the picked ones)
+// and P1^-1.  The weights with P^T w = p are w = (w0 - T^T y, y) with
+// w0 = P1^-T p, and with Z = [-T^T; I] the y solve the N2 x N2 system
+//     S y = Z^T (b - Phi w0),   S = Z^T Phi Z,   N2 = n - NP.
+// For r^m with m odd and degree >= (m-1)/2, S is definite, so it is inverted
+// without pivoting.  One step of refinement on the full residual b - Phi w
+// follows; the weights are then as accurate as an LU solve of the whole
+// system (both sit at the rounding of Phi itself: median 7.6e-13 against
+// 7.6e-13 at n = 31, maximum 2.6e-11 against 2.7e-11, over 1,224 stencils
+// against a 113-bit solve; without the step 1.5 to 3 times that).
+//
+// Why: the solve is bound by VALU issue.  Elimination of the whole system
+// takes n + NP dependent steps of pivot search, row publication through LDS
+// and broadcasts around its FMAs.  Here only the NP panel steps search and
+// publish (rows of NP entries); everything after them is products of small
+// matrices whose broadcasts are fused into the FMA (v_fmac_f64_dpp with
+// row_newbcast: one instruction per multiply-add, no LDS), since lane k of a
+// group holds row k.  About half the multiply-adds remain.
+//
+// Measured, 1M stencils, three operators, against the Gauss-Jordan kernel:
+// n = 31 3.41 against 6.87 ms, n = 21 2.00 against 3.97 ms; six operators at
+// n = 20 2.54 against 4.42 ms; 262,144 stencils of n = 31 with 1M output rows
+// 1.95 against 4.36 ms.  A wavefront of four stencils issues 4,880 VALU
+// instructions at n = 31 (8,440 there), on 66% of its SIMD's cycles; the rest
+// are waits on the panel's LDS round trips and on dependent steps of S^-1 that
+// two wavefronts per SIMD do not cover.  n = 13 stays with the elimination:
+// 1.16 against 1.17 ms with three operators, 1.66 against 1.33 ms with six (its
+// seven unpicked nodes fill less than half of the 16 lanes).
+//
+// What it cannot solve it hands back: a stencil with a zero panel pivot, a
+// pivot of S of the wrong sign or below kNsPivotTol of the largest, or
+// weights that are not finite goes to a list that the pivoting Gauss-Jordan
+// kernel solves afterwards (which also reports singular systems).
+//
+// A task is one stencil with the output rows that use it (one row, or the
+// grouped rows of an X node): after the factorisation each row's right-hand
+// sides are solved in chunks of RC operators.  A column sees the same
+// operations wherever it sits, so grouped and single rows get the same bits.
+#pragma once
+#include "stencil_lu.hpp"
+
+namespace rbffd {
+
+// A pivot of S below this share of the largest pivot (or of the wrong sign)
+// sends the stencil to the pivoting kernel.  Against a 113-bit solve of 14,472
+// stencils of clustered nodes, by that share: above 1e-4 the weights' error is
+// 0.87 of an LU solve's of the whole system (geometric mean), 1e-5 to 1e-4
+// 0.42, 1e-7 to 1e-6 0.05, below 1e-8 0.01; the refinement step contracts the
+// error by 1e-2 or better down to 1e-9 and no longer at 1e-10.  Jittered grids
+// reach down to 1e-4 (n = 57) and 7e-3 (n = 13), uniform random nodes to 2e-7.
+constexpr double kNsPivotTol = 9.313225746154785e-10;  // 2^-30
+
+// ---- multiply-adds with a fused broadcast: lane L of each 16-lane DPP row.
+// A DPP read needs two wait states after a VALU write of its source; the
+// compiler does not see inside the asm, so every block starts with them.
+#define RBFFD_FB(d, s, m, l) "v_fmac_f64_dpp %" #d ", %" #s ", %" #m " row_newbcast:%" #l " row_mask:0xf bank_mask:0xf\n\t"
+
+// a_i += s_i(lane L) * m
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double &a6, double &a7, double s0, double s1, double s2, double s3, double s4, double s5, double s6,
+        double s7, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 8, 16, 17) RBFFD_FB(1, 9, 16, 17) RBFFD_FB(2, 10, 16, 17) RBFFD_FB(3, 11, 16,
+            17) RBFFD_FB(4, 12, 16, 17) RBFFD_FB(5, 13, 16, 17) RBFFD_FB(6, 14, 16, 17) RBFFD_FB(7, 15, 16, 17)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(s5), "v"(s6), "v"(s7), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double &a6, double s0, double s1, double s2, double s3, double s4, double s5, double s6, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 7, 14, 15) RBFFD_FB(1, 8, 14, 15) RBFFD_FB(2, 9, 14, 15) RBFFD_FB(3, 10, 14, 15)
+            RBFFD_FB(4, 11, 14, 15) RBFFD_FB(5, 12, 14, 15) RBFFD_FB(6, 13, 14, 15)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(s5), "v"(s6), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double s0, double s1, double s2, double s3, double s4, double s5, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 6, 12, 13) RBFFD_FB(1, 7, 12, 13) RBFFD_FB(2, 8, 12, 13) RBFFD_FB(3, 9, 12, 13)
+            RBFFD_FB(4, 10, 12, 13) RBFFD_FB(5, 11, 12, 13)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(s5), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double &a3, double &a4, double s0,
+        double s1, double s2, double s3, double s4, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 5, 10, 11) RBFFD_FB(1, 6, 10, 11) RBFFD_FB(2, 7, 10, 11) RBFFD_FB(3, 8, 10, 11)
+            RBFFD_FB(4, 9, 10, 11)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double &a3, double s0, double s1,
+        double s2, double s3, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 4, 8, 9) RBFFD_FB(1, 5, 8, 9) RBFFD_FB(2, 6, 8, 9) RBFFD_FB(3, 7, 8, 9)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double &a2, double s0, double s1, double s2, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 7) RBFFD_FB(1, 4, 6, 7) RBFFD_FB(2, 5, 6, 7)
+        : "+v"(a0), "+v"(a1), "+v"(a2)
+        : "v"(s0), "v"(s1), "v"(s2), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double &a1, double s0, double s1, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 5) RBFFD_FB(1, 3, 4, 5)
+        : "+v"(a0), "+v"(a1)
+        : "v"(s0), "v"(s1), "v"(m), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_row(double &a0, double s0, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 3)
+        : "+v"(a0)
+        : "v"(s0), "v"(m), "i"(L));
+}
+// a_i += s(lane L_i) * m
+template <int L0, int L1, int L2, int L3, int L4, int L5, int L6, int L7>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double &a6, double &a7, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 8, 9, 10) RBFFD_FB(1, 8, 9, 11) RBFFD_FB(2, 8, 9, 12) RBFFD_FB(3, 8, 9, 13)
+            RBFFD_FB(4, 8, 9, 14) RBFFD_FB(5, 8, 9, 15) RBFFD_FB(6, 8, 9, 16) RBFFD_FB(7, 8, 9, 17)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2), "i"(L3), "i"(L4), "i"(L5), "i"(L6), "i"(L7));
+}
+template <int L0, int L1, int L2, int L3, int L4, int L5, int L6>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double &a6, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 7, 8, 9) RBFFD_FB(1, 7, 8, 10) RBFFD_FB(2, 7, 8, 11) RBFFD_FB(3, 7, 8, 12)
+            RBFFD_FB(4, 7, 8, 13) RBFFD_FB(5, 7, 8, 14) RBFFD_FB(6, 7, 8, 15)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2), "i"(L3), "i"(L4), "i"(L5), "i"(L6));
+}
+template <int L0, int L1, int L2, int L3, int L4, int L5>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double &a3, double &a4, double &a5,
+        double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 6, 7, 8) RBFFD_FB(1, 6, 7, 9) RBFFD_FB(2, 6, 7, 10) RBFFD_FB(3, 6, 7, 11)
+            RBFFD_FB(4, 6, 7, 12) RBFFD_FB(5, 6, 7, 13)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2), "i"(L3), "i"(L4), "i"(L5));
+}
+template <int L0, int L1, int L2, int L3, int L4>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double &a3, double &a4, double s,
+        double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 5, 6, 7) RBFFD_FB(1, 5, 6, 8) RBFFD_FB(2, 5, 6, 9) RBFFD_FB(3, 5, 6, 10)
+            RBFFD_FB(4, 5, 6, 11)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2), "i"(L3), "i"(L4));
+}
+template <int L0, int L1, int L2, int L3>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double &a3, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 4, 5, 6) RBFFD_FB(1, 4, 5, 7) RBFFD_FB(2, 4, 5, 8) RBFFD_FB(3, 4, 5, 9)
+        : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2), "i"(L3));
+}
+template <int L0, int L1, int L2>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double &a2, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 4, 5) RBFFD_FB(1, 3, 4, 6) RBFFD_FB(2, 3, 4, 7)
+        : "+v"(a0), "+v"(a1), "+v"(a2)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1), "i"(L2));
+}
+template <int L0, int L1>
+__device__ __forceinline__ void fb_lane(double &a0, double &a1, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 3, 4) RBFFD_FB(1, 2, 3, 5)
+        : "+v"(a0), "+v"(a1)
+        : "v"(s), "v"(m), "i"(L0), "i"(L1));
+}
+template <int L0>
+__device__ __forceinline__ void fb_lane(double &a0, double s, double m)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 3)
+        : "+v"(a0)
+        : "v"(s), "v"(m), "i"(L0));
+}
+// a_o += sum over i of s_o(lane L + i) * m_i, the columns interleaved
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6, double m7)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 10) RBFFD_FB(0, 1, 3, 11) RBFFD_FB(0, 1, 4, 12) RBFFD_FB(0, 1, 5, 13)
+            RBFFD_FB(0, 1, 6, 14) RBFFD_FB(0, 1, 7, 15) RBFFD_FB(0, 1, 8, 16) RBFFD_FB(0, 1, 9, 17)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "v"(m7), "i"(L), "i"(L + 1),
+                "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6), "i"(L + 7));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 9) RBFFD_FB(0, 1, 3, 10) RBFFD_FB(0, 1, 4, 11) RBFFD_FB(0, 1, 5, 12)
+            RBFFD_FB(0, 1, 6, 13) RBFFD_FB(0, 1, 7, 14) RBFFD_FB(0, 1, 8, 15)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "i"(L), "i"(L + 1), "i"(L + 2),
+                "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2,
+        double m3, double m4, double m5)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 8) RBFFD_FB(0, 1, 3, 9) RBFFD_FB(0, 1, 4, 10) RBFFD_FB(0, 1, 5, 11)
+            RBFFD_FB(0, 1, 6, 12) RBFFD_FB(0, 1, 7, 13)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "i"(L), "i"(L + 1), "i"(L + 2),
+                "i"(L + 3), "i"(L + 4), "i"(L + 5));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2,
+        double m3, double m4)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 7) RBFFD_FB(0, 1, 3, 8) RBFFD_FB(0, 1, 4, 9) RBFFD_FB(0, 1, 5, 10)
+            RBFFD_FB(0, 1, 6, 11)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "i"(L), "i"(L + 1), "i"(L + 2), "i"(L + 3),
+                "i"(L + 4));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2,
+        double m3)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 6) RBFFD_FB(0, 1, 3, 7) RBFFD_FB(0, 1, 4, 8) RBFFD_FB(0, 1, 5, 9)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "i"(L), "i"(L + 1), "i"(L + 2), "i"(L + 3));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1, double m2)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 5) RBFFD_FB(0, 1, 3, 6) RBFFD_FB(0, 1, 4, 7)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "v"(m2), "i"(L), "i"(L + 1), "i"(L + 2));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0, double m1)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 4) RBFFD_FB(0, 1, 3, 5)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "v"(m1), "i"(L), "i"(L + 1));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[1], const double (&s)[1], double m0)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 1, 2, 3)
+        : "+v"(a[0])
+        : "v"(s[0]), "v"(m0), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6, double m7)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 12) RBFFD_FB(1, 3, 4, 12) RBFFD_FB(0, 2, 5, 13) RBFFD_FB(1, 3, 5, 13)
+            RBFFD_FB(0, 2, 6, 14) RBFFD_FB(1, 3, 6, 14) RBFFD_FB(0, 2, 7, 15) RBFFD_FB(1, 3, 7, 15) RBFFD_FB(0, 2,
+            8, 16) RBFFD_FB(1, 3, 8, 16) RBFFD_FB(0, 2, 9, 17) RBFFD_FB(1, 3, 9, 17) RBFFD_FB(0, 2, 10, 18)
+            RBFFD_FB(1, 3, 10, 18) RBFFD_FB(0, 2, 11, 19) RBFFD_FB(1, 3, 11, 19)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "v"(m7), "i"(L),
+                "i"(L + 1), "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6), "i"(L + 7));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 11) RBFFD_FB(1, 3, 4, 11) RBFFD_FB(0, 2, 5, 12) RBFFD_FB(1, 3, 5, 12)
+            RBFFD_FB(0, 2, 6, 13) RBFFD_FB(1, 3, 6, 13) RBFFD_FB(0, 2, 7, 14) RBFFD_FB(1, 3, 7, 14) RBFFD_FB(0, 2,
+            8, 15) RBFFD_FB(1, 3, 8, 15) RBFFD_FB(0, 2, 9, 16) RBFFD_FB(1, 3, 9, 16) RBFFD_FB(0, 2, 10, 17)
+            RBFFD_FB(1, 3, 10, 17)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "i"(L), "i"(L + 1),
+                "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2,
+        double m3, double m4, double m5)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 10) RBFFD_FB(1, 3, 4, 10) RBFFD_FB(0, 2, 5, 11) RBFFD_FB(1, 3, 5, 11)
+            RBFFD_FB(0, 2, 6, 12) RBFFD_FB(1, 3, 6, 12) RBFFD_FB(0, 2, 7, 13) RBFFD_FB(1, 3, 7, 13) RBFFD_FB(0, 2,
+            8, 14) RBFFD_FB(1, 3, 8, 14) RBFFD_FB(0, 2, 9, 15) RBFFD_FB(1, 3, 9, 15)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "i"(L), "i"(L + 1),
+                "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2,
+        double m3, double m4)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 9) RBFFD_FB(1, 3, 4, 9) RBFFD_FB(0, 2, 5, 10) RBFFD_FB(1, 3, 5, 10)
+            RBFFD_FB(0, 2, 6, 11) RBFFD_FB(1, 3, 6, 11) RBFFD_FB(0, 2, 7, 12) RBFFD_FB(1, 3, 7, 12) RBFFD_FB(0, 2,
+            8, 13) RBFFD_FB(1, 3, 8, 13)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "i"(L), "i"(L + 1), "i"(L + 2),
+                "i"(L + 3), "i"(L + 4));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2,
+        double m3)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 8) RBFFD_FB(1, 3, 4, 8) RBFFD_FB(0, 2, 5, 9) RBFFD_FB(1, 3, 5, 9)
+            RBFFD_FB(0, 2, 6, 10) RBFFD_FB(1, 3, 6, 10) RBFFD_FB(0, 2, 7, 11) RBFFD_FB(1, 3, 7, 11)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "i"(L), "i"(L + 1), "i"(L + 2), "i"(L + 3));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1, double m2)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 7) RBFFD_FB(1, 3, 4, 7) RBFFD_FB(0, 2, 5, 8) RBFFD_FB(1, 3, 5, 8)
+            RBFFD_FB(0, 2, 6, 9) RBFFD_FB(1, 3, 6, 9)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "v"(m2), "i"(L), "i"(L + 1), "i"(L + 2));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0, double m1)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 6) RBFFD_FB(1, 3, 4, 6) RBFFD_FB(0, 2, 5, 7) RBFFD_FB(1, 3, 5, 7)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "v"(m1), "i"(L), "i"(L + 1));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[2], const double (&s)[2], double m0)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 2, 4, 5) RBFFD_FB(1, 3, 4, 5)
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(s[0]), "v"(s[1]), "v"(m0), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6, double m7)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 14) RBFFD_FB(1, 4, 6, 14) RBFFD_FB(2, 5, 6, 14) RBFFD_FB(0, 3, 7, 15)
+            RBFFD_FB(1, 4, 7, 15) RBFFD_FB(2, 5, 7, 15) RBFFD_FB(0, 3, 8, 16) RBFFD_FB(1, 4, 8, 16) RBFFD_FB(2, 5,
+            8, 16) RBFFD_FB(0, 3, 9, 17) RBFFD_FB(1, 4, 9, 17) RBFFD_FB(2, 5, 9, 17) RBFFD_FB(0, 3, 10, 18)
+            RBFFD_FB(1, 4, 10, 18) RBFFD_FB(2, 5, 10, 18) RBFFD_FB(0, 3, 11, 19) RBFFD_FB(1, 4, 11, 19) RBFFD_FB(2,
+            5, 11, 19) RBFFD_FB(0, 3, 12, 20) RBFFD_FB(1, 4, 12, 20) RBFFD_FB(2, 5, 12, 20) RBFFD_FB(0, 3, 13, 21)
+            RBFFD_FB(1, 4, 13, 21) RBFFD_FB(2, 5, 13, 21)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "v"(m7),
+                "i"(L), "i"(L + 1), "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6), "i"(L + 7));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2,
+        double m3, double m4, double m5, double m6)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 13) RBFFD_FB(1, 4, 6, 13) RBFFD_FB(2, 5, 6, 13) RBFFD_FB(0, 3, 7, 14)
+            RBFFD_FB(1, 4, 7, 14) RBFFD_FB(2, 5, 7, 14) RBFFD_FB(0, 3, 8, 15) RBFFD_FB(1, 4, 8, 15) RBFFD_FB(2, 5,
+            8, 15) RBFFD_FB(0, 3, 9, 16) RBFFD_FB(1, 4, 9, 16) RBFFD_FB(2, 5, 9, 16) RBFFD_FB(0, 3, 10, 17)
+            RBFFD_FB(1, 4, 10, 17) RBFFD_FB(2, 5, 10, 17) RBFFD_FB(0, 3, 11, 18) RBFFD_FB(1, 4, 11, 18) RBFFD_FB(2,
+            5, 11, 18) RBFFD_FB(0, 3, 12, 19) RBFFD_FB(1, 4, 12, 19) RBFFD_FB(2, 5, 12, 19)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "v"(m6), "i"(L),
+                "i"(L + 1), "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5), "i"(L + 6));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2,
+        double m3, double m4, double m5)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 12) RBFFD_FB(1, 4, 6, 12) RBFFD_FB(2, 5, 6, 12) RBFFD_FB(0, 3, 7, 13)
+            RBFFD_FB(1, 4, 7, 13) RBFFD_FB(2, 5, 7, 13) RBFFD_FB(0, 3, 8, 14) RBFFD_FB(1, 4, 8, 14) RBFFD_FB(2, 5,
+            8, 14) RBFFD_FB(0, 3, 9, 15) RBFFD_FB(1, 4, 9, 15) RBFFD_FB(2, 5, 9, 15) RBFFD_FB(0, 3, 10, 16)
+            RBFFD_FB(1, 4, 10, 16) RBFFD_FB(2, 5, 10, 16) RBFFD_FB(0, 3, 11, 17) RBFFD_FB(1, 4, 11, 17) RBFFD_FB(2,
+            5, 11, 17)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "v"(m5), "i"(L), "i"(L + 1),
+                "i"(L + 2), "i"(L + 3), "i"(L + 4), "i"(L + 5));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2,
+        double m3, double m4)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 11) RBFFD_FB(1, 4, 6, 11) RBFFD_FB(2, 5, 6, 11) RBFFD_FB(0, 3, 7, 12)
+            RBFFD_FB(1, 4, 7, 12) RBFFD_FB(2, 5, 7, 12) RBFFD_FB(0, 3, 8, 13) RBFFD_FB(1, 4, 8, 13) RBFFD_FB(2, 5,
+            8, 13) RBFFD_FB(0, 3, 9, 14) RBFFD_FB(1, 4, 9, 14) RBFFD_FB(2, 5, 9, 14) RBFFD_FB(0, 3, 10, 15)
+            RBFFD_FB(1, 4, 10, 15) RBFFD_FB(2, 5, 10, 15)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "v"(m4), "i"(L), "i"(L + 1),
+                "i"(L + 2), "i"(L + 3), "i"(L + 4));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2,
+        double m3)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 10) RBFFD_FB(1, 4, 6, 10) RBFFD_FB(2, 5, 6, 10) RBFFD_FB(0, 3, 7, 11)
+            RBFFD_FB(1, 4, 7, 11) RBFFD_FB(2, 5, 7, 11) RBFFD_FB(0, 3, 8, 12) RBFFD_FB(1, 4, 8, 12) RBFFD_FB(2, 5,
+            8, 12) RBFFD_FB(0, 3, 9, 13) RBFFD_FB(1, 4, 9, 13) RBFFD_FB(2, 5, 9, 13)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "v"(m3), "i"(L), "i"(L + 1), "i"(L + 2),
+                "i"(L + 3));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1, double m2)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 9) RBFFD_FB(1, 4, 6, 9) RBFFD_FB(2, 5, 6, 9) RBFFD_FB(0, 3, 7, 10)
+            RBFFD_FB(1, 4, 7, 10) RBFFD_FB(2, 5, 7, 10) RBFFD_FB(0, 3, 8, 11) RBFFD_FB(1, 4, 8, 11) RBFFD_FB(2, 5,
+            8, 11)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "v"(m2), "i"(L), "i"(L + 1), "i"(L + 2));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0, double m1)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 8) RBFFD_FB(1, 4, 6, 8) RBFFD_FB(2, 5, 6, 8) RBFFD_FB(0, 3, 7, 9)
+            RBFFD_FB(1, 4, 7, 9) RBFFD_FB(2, 5, 7, 9)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "v"(m1), "i"(L), "i"(L + 1));
+}
+template <int L>
+__device__ __forceinline__ void fb_dot(double (&a)[3], const double (&s)[3], double m0)
+{
+    asm("s_nop 1\n\t" RBFFD_FB(0, 3, 6, 7) RBFFD_FB(1, 4, 6, 7) RBFFD_FB(2, 5, 6, 7)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2])
+        : "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(m0), "i"(L));
+}
+
+// a[j] += s[j](lane L) * m for CNT columns j = J, J + 1, ... (mod W)
+template <int L, int J, int CNT, int W>
+__device__ __forceinline__ void fb_cols(double (&a)[W], const double (&s)[W], double m)
+{
+    if constexpr (CNT > 8) {
+        fb_cols<L, J, 8>(a, s, m);
+        fb_cols<L, J + 8, CNT - 8>(a, s, m);
+    } else if constexpr (CNT == 8)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], a[(J + 3) % W], a[(J + 4) % W], a[(J + 5) % W],
+                a[(J + 6) % W], a[(J + 7) % W], s[(J + 0) % W], s[(J + 1) % W], s[(J + 2) % W], s[(J + 3) % W],
+                s[(J + 4) % W], s[(J + 5) % W], s[(J + 6) % W], s[(J + 7) % W], m);
+    else if constexpr (CNT == 7)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], a[(J + 3) % W], a[(J + 4) % W], a[(J + 5) % W],
+                a[(J + 6) % W], s[(J + 0) % W], s[(J + 1) % W], s[(J + 2) % W], s[(J + 3) % W], s[(J + 4) % W],
+                s[(J + 5) % W], s[(J + 6) % W], m);
+    else if constexpr (CNT == 6)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], a[(J + 3) % W], a[(J + 4) % W], a[(J + 5) % W],
+                s[(J + 0) % W], s[(J + 1) % W], s[(J + 2) % W], s[(J + 3) % W], s[(J + 4) % W], s[(J + 5) % W], m);
+    else if constexpr (CNT == 5)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], a[(J + 3) % W], a[(J + 4) % W], s[(J + 0) % W],
+                s[(J + 1) % W], s[(J + 2) % W], s[(J + 3) % W], s[(J + 4) % W], m);
+    else if constexpr (CNT == 4)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], a[(J + 3) % W], s[(J + 0) % W], s[(J + 1) % W],
+                s[(J + 2) % W], s[(J + 3) % W], m);
+    else if constexpr (CNT == 3)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], a[(J + 2) % W], s[(J + 0) % W], s[(J + 1) % W], s[(J + 2) % W], m);
+    else if constexpr (CNT == 2)
+        fb_row<L>(a[(J + 0) % W], a[(J + 1) % W], s[(J + 0) % W], s[(J + 1) % W], m);
+    else if constexpr (CNT == 1)
+        fb_row<L>(a[(J + 0) % W], s[(J + 0) % W], m);
+}
+// a[j] += s[j / 16](lane j % 16) * m for CNT columns j = J, J + 1, ... (mod W);
+// one asm block stays inside one 16-column slot of s
+template <int J, int CNT, int W, int NB>
+__device__ __forceinline__ void fb_lanes(double (&a)[W], const double (&s)[NB], double m)
+{
+    if constexpr (CNT > 0) {
+        constexpr int j0 = J % W, sl = j0 / 16;
+        // columns up to the next slot or the wrap (with one slot the wrap may sit inside a block)
+        constexpr int room = NB == 1 ? CNT : ((16 * sl + 16 < W ? 16 * sl + 16 : W) - j0);
+        constexpr int run = CNT < room ? CNT : room;
+        constexpr int n = run < 8 ? run : 8;
+#define RBFFD_L(i) (((J + i) % W) % 16)
+#define RBFFD_A(i) a[(J + i) % W]
+        if constexpr (n == 8)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2), RBFFD_L(3), RBFFD_L(4), RBFFD_L(5), RBFFD_L(6),
+                    RBFFD_L(7)>(RBFFD_A(0), RBFFD_A(1), RBFFD_A(2), RBFFD_A(3), RBFFD_A(4), RBFFD_A(5), RBFFD_A(6),
+                    RBFFD_A(7), s[sl], m);
+        else if constexpr (n == 7)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2), RBFFD_L(3), RBFFD_L(4), RBFFD_L(5), RBFFD_L(6)>(RBFFD_A(0),
+                    RBFFD_A(1), RBFFD_A(2), RBFFD_A(3), RBFFD_A(4), RBFFD_A(5), RBFFD_A(6), s[sl], m);
+        else if constexpr (n == 6)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2), RBFFD_L(3), RBFFD_L(4), RBFFD_L(5)>(RBFFD_A(0), RBFFD_A(1),
+                    RBFFD_A(2), RBFFD_A(3), RBFFD_A(4), RBFFD_A(5), s[sl], m);
+        else if constexpr (n == 5)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2), RBFFD_L(3), RBFFD_L(4)>(RBFFD_A(0), RBFFD_A(1), RBFFD_A(2),
+                    RBFFD_A(3), RBFFD_A(4), s[sl], m);
+        else if constexpr (n == 4)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2), RBFFD_L(3)>(RBFFD_A(0), RBFFD_A(1), RBFFD_A(2), RBFFD_A(3),
+                    s[sl], m);
+        else if constexpr (n == 3)
+            fb_lane<RBFFD_L(0), RBFFD_L(1), RBFFD_L(2)>(RBFFD_A(0), RBFFD_A(1), RBFFD_A(2), s[sl], m);
+        else if constexpr (n == 2)
+            fb_lane<RBFFD_L(0), RBFFD_L(1)>(RBFFD_A(0), RBFFD_A(1), s[sl], m);
+        else if constexpr (n == 1)
+            fb_lane<RBFFD_L(0)>(RBFFD_A(0), s[sl], m);
+#undef RBFFD_L
+#undef RBFFD_A
+        fb_lanes<J + n, CNT - n>(a, s, m);
+    }
+}
+// a[o] += sum over k in K0..K1-1 of s[k / 16][o](lane k % 16) * m[k]
+template <int K0, int K1, int RC, int NB, int W>
+__device__ __forceinline__ void fb_sum(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
+{
+    if constexpr (K1 > K0) {
+        constexpr int sl = K0 / 16, l = K0 % 16;
+        constexpr int run = K1 - K0 < 16 - l ? K1 - K0 : 16 - l;
+        constexpr int n = run < 8 ? run : 8;
+        if constexpr (n == 8)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2], m[K0 + 3], m[K0 + 4], m[K0 + 5], m[K0 + 6], m[K0 + 7]);
+        else if constexpr (n == 7)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2], m[K0 + 3], m[K0 + 4], m[K0 + 5], m[K0 + 6]);
+        else if constexpr (n == 6)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2], m[K0 + 3], m[K0 + 4], m[K0 + 5]);
+        else if constexpr (n == 5)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2], m[K0 + 3], m[K0 + 4]);
+        else if constexpr (n == 4)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2], m[K0 + 3]);
+        else if constexpr (n == 3)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1], m[K0 + 2]);
+        else if constexpr (n == 2)
+            fb_dot<l>(a, s[sl], m[K0], m[K0 + 1]);
+        else if constexpr (n == 1)
+            fb_dot<l>(a, s[sl], m[K0]);
+        fb_sum<K0 + n, K1>(a, s, m);
+    }
+}
+
+__device__ __forceinline__ uint32_t lds_address(const void *p)
+{
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+
+// Two doubles to slots I and J of a row in LDS.  Written out because the
+// compiler makes ds_write_b128 of neighbouring stores, whose data must first be
+// moved into four consecutive registers (382 moves in the panel at n = 31);
+// this takes each from where it is.  A store needs no wait of its own: LDS
+// serves a wavefront in order, and the compiler's counts for the reads behind
+// it only get more cautious.
+template <int I, int J>
+__device__ __forceinline__ void lds_write2(uint32_t a, double x, double y)
+{
+    asm volatile("ds_write2_b64 %0, %1, %2 offset0:%3 offset1:%4" ::"v"(a), "v"(x), "v"(y), "i"(I), "i"(J) : "memory");
+}
+
+// v with its high word replaced by hi where c holds
+__device__ __forceinline__ double hi_if(double v, bool c, uint32_t hi)
+{
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t h = c ? hi : (uint32_t)(b >> 32);
+    return __longlong_as_double((long long)(((uint64_t)h << 32) | (uint32_t)b));
+}
+
+// whether row slot S of this lane, t + 16 S, is at most c
+template <int S>
+__device__ __forceinline__ bool upto(int c)
+{
+    const int e = c - 16 * S;
+    const uint64_t m = e < 0 ? 0ull : (e >= 15 ? 0xFFFFull : (2ull << e) - 1ull);
+    return __builtin_amdgcn_inverse_ballot_w64(m * 0x0001000100010001ull);
+}
+
+// 1 / x to within an ulp (x finite and not zero): the instruction gives 23
+// bits, one cubic step the rest
+__device__ __forceinline__ double rcp_nr(double x)
+{
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+
+// sqrt(x) for x >= 2^-700 by the correction steps the compiler uses, without
+// its scaling of smaller arguments (7 instructions fewer); x = 0 gives NaN, so
+// a duplicated node fails the finiteness check
+__device__ __forceinline__ double ns_sqrt(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(g, r, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// Powers of r = |v| at one point for the closed-form operators.
+struct NsPhsAt {
+    double r2, r, rm2, rm4;  // r^2, r, r^(m-2), r^(m-4)
+};
+
+__device__ __forceinline__ NsPhsAt ns_phs_at(int m, double vx, double vy)
+{
+    NsPhsAt q;
+    q.r2 = sq_sum(vx, vy);
+    q.r = ns_sqrt(q.r2);
+    if (m >= 5) {  // uniform
+        q.rm4 = upow(q.r2, (m - 5) >> 1) * q.r;
+        q.rm2 = q.rm4 * q.r2;
+    } else {
+        q.rm2 = m == 3 ? q.r : q.r / q.r2;
+        q.rm4 = q.rm2 / q.r2;
+    }
+    return q;
+}
+
+// Operator applied to the PHS (m odd): closed forms; for the pure k-th
+// derivatives the chain rule over t -> t^2 + const,
+//   t^(k mod 2) r^(m-2k) sum_i c[i] (t^2)^(h-i) (r^2)^i,   h = k / 2,
+// with the constants c precomputed by the host.
+template <class C>
+__device__ __forceinline__ double ns_op_phs(int op, int k, int m, const C &c, double vx, double vy, double sx,
+                                            double sy, const NsPhsAt &q)
+{
+    // no contraction: a column's bits do not depend on the code around it
+#pragma clang fp contract(off)
+    if (op == OP_E) return upow(q.r2, m >> 1) * q.r;
+    const double dm = (double)m;
+    switch (op) {
+    case OP_DX:  return dm * vx * q.rm2;
+    case OP_DY:  return dm * vy * q.rm2;
+    case OP_DXX: return dm * q.rm2 + dm * (dm - 2.0) * vx * vx * q.rm4;
+    case OP_DYY: return dm * q.rm2 + dm * (dm - 2.0) * vy * vy * q.rm4;
+    case OP_DXY: return dm * (dm - 2.0) * vx * vy * q.rm4;
+    case OP_LAP: {
+        const double fxx = dm * q.rm2 + dm * (dm - 2.0) * vx * vx * q.rm4;
+        const double fyy = dm * q.rm2 + dm * (dm - 2.0) * vy * vy * q.rm4;
+        return sx * sx * fxx + sy * sy * fyy;
+    }
+    default: {  // OP_XK, OP_YK
+        const double t = op == OP_XK ? vx : vy;
+        const double t2 = t * t;
+        double s = c[0], rp = 1.0;
+        for (int i = 1; i <= (k >> 1); ++i) {
+            rp *= q.r2;
+            s = s * t2 + c[i] * rp;
+        }
+        if (k & 1) s *= t;
+        const int e = m - 2 * k;  // odd
+        return e > 0 ? s * (upow(q.r2, e >> 1) * q.r) : s * (q.r / upow(q.r2, (1 - e) >> 1));
+    }
+    }
+}
+
+// x^e for a per-lane exponent 0 <= e < 8
+__device__ __forceinline__ double lpow(double x, int e)
+{
+    double p = e & 1 ? x : 1.0;
+    x *= x;
+    p = e & 2 ? p * x : p;
+    x *= x;
+    return e & 4 ? p * x : p;
+}
+
+// d^a/dx^a d^b/dy^b of x^ea y^eb (a, b uniform, the exponents per lane)
+__device__ __forceinline__ double ns_mono(int ea, int eb, int a, int b, double x, double y)
+{
+#pragma clang fp contract(off)
+    double c = 1.0;
+    for (int t = 0; t < a; ++t) c *= (double)(ea - t);  // zero once a > ea
+    for (int t = 0; t < b; ++t) c *= (double)(eb - t);
+    return c * (lpow(x, max(ea - a, 0)) * lpow(y, max(eb - b, 0)));
+}
+
+__device__ __forceinline__ double ns_op_mono(int op, int k, int ea, int eb, double x, double y, double sx, double sy)
+{
+#pragma clang fp contract(off)
+    if (op == OP_LAP) return sx * sx * ns_mono(ea, eb, 2, 0, x, y) + sy * sy * ns_mono(ea, eb, 0, 2, x, y);
+    int a = 0, b = 0;
+    switch (op) {
+    case OP_DX: a = 1; break;
+    case OP_DY: b = 1; break;
+    case OP_DXX: a = 2; break;
+    case OP_DYY: b = 2; break;
+    case OP_DXY: a = 1; b = 1; break;
+    case OP_XK: a = k; break;
+    case OP_YK: b = k; break;
+    default: break;
+    }
+    return ns_mono(ea, eb, a, b, x, y);
+}
+
+template <int NN, int NP>
+struct NsShape {
+    static constexpr int N2 = NN - NP;
+    static constexpr int NB1 = (NP + 15) / 16, NB2 = (N2 + 15) / 16;  // row slots of the two node sets
+    static constexpr int NODES = (NN + 15) / 16;
+    static constexpr int TS = NP | 1;  // row stride of the panel's result: odd, so a column read has no bank conflicts
+    // Phi by position: the picked nodes' upper triangle, the NP x N2 block, the others' upper triangle
+    // (rows of the block an odd stride apart: its rows are read across lanes too)
+    static constexpr int WS = N2 | 1;
+    static constexpr int F11 = 0, F12 = NP * (NP + 1) / 2, F22 = F12 + NP * WS;
+    static constexpr int PHI = F22 + N2 * (N2 + 1) / 2;
+    static constexpr int RPS = cmax_<PHI, NN * TS>::v;  // reciprocal pivots of S, behind Phi
+    // per group: 16 modulo 32 doubles, so two groups' odd-stride reads fall on all 64 banks
+    static constexpr int U = (RPS + N2 + 15) / 32 * 32 + 16;
+    static constexpr __host__ __device__ int tri(int w, int a) { return a * (2 * w - a + 1) / 2 - a; }
+};
+
+template <int NN, int NP>
+struct alignas(16) NsLDS {
+    using T = NsShape<NN, NP>;
+    double u[4][T::U];      // the panel's pivot row, then P1^-1 and T, then Phi
+    double xi[4][2 * NN];   // scaled coordinates by position
+    double frame[4][4];     // centre and scales
+    int g[4][NN], rank[4][NN];  // global index and output column by position
+};
+
+// Wavefronts per SIMD the kernel is compiled for.  n = 31: LDS (20 KB a
+// wavefront) and the row registers hold it to two.  n = 20 and 21: three, with
+// 30 registers spilled, take 2.00 ms per 1M stencils of n = 21 where two
+// without spills take 2.29 ms.
+template <int NN, int NP>
+constexpr int ns_min_waves()
+{
+    return NN <= 21 ? 3 : 2;
+}
+
+template <int NN, int NP, int RC>
+__global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(const NsArgs a)
+{
+    using T = NsShape<NN, NP>;
+    constexpr int N2 = T::N2, NB1 = T::NB1, NB2 = T::NB2, NODES = T::NODES;
+    constexpr int DEG = mono_deg(NP - 1);
+    __shared__ NsLDS<NN, NP> L;
+    const int lane = threadIdx.x & 63, grp = lane >> 4, t = lane & 15;
+    double *const U = L.u[grp];
+    const bool grouped = a.grp_x != nullptr;
+    long ntasks = a.ntasks;
+    if (a.ntasks_dev) ntasks = min(ntasks, (long)*a.ntasks_dev);
+    const long task0 = (long)blockIdx.x * 4;
+    if (task0 >= ntasks) return;  // whole wavefront
+    // a group without a task works on a copy of the first and stores nothing
+    const bool live = task0 + grp < ntasks;
+    const long task = live ? task0 + grp : task0;
+    long xs;
+    int yk, ybase = 0, ny = 1;
+    if (grouped) {
+        xs = a.grp_x[task];
+        ybase = a.grp_start[task];
+        ny = a.grp_count[task];
+        yk = a.ylist[ybase];
+    } else {
+        yk = a.rows ? a.rows[task] : (int)task;
+        xs = a.y2x ? a.y2x[yk] : yk;
+    }
+    const int m = a.m;
+    const bool m3 = a.method == 3;
+
+    // ---- stencil frame (src/scalestencil.jl:10-21, src/generate_operator.jl:100-134)
+    double C[NODES][NP];  // this lane's rows of P: nodes t + 16 r
+    uint32_t alive[NODES];
+    double sx = 1.0, sy = 1.0, cx, cy;
+    double nx[NODES], nyy[NODES];
+    int gid[NODES], rk[NODES];
+    {
+#pragma clang fp contract(off)
+        const int c = max(a.stencils[xs * NN], 0);  // a failed search leaves -1: every read stays in X
+        cx = a.X[2 * (long)c];
+        cy = a.X[2 * (long)c + 1];
+        double mx = 0.0, my = 0.0;
+        int *gl = reinterpret_cast<int *>(U);
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            const int i = t + 16 * r;
+            gid[r] = i < NN ? max(a.stencils[xs * NN + i], 0) : c;
+            if (i < NN) gl[i] = gid[r];
+            nx[r] = a.X[2 * (long)gid[r]] - cx;
+            nyy[r] = a.X[2 * (long)gid[r] + 1] - cy;
+            mx = fmax(mx, __builtin_fabs(nx[r]));
+            my = fmax(my, __builtin_fabs(nyy[r]));
+        }
+        if (!m3) {
+            mx = group_max_nonneg_f64<16>(mx);
+            my = group_max_nonneg_f64<16>(my);
+            sx = 1.0 / mx;
+            sy = 1.0 / my;
+        }
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            // method 3 leaves the frame unscaled, its centre at (eps, eps) (src/generate_operator.jl:393-410)
+            nx[r] = m3 ? (t + 16 * r == 0 ? kEps : nx[r]) : nx[r] * sx;
+            nyy[r] = m3 ? (t + 16 * r == 0 ? kEps : nyy[r]) : nyy[r] * sy;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // the output column of each node: the rank of its global index inside the stencil
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) rk[r] = 0;
+#pragma unroll
+        for (int j = 0; j < NN; ++j) {
+            const int gj = gl[j];
+#pragma unroll
+            for (int r = 0; r < NODES; ++r) rk[r] += gj < gid[r] ? 1 : 0;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    if (t == 0) {
+        L.frame[grp][0] = cx;
+        L.frame[grp][1] = cy;
+        L.frame[grp][2] = sx;
+        L.frame[grp][3] = sy;
+    }
+
+    // ---- the panel: in-place Gauss-Jordan of P with row pivoting.  Rows keep
+    // their scale (a picked row is multiplied by its reciprocal pivot at the
+    // end); column k becomes the inverse's once step k is done.
+#pragma unroll
+    for (int r = 0; r < NODES; ++r) {
+        double px[DEG + 1], py[DEG + 1];
+        px[0] = py[0] = 1.0;
+#pragma unroll
+        for (int d = 1; d <= DEG; ++d) { px[d] = px[d - 1] * nx[r]; py[d] = py[d - 1] * nyy[r]; }
+        alive[r] = t + 16 * r < NN ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) C[r][q] = px[mono_ea(q)] * py[mono_eb(q)];
+    }
+    int pos[NODES];
+    double fin[NODES];
+#pragma unroll
+    for (int r = 0; r < NODES; ++r) { pos[r] = 0; fin[r] = 1.0; }
+    uint32_t weakest = 0xFFFFFFFFu;
+    const uint32_t ua = lds_address(U);
+    for_blocks<0, NP>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        // pivot search: the largest |C[.][k]| among rows not yet picked, as a
+        // key whose low 7 bits name the node
+        uint32_t key = 0;
+        double cv = C[0][k];
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            const uint32_t kr = ((__float_as_uint((float)C[r][k]) & 0x7FFFFF00u) |
+                                 (0x80u | (uint32_t)(127 - (t + 16 * r)))) & alive[r];
+            if (r == 0) {
+                key = kr;
+            } else if (kr > key) {
+                key = kr;
+                cv = C[r][k];
+            }
+        }
+        const double crp = rcp_nr(cv);
+        key = group_max_u32<16>(key);
+        weakest = min(weakest, key);
+        const int v = 127 - (int)(key & 127u);
+        const bool iam = t == (v & 15);
+        // the picked row goes to the group, its reciprocal pivot in the pivot's place
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            if (iam && (v >> 4) == r) {
+                for_blocks<0, NP / 2>([&](auto jc) {
+                    constexpr int j = 2 * decltype(jc)::value;
+                    lds_write2<j, j + 1>(ua, j == k ? crp : C[r][j], j + 1 == k ? crp : C[r][j + 1]);
+                });
+                if constexpr (NP % 2) U[NP - 1] = NP - 1 == k ? crp : C[r][NP - 1];
+                alive[r] = 0u;
+                pos[r] = k;
+                fin[r] = crp;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        double pr[NB1];
+#pragma unroll
+        for (int b = 0; b < NB1; ++b) pr[b] = U[t + 16 * b];
+        const double rp = row_bcast64<k % 16>(pr[k / 16]);
+        double l[NODES];
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            const bool me = iam && (v >> 4) == r;
+            // the picked row's multiplier: its high word zeroed leaves a value below 2^-1022, which the additions lose
+            l[r] = hi_if(-(C[r][k] * rp), me, 0u);
+            C[r][k] = me ? 1.0 : l[r];
+            // the next step's column first
+            if constexpr (k + 1 < NP) fb_lanes<k + 1, 1>(C[r], pr, l[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < NODES; ++r)
+            fb_lanes<(k + 1 < NP ? k + 2 : k + 1) % NP, NP - 1 - (k + 1 < NP)>(C[r], pr, l[r]);
+        __builtin_amdgcn_wave_barrier();
+    });
+    // positions of the rows that were not picked: slot by slot, lane by lane
+    {
+        int base = NP;
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            const bool fr = alive[r] != 0u;
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(fr);
+            const uint32_t gm = (uint32_t)(bal >> (grp * 16)) & 0xFFFFu;
+            if (fr) pos[r] = base + __builtin_popcount(gm & ((1u << t) - 1u));
+            base += __builtin_popcount(gm);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < NODES; ++r) {
+        if (t + 16 * r < NN) {
+#pragma unroll
+            for (int j = 0; j < NP; ++j) U[pos[r] * T::TS + j] = C[r][j] * fin[r];
+            L.xi[grp][2 * pos[r]] = nx[r];
+            L.xi[grp][2 * pos[r] + 1] = nyy[r];
+            L.g[grp][pos[r]] = gid[r];
+            L.rank[grp][pos[r]] = rk[r];
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    // this lane's rows from here on: picked nodes kb[s] = t + 16 s, others
+    // qa[s] = t + 16 s (lanes past the end repeat the last row and store nothing)
+    int kb[NB1], qa[NB2];
+    double xb[NB1], yb[NB1], xa[NB2], ya[NB2];
+    double nT[NB2][NP];   // -T, row qa
+    double nTt[NB1][N2];  // -T, column kb
+    double Pit[NB1][NP];  // P1^-1, column kb
+#pragma unroll
+    for (int s = 0; s < NB1; ++s) {
+        kb[s] = min(t + 16 * s, NP - 1);
+        xb[s] = L.xi[grp][2 * kb[s]];
+        yb[s] = L.xi[grp][2 * kb[s] + 1];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) Pit[s][k] = U[k * T::TS + kb[s]];
+#pragma unroll
+        for (int i = 0; i < N2; ++i) nTt[s][i] = U[(NP + i) * T::TS + kb[s]];
+    }
+#pragma unroll
+    for (int s = 0; s < NB2; ++s) {
+        qa[s] = min(t + 16 * s, N2 - 1);
+        xa[s] = L.xi[grp][2 * (NP + qa[s])];
+        ya[s] = L.xi[grp][2 * (NP + qa[s]) + 1];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) nT[s][k] = U[(NP + qa[s]) * T::TS + k];
+    }
+    __builtin_amdgcn_wave_barrier();
+
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- Phi by position, each pair once
+    {
+        auto pairs = [&](auto mc) {
+            constexpr int MC = decltype(mc)::value;
+            const int mm = MC > 0 ? MC : m;
+            auto phs = [&](double x0, double y0, int p) {
+                const double dx = x0 - L.xi[grp][2 * p], dy = y0 - L.xi[grp][2 * p + 1];
+                const double r2 = sq_sum(dx, dy);
+                return upow(r2, mm >> 1) * ns_sqrt(r2);
+            };
+#pragma unroll
+            for (int s = 0; s < NB2; ++s) {
+                if (t + 16 * s < N2) {
+#pragma unroll 3
+                    for (int k = 0; k < NP; ++k) U[T::F12 + k * T::WS + qa[s]] = phs(xa[s], ya[s], k);
+                    U[T::F22 + T::tri(N2, qa[s]) + qa[s]] = 0.0;
+#pragma unroll 2
+                    for (int d = 1; d <= N2 / 2; ++d) {
+                        int j = qa[s] + d;
+                        if (j >= N2) j -= N2;
+                        U[T::F22 + T::tri(N2, min(qa[s], j)) + max(qa[s], j)] = phs(xa[s], ya[s], NP + j);
+                    }
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < NB1; ++s) {
+                if (t + 16 * s < NP) {
+                    U[T::F11 + T::tri(NP, kb[s]) + kb[s]] = 0.0;
+#pragma unroll 2
+                    for (int d = 1; d <= NP / 2; ++d) {
+                        int j = kb[s] + d;
+                        if (j >= NP) j -= NP;
+                        U[T::F11 + T::tri(NP, min(kb[s], j)) + max(kb[s], j)] = phs(xb[s], yb[s], j);
+                    }
+                }
+            }
+        };
+        switch (m) {
+        case 3: pairs(std::integral_constant<int, 3>{}); break;
+        case 5: pairs(std::integral_constant<int, 5>{}); break;
+        case 7: pairs(std::integral_constant<int, 7>{}); break;
+        case 9: pairs(std::integral_constant<int, 9>{}); break;
+        default: pairs(std::integral_constant<int, 0>{}); break;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    // Phi(picked row kb, picked column c), Phi(kb, other j), Phi(other row qa, picked c), Phi(qa, other j)
+    // the two triangles: one addition and a select per entry, by lane masks known at compile time
+    auto f11 = [&](int k, auto sc, auto cc) {
+        constexpr int s = decltype(sc)::value, c = decltype(cc)::value;
+        const int up = T::F11 + T::tri(NP, k), lo = k + (T::F11 + T::tri(NP, c) - c);
+        return U[(upto<s>(c) ? up : lo) + c];
+    };
+    auto f12 = [&](int k, int j) { return U[T::F12 + k * T::WS + j]; };
+    auto f21 = [&](int q, int c) { return U[T::F12 + c * T::WS + q]; };
+    auto f22 = [&](int q, auto sc, auto jc) {
+        constexpr int s = decltype(sc)::value, j = decltype(jc)::value;
+        const int up = T::F22 + T::tri(N2, q), lo = q + (T::F22 + T::tri(N2, j) - j);
+        return U[(upto<s>(j) ? up : lo) + j];
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- S = Phi22 - T Phi12 - (Phi21 - T Phi11) T^T, one row per lane slot
+    double S[NB2][N2];
+    {
+        double V[NB2][NP], B[NB1][NP];
+        for_blocks<0, NB1>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            for_blocks<0, NP>([&](auto cc) { B[s][decltype(cc)::value] = f11(kb[s], sc, cc); });
+        });
+#pragma unroll
+        for (int s = 0; s < NB2; ++s) {
+#pragma unroll
+            for (int c = 0; c < NP; ++c) V[s][c] = f21(qa[s], c);
+            for_blocks<0, NP>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                fb_cols<k % 16, 0, NP>(V[s], B[k / 16], nT[s][k]);
+            });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        for_blocks<0, NB2>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            for_blocks<0, N2>([&](auto jc) { S[s][decltype(jc)::value] = f22(qa[s], sc, jc); });
+        });
+        // + V (-T)^T: column c of -T, over the lanes of the other nodes
+        for_blocks<0, NP>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            double tc[NB2];
+#pragma unroll
+            for (int s = 0; s < NB2; ++s) tc[s] = nT[s][c];
+#pragma unroll
+            for (int s = 0; s < NB2; ++s) fb_lanes<0, N2>(S[s], tc, V[s][c]);
+        });
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        double B[NB1][N2];
+#pragma unroll
+        for (int s = 0; s < NB1; ++s)
+#pragma unroll
+            for (int j = 0; j < N2; ++j) B[s][j] = f12(kb[s], j);
+#pragma unroll
+        for (int s = 0; s < NB2; ++s)
+            for_blocks<0, NP>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                fb_cols<k % 16, 0, N2>(S[s], B[k / 16], nT[s][k]);
+            });
+    }
+
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- S^-1 in place without pivoting (S is definite); row q stays scaled
+    // by its pivot, whose reciprocal (rps) multiplies the products
+    for_blocks<0, N2>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const double p = row_bcast64<k % 16>(S[k / 16][k]);
+        const double rp = rcp_nr(p);
+        U[T::RPS + k] = rp;  // the same value from every lane of the group
+        double l[NB2];
+#pragma unroll
+        for (int s = 0; s < NB2; ++s) {
+            const bool me = s == k / 16 && __builtin_amdgcn_inverse_ballot_w64(0x0001000100010001ull << (k % 16));
+            l[s] = hi_if(-(S[s][k] * rp), me, 0u);
+            S[s][k] = me ? 1.0 : l[s];
+        }
+#pragma unroll
+        for (int s = 0; s < NB2; ++s)
+            if constexpr (k + 1 < N2) fb_cols<k % 16, k + 1, 1>(S[s], S[k / 16], l[s]);
+#pragma unroll
+        for (int s = 0; s < NB2; ++s)
+            fb_cols<k % 16, (k + 1 < N2 ? k + 2 : k + 1) % N2, N2 - 1 - (k + 1 < N2)>(S[s], S[k / 16], l[s]);
+    });
+    // pivots: the reciprocals' extremes over the group
+    double rps[NB2], rmin = 1e300, rmax = -1e300;
+    const double sgn = ((m + 1) >> 1) & 1 ? -1.0 : 1.0;  // sign of the definite form, (-1)^((m+1)/2)
+#pragma unroll
+    for (int s = 0; s < NB2; ++s) {
+        rps[s] = U[T::RPS + qa[s]];
+        rmin = fmin(rmin, sgn * rps[s]);
+        rmax = fmax(rmax, sgn * rps[s]);
+    }
+    // a wrong sign makes rmin negative, a NaN fails the finiteness check of the weights
+    const bool definite = !(rmin <= 0.0);
+    rmax = group_max_nonneg_f64<16>(fmax(rmax, 0.0));
+    const double imax = group_max_nonneg_f64<16>(definite ? 1.0 / rmin : 1e300);
+    __builtin_amdgcn_sched_barrier(0);
+    // the smallest pivot is 1 / rmax, the largest imax
+    bool bad = (weakest & 0x7FFFFF00u) == 0u || !definite || !(kNsPivotTol * imax * rmax < 1.0);
+
+    // ---- the rows' right-hand sides, RC operators at a time
+    double gx = a.Y[2 * (long)yk], gy = a.Y[2 * (long)yk + 1];
+    for (int sub = 0;; ++sub) {
+        const bool on = live && sub < ny;
+        if (!__builtin_amdgcn_ballot_w64(sub < ny)) break;
+        const long row = yk;
+        // the arguments are read again for each row: held over the loop they
+        // outgrow the scalar registers
+        auto *ap = (const __attribute__((address_space(4))) NsArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(ap));
+        int fo = 0;
+        asm volatile("" : "+v"(fo));  // read back from LDS here, not held in registers
+        const double hx = L.frame[grp][2 + fo], hy = L.frame[grp][3 + fo];
+        double px, py;
+        {
+#pragma clang fp contract(off)
+            px = m3 ? kEps : (gx - L.frame[grp][fo]) * hx;
+            py = m3 ? kEps : (gy - L.frame[grp][1 + fo]) * hy;
+        }
+        if (sub + 1 < ny) {  // the next row's point
+            yk = ap->ylist[ybase + sub + 1];
+            gx = ap->Y[2 * (long)yk];
+            gy = ap->Y[2 * (long)yk + 1];
+        }
+        // u = Y - xi with exact zeros -> eps (src/generate_operator.jl:125-154)
+        auto u_at = [&](double x, double y, double &ux, double &uy) {
+            ux = m3 ? x : px - x;
+            uy = m3 ? y : py - y;
+            if (!m3 && ux == 0.0) ux = kEps;
+            if (!m3 && uy == 0.0) uy = kEps;
+        };
+        for (int o0 = 0; o0 < ap->nops; o0 += RC) {
+            double ba[NB2][RC], bb[NB1][RC], np[NB1][RC];
+            // kept inside the row loop: hoisted out of it, what depends on the
+            // operators costs more registers than it saves work
+            int kind[RC], ord[RC];
+            int mh = m;
+            asm volatile("" : "+s"(mh));
+#pragma unroll
+            for (int o = 0; o < RC; ++o) {
+                kind[o] = ap->op_kind[min(o0 + o, ap->nops - 1)];
+                ord[o] = ap->op_k[min(o0 + o, ap->nops - 1)];
+                asm volatile("" : "+s"(kind[o]), "+s"(ord[o]));
+            }
+            auto rhs_at = [&](int p, double (&b)[RC]) {
+                double ux, uy;
+                u_at(L.xi[grp][2 * p], L.xi[grp][2 * p + 1], ux, uy);
+                const NsPhsAt q = ns_phs_at(mh, ux, uy);
+#pragma unroll
+                for (int o = 0; o < RC; ++o) {
+                    b[o] = ns_op_phs(kind[o], ord[o], mh, ap->xk_c[min(o0 + o, ap->nops - 1)], ux, uy, hx, hy, q);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+#pragma unroll
+            for (int s = 0; s < NB2; ++s) rhs_at(NP + qa[s], ba[s]);
+#pragma unroll
+            for (int s = 0; s < NB1; ++s) {
+                rhs_at(kb[s], bb[s]);
+                int q = kb[s];  // the exponents of monomial kb
+                asm volatile("" : "+v"(q));
+                const int d = (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15) + (q >= 21);
+                const int ea = q - d * (d + 1) / 2, eb = d - ea;
+#pragma unroll
+                for (int o = 0; o < RC; ++o) {
+                    np[s][o] = -ns_op_mono(kind[o], ord[o], ea, eb, px, py, hx, hy);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // the negated weights: w1n = -w0 first, w2n = 0
+            double w1n[NB1][RC], w2n[NB2][RC];
+#pragma unroll
+            for (int s = 0; s < NB1; ++s) {
+#pragma unroll
+                for (int o = 0; o < RC; ++o) w1n[s][o] = 0.0;
+                fb_sum<0, NP>(w1n[s], np, Pit[s]);
+            }
+#pragma unroll
+            for (int s = 0; s < NB2; ++s)
+#pragma unroll
+                for (int o = 0; o < RC; ++o) w2n[s][o] = 0.0;
+            // the solve, then one step of refinement: residual b - Phi w,
+            // projected on the null space, through S^-1
+#pragma nounroll
+            for (int it = 0; it < 2; ++it) {
+                double ra[NB2][RC], rb[NB1][RC];
+                int kh[NB1], qh[NB2];  // addresses formed here each time, not held in registers
+#pragma unroll
+                for (int s = 0; s < NB1; ++s) {
+                    kh[s] = kb[s];
+                    asm volatile("" : "+v"(kh[s]));
+                }
+#pragma unroll
+                for (int s = 0; s < NB2; ++s) {
+                    qh[s] = qa[s];
+                    asm volatile("" : "+v"(qh[s]));
+                }
+#pragma unroll
+                for (int s = 0; s < NB2; ++s) {
+                    double f[NP];
+#pragma unroll
+                    for (int c = 0; c < NP; ++c) f[c] = f21(qh[s], c);
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) ra[s][o] = ba[s][o];
+                    fb_sum<0, NP>(ra[s], w1n, f);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                for_blocks<0, NB1>([&](auto sc) {
+                    constexpr int s = decltype(sc)::value;
+                    double f[NP];
+                    for_blocks<0, NP>([&](auto cc) { f[decltype(cc)::value] = f11(kh[s], sc, cc); });
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) rb[s][o] = bb[s][o];
+                    fb_sum<0, NP>(rb[s], w1n, f);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                if (it) {
+                    for_blocks<0, NB2>([&](auto sc) {
+                        constexpr int s = decltype(sc)::value;
+                        double f[N2];
+                        for_blocks<0, N2>([&](auto jc) { f[decltype(jc)::value] = f22(qh[s], sc, jc); });
+                        fb_sum<0, N2>(ra[s], w2n, f);
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
+#pragma unroll
+                    for (int s = 0; s < NB1; ++s) {
+                        double f[N2];
+#pragma unroll
+                        for (int j = 0; j < N2; ++j) f[j] = f12(kh[s], j);
+                        fb_sum<0, N2>(rb[s], w2n, f);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < NB2; ++s) fb_sum<0, NP>(ra[s], rb, nT[s]);
+                double dn[NB2][RC];
+#pragma unroll
+                for (int s = 0; s < NB2; ++s) {
+                    double y[RC];
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) y[o] = 0.0;
+                    fb_sum<0, N2>(y, ra, S[s]);
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) {
+                        dn[s][o] = -rps[s] * y[o];
+                        w2n[s][o] += dn[s][o];
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < NB1; ++s) fb_sum<0, N2>(w1n[s], dn, nTt[s]);
+            }
+            // ---- CSR output, columns sorted by global index
+#pragma unroll
+            for (int o = 0; o < RC; ++o) {
+                if (o0 + o < ap->nops) {
+                    const double f = m3 ? -1.0 : -op_post_scale(kind[o], ord[o], hx, hy);
+                    double *out = ap->vals[o0 + o] + row * NN;
+#pragma unroll
+                    for (int s = 0; s < NB2; ++s) {
+                        if (t + 16 * s < N2) {
+                            const double wv = f * w2n[s][o];
+                            bad |= !__builtin_isfinite(wv);
+                            if (on) out[L.rank[grp][NP + qa[s]]] = wv;
+                        }
+                    }
+#pragma unroll
+                    for (int s = 0; s < NB1; ++s) {
+                        if (t + 16 * s < NP) {
+                            const double wv = f * w1n[s][o];
+                            bad |= !__builtin_isfinite(wv);
+                            if (on) out[L.rank[grp][kb[s]]] = wv;
+                        }
+                    }
+                }
+            }
+        }
+        if (ap->colidx && on) {
+#pragma unroll
+            for (int s = 0; s < NB2; ++s)
+                if (t + 16 * s < N2) ap->colidx[row * NN + L.rank[grp][NP + qa[s]]] = L.g[grp][NP + qa[s]];
+#pragma unroll
+            for (int s = 0; s < NB1; ++s)
+                if (t + 16 * s < NP) ap->colidx[row * NN + L.rank[grp][kb[s]]] = L.g[grp][kb[s]];
+        }
+        if (ap->status && on && t == 0 && !ap->status_accumulate) ap->status[row] = 0;
+    }
+    // rows for the pivoting kernel
+    const uint64_t bb = __builtin_amdgcn_ballot_w64(bad);
+    if (((bb >> (grp * 16)) & 0xFFFFu) && live) {
+        for (int q = t; q < ny; q += 16)
+            a.redo[1 + atomicAdd(a.redo, 1)] = grouped ? a.ylist[ybase + q] : yk;
+    }
+}
+
+// One wavefront (four stencils) per block.
+template <int NN, int NP>
+void launch_ns_shape(const NsArgs &a, hipStream_t s)
+{
+    const unsigned nb = (unsigned)((a.ntasks + 3) / 4);
+    if (a.nops == 1) solve_ns_kernel<NN, NP, 1><<<nb, 64, 0, s>>>(a);
+    else if (a.nops == 2) solve_ns_kernel<NN, NP, 2><<<nb, 64, 0, s>>>(a);
+    else solve_ns_kernel<NN, NP, 3><<<nb, 64, 0, s>>>(a);
+}
+
+}  // namespace rbffd
+
+#define RBFFD_DEFINE_NS(nn, pp) \
+    namespace rbffd {           \
+    void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_shape<nn, pp>(a, s); } \
+    }

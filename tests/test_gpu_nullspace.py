@@ -1,0 +1,95 @@
+"""The null-space solve (odd PHS powers with polynomials of degree at least
+(m - 1) / 2): weights against the high-precision oracle on node sets from
+even to clustered, and what it hands to the pivoting kernel (duplicated and
+nearly duplicated nodes, coordinates that are not finite) against that kernel
+alone (RBFFD_NULLSPACE=0).
+
+Bar: per-row relative error at most 1e-10, or 4 times that of an FP64 LU solve
+of the same row's system, with the node set's median LU error as the least LU
+error counted (single rows of an LU solve can be right by luck)."""
+import numpy as np
+import pytest
+
+from rbffd_amd.nodes import jittered_grid
+
+pytestmark = pytest.mark.gpu
+
+# (PHS power, polynomial degree, stencil size)
+SHAPES = [(3, 3, 20), (5, 3, 21), (7, 3, 21), (7, 4, 31), (9, 4, 31)]
+OPS = ["E", "Dx", "Dyy", "Dxy", "Lap", "Dxk", "Dyk"]
+
+
+def _weights(ctx, X, st, p, polydeg, ops, k, method=1):
+    import rbffd_amd
+
+    eng = rbffd_amd.Engine(ctx)
+    Xd = ctx.to_device(X)
+    col, vals, status = eng.weights(Xd, Xd, ctx.to_device(st.astype(np.int32)), None, p, polydeg, ops, k=k,
+                                    method=method)
+    return col.get(), [v.get() for v in vals], status.get()
+
+
+def _nodes(kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "grid":
+        return jittered_grid(23, 21, 0.3, seed=seed)  # 483 rows: three stencils past a full wavefront
+    if kind == "uniform":
+        return rng.uniform(0, 1, (401, 2))
+    return np.concatenate([rng.uniform(0, 1, (200, 2)), 0.5 + 0.02 * rng.standard_normal((202, 2))])
+
+
+@pytest.mark.parametrize("p,polydeg,n", SHAPES)
+@pytest.mark.parametrize("kind", ["grid", "uniform", "clustered"])
+def test_against_the_oracle(ctx, O, p, polydeg, n, kind):
+    X = _nodes(kind, n + p)
+    k = 2
+    print(f"null-space solve p={p} deg={polydeg} n={n} {kind}", flush=True)
+    st, _ = O.knn(X, X, n)
+    col, vals, status = _weights(ctx, X, st, p, polydeg, OPS, k)
+    assert not status.any()
+    opl = [(O.OP_NAMES[o], k if o in ("Dxk", "Dyk") else 0) for o in OPS]
+    Wq, _, _ = O.weights(X, X, st, None, p, polydeg, opl, quad=True)
+    Wl, _, _ = O.weights(X, X, st, None, p, polydeg, opl, solve="lu")
+    order = np.argsort(st, axis=1, kind="stable")
+    assert np.array_equal(col, np.take_along_axis(st, order, 1))
+    for o, name in enumerate(OPS):
+        q = np.take_along_axis(Wq[:, o, :], order, 1)
+        scale = np.abs(q).max(axis=1)
+        e = np.abs(vals[o] - q).max(axis=1) / scale
+        lu = np.abs(np.take_along_axis(Wl[:, o, :], order, 1) - q).max(axis=1) / scale
+        print(f"  {name}: max {e.max():.2e} median {np.median(e):.2e} (LU {lu.max():.2e} {np.median(lu):.2e})",
+              flush=True)
+        assert e.max() <= max(1e-10, 4 * lu.max())
+        assert np.median(e) <= max(1e-13, 2 * np.median(lu))
+
+
+@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31)])
+@pytest.mark.parametrize("nops", [1, 2, 7])
+def test_handed_back_rows(ctx, O, p, polydeg, n, nops, monkeypatch):
+    """Rows whose stencil holds a duplicated or nearly duplicated node or a NaN
+    get what the pivoting kernel alone gives them, bits and status; the other
+    rows agree to rounding."""
+    X = jittered_grid(24, 22, 0.25, seed=n)
+    h = 1.0 / 23
+    extra = X[[100, 260]].copy()                      # two exact duplicates
+    near = X[[150, 400, 410]] + h * np.array([[1e-9, 0], [0, 1e-11], [3e-13, 1e-13]])
+    X = np.concatenate([X, extra, near])
+    st, _ = O.knn(X, X, n)
+    Xn = X.copy()
+    Xn[30, 1] = np.nan                                # after the search: its stencils carry a NaN
+    ops = OPS[1:1 + nops] if nops < 7 else OPS
+    print(f"handed-back rows p={p} n={n}, {nops} operators", flush=True)
+    hit = np.isin(st, [100, 260, len(X) - 5, len(X) - 4]).sum(axis=1) > 0
+    touched = np.isin(st, [30, 100, 260, 150, 400, 410] + list(range(len(X) - 5, len(X)))).any(axis=1)
+    col, vals, status = _weights(ctx, Xn, st, p, polydeg, ops, 2)
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = _weights(ctx, Xn, st, p, polydeg, ops, 2)
+    assert np.array_equal(col, col0)
+    assert np.array_equal(status, status0)
+    assert status[np.isin(st, [30]).any(axis=1)].all() and hit.any()
+    for a, b in zip(vals, vals0):
+        ok = ~touched
+        d = np.abs(a[ok] - b[ok]).max(axis=1) / np.abs(b[ok]).max(axis=1)
+        assert d.max() <= 1e-9
+        bad = status0 != 0
+        assert np.array_equal(a[bad], b[bad], equal_nan=True)
