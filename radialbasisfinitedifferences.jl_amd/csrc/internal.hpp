@@ -133,7 +133,7 @@ void launch_solve(const SolveArgs &a, int precision, hipStream_t s);
 bool ns_applies(int n, int polydeg, int m, int nops, const int *ops);
 void launch_ns(const NsArgs &a, hipStream_t s);
 void ns_deriv_constants(int m, int k, double *c);
-#define RBFFD_NS_SHAPES(X) X(20, 10) X(21, 10) X(31, 15)
+#define RBFFD_NS_SHAPES(X) X(20, 10) X(21, 10) X(31, 15) X(42, 21) X(43, 21) X(57, 28)
 #define RBFFD_DECLARE_NS(nn, pp) void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s);
 RBFFD_NS_SHAPES(RBFFD_DECLARE_NS)
 #undef RBFFD_DECLARE_NS

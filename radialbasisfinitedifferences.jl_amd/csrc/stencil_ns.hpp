@@ -462,6 +462,34 @@ __device__ __forceinline__ void fb_cols(double (&a)[W], const double (&s)[W], do
     else if constexpr (CNT == 1)
         fb_row<L>(a[(J + 0) % W], s[(J + 0) % W], m);
 }
+// a[JA + i] += s[JS + i](lane L) * m for i < CNT
+template <int L, int JA, int JS, int CNT, int WA, int WS>
+__device__ __forceinline__ void fb_sub(double (&a)[WA], const double (&s)[WS], double m)
+{
+    if constexpr (CNT > 8) {
+        fb_sub<L, JA, JS, 8>(a, s, m);
+        fb_sub<L, JA + 8, JS + 8, CNT - 8>(a, s, m);
+    } else if constexpr (CNT == 8)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], a[JA + 3], a[JA + 4], a[JA + 5], a[JA + 6], a[JA + 7], s[JS + 0],
+                s[JS + 1], s[JS + 2], s[JS + 3], s[JS + 4], s[JS + 5], s[JS + 6], s[JS + 7], m);
+    else if constexpr (CNT == 7)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], a[JA + 3], a[JA + 4], a[JA + 5], a[JA + 6], s[JS + 0], s[JS + 1],
+                s[JS + 2], s[JS + 3], s[JS + 4], s[JS + 5], s[JS + 6], m);
+    else if constexpr (CNT == 6)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], a[JA + 3], a[JA + 4], a[JA + 5], s[JS + 0], s[JS + 1], s[JS + 2],
+                s[JS + 3], s[JS + 4], s[JS + 5], m);
+    else if constexpr (CNT == 5)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], a[JA + 3], a[JA + 4], s[JS + 0], s[JS + 1], s[JS + 2], s[JS + 3],
+                s[JS + 4], m);
+    else if constexpr (CNT == 4)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], a[JA + 3], s[JS + 0], s[JS + 1], s[JS + 2], s[JS + 3], m);
+    else if constexpr (CNT == 3)
+        fb_row<L>(a[JA + 0], a[JA + 1], a[JA + 2], s[JS + 0], s[JS + 1], s[JS + 2], m);
+    else if constexpr (CNT == 2)
+        fb_row<L>(a[JA + 0], a[JA + 1], s[JS + 0], s[JS + 1], m);
+    else if constexpr (CNT == 1)
+        fb_row<L>(a[JA + 0], s[JS + 0], m);
+}
 // a[j] += s[j / 16](lane j % 16) * m for CNT columns j = J, J + 1, ... (mod W);
 // one asm block stays inside one 16-column slot of s
 template <int J, int CNT, int W, int NB>
@@ -530,6 +558,20 @@ __device__ __forceinline__ void fb_sum(double (&a)[RC], const double (&s)[NB][RC
     }
 }
 
+// The same sum in two chains of half the length, added to a at the end: the
+// residual's rounding is what is left of the solve's error
+template <int K1, int RC, int NB, int W>
+__device__ __forceinline__ void fb_sum2(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
+{
+    double h0[RC], h1[RC];
+#pragma unroll
+    for (int o = 0; o < RC; ++o) h0[o] = h1[o] = 0.0;
+    fb_sum<0, K1 / 2>(h0, s, m);
+    fb_sum<K1 / 2, K1>(h1, s, m);
+#pragma unroll
+    for (int o = 0; o < RC; ++o) a[o] += h0[o] + h1[o];
+}
+
 __device__ __forceinline__ uint32_t lds_address(const void *p)
 {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
@@ -555,13 +597,57 @@ __device__ __forceinline__ double hi_if(double v, bool c, uint32_t hi)
     return __longlong_as_double((long long)(((uint64_t)h << 32) | (uint32_t)b));
 }
 
-// whether row slot S of this lane, t + 16 S, is at most c
-template <int S>
+// whether row S of this lane, (lane mod G) + G S, is at most c: a lane mask known
+// at compile time
+template <int G, int S>
 __device__ __forceinline__ bool upto(int c)
 {
-    const int e = c - 16 * S;
-    const uint64_t m = e < 0 ? 0ull : (e >= 15 ? 0xFFFFull : (2ull << e) - 1ull);
-    return __builtin_amdgcn_inverse_ballot_w64(m * 0x0001000100010001ull);
+    const int e = c - G * S;
+    const uint64_t m = e < 0 ? 0ull : (2ull << (e >= G ? G - 1 : e)) - 1ull;
+    return __builtin_amdgcn_inverse_ballot_w64(m * (G == 16 ? 0x0001000100010001ull : 0x0000000100000001ull));
+}
+
+// Per-lane rows as broadcast sources: src[b] holds, in every 16-lane DPP row of
+// a group, rows 16 b .. 16 b + 15.  With 16 lanes these are the lane's own row
+// slots; with 32, v_permlane16_swap gives both halves to both DPP rows.
+template <int G, int S, int R>
+__device__ __forceinline__ void spread(const double (&own)[S], double (&src)[R])
+{
+    if constexpr (G == 16) {
+        static_assert(S == R, "row slots");
+#pragma unroll
+        for (int b = 0; b < R; ++b) src[b] = own[b];
+    } else {
+        static_assert(S == 1 && R <= 2, "row slots");
+        const uint64_t v = (uint64_t)__double_as_longlong(own[0]);
+        const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+#pragma unroll
+        for (int b = 0; b < R; ++b)
+            src[b] = __longlong_as_double((long long)(((uint64_t)(uint32_t)hi[b] << 32) | (uint32_t)lo[b]));
+    }
+}
+// x's odd 16-lane rows exchanged with y's even ones (v_permlane16_swap)
+__device__ __forceinline__ void swap_rows(double x, double y, double &p, double &q)
+{
+    const uint64_t a = (uint64_t)__double_as_longlong(x), b = (uint64_t)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)a, (uint32_t)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(a >> 32), (uint32_t)(b >> 32), false, false);
+    p = __longlong_as_double((long long)(((uint64_t)(uint32_t)hi[0] << 32) | (uint32_t)lo[0]));
+    q = __longlong_as_double((long long)(((uint64_t)(uint32_t)hi[1] << 32) | (uint32_t)lo[1]));
+}
+template <int G, int S, int R, int RC>
+__device__ __forceinline__ void spread(const double (&own)[S][RC], double (&src)[R][RC])
+{
+#pragma unroll
+    for (int o = 0; o < RC; ++o) {
+        double a[S], b[R];
+#pragma unroll
+        for (int i = 0; i < S; ++i) a[i] = own[i][o];
+        spread<G>(a, b);
+#pragma unroll
+        for (int i = 0; i < R; ++i) src[i][o] = b[i];
+    }
 }
 
 // 1 / x to within an ulp (x finite and not zero): the instruction gives 23
@@ -683,11 +769,13 @@ __device__ __forceinline__ double ns_op_mono(int op, int k, int ea, int eb, doub
     return ns_mono(ea, eb, a, b, x, y);
 }
 
-template <int NN, int NP>
+template <int NN, int NP, int G>
 struct NsShape {
     static constexpr int N2 = NN - NP;
-    static constexpr int NB1 = (NP + 15) / 16, NB2 = (N2 + 15) / 16;  // row slots of the two node sets
-    static constexpr int NODES = (NN + 15) / 16;
+    static constexpr int S = 64 / G;                                      // stencils per wavefront
+    static constexpr int S1 = (NP + G - 1) / G, S2 = (N2 + G - 1) / G;    // row slots per lane of the two node sets
+    static constexpr int B1 = (NP + 15) / 16, B2 = (N2 + 15) / 16;        // their 16-row broadcast sources
+    static constexpr int NODES = (NN + G - 1) / G;
     static constexpr int TS = NP | 1;  // row stride of the panel's result: odd, so a column read has no bank conflicts
     // Phi by position: the picked nodes' upper triangle, the NP x N2 block, the others' upper triangle
     // (rows of the block an odd stride apart: its rows are read across lanes too)
@@ -695,43 +783,49 @@ struct NsShape {
     static constexpr int F11 = 0, F12 = NP * (NP + 1) / 2, F22 = F12 + NP * WS;
     static constexpr int PHI = F22 + N2 * (N2 + 1) / 2;
     static constexpr int RPS = cmax_<PHI, NN * TS>::v;  // reciprocal pivots of S, behind Phi
-    // per group: 16 modulo 32 doubles, so two groups' odd-stride reads fall on all 64 banks
-    static constexpr int U = (RPS + N2 + 15) / 32 * 32 + 16;
+    // per group; with 16 lanes 16 modulo 32 doubles, so two groups' odd-stride reads fall on all 64 banks
+    static constexpr int U = G == 16 ? (RPS + N2 + 15) / 32 * 32 + 16 : (RPS + N2 + 1) & ~1;
     static constexpr __host__ __device__ int tri(int w, int a) { return a * (2 * w - a + 1) / 2 - a; }
 };
 
-template <int NN, int NP>
+template <int NN, int NP, int G>
 struct alignas(16) NsLDS {
-    using T = NsShape<NN, NP>;
-    double u[4][T::U];      // the panel's pivot row, then P1^-1 and T, then Phi
-    double xi[4][2 * NN];   // scaled coordinates by position
-    double frame[4][4];     // centre and scales
-    int g[4][NN], rank[4][NN];  // global index and output column by position
+    using T = NsShape<NN, NP, G>;
+    double u[T::S][T::U];       // the panel's pivot row, then P1^-1 and T, then Phi
+    double xi[T::S][2 * NN];    // scaled coordinates by position
+    double frame[T::S][4];      // centre and scales
+    int g[T::S][NN], rank[T::S][NN];  // global index and output column by position
 };
 
 // Wavefronts per SIMD the kernel is compiled for.  n = 31: LDS (20 KB a
 // wavefront) and the row registers hold it to two.  n = 20 and 21: three, with
 // 30 registers spilled, take 2.00 ms per 1M stencils of n = 21 where two
 // without spills take 2.29 ms.
-template <int NN, int NP>
+template <int NN, int NP, int G>
 constexpr int ns_min_waves()
 {
+    if (G == 32) return NN <= 43 ? 2 : 1;
     return NN <= 21 ? 3 : 2;
 }
 
-template <int NN, int NP, int RC>
-__global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(const NsArgs a)
+// NN nodes (GEN: at most NN, a.n of them), NP monomials, G lanes per stencil,
+// RC operators at a time
+template <int NN, int NP, int G, int RC, bool GEN>
+__global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kernel(const NsArgs a)
 {
-    using T = NsShape<NN, NP>;
-    constexpr int N2 = T::N2, NB1 = T::NB1, NB2 = T::NB2, NODES = T::NODES;
+    using T = NsShape<NN, NP, G>;
+    constexpr int N2 = T::N2, S1 = T::S1, S2 = T::S2, B1 = T::B1, B2 = T::B2, NODES = T::NODES;
     constexpr int DEG = mono_deg(NP - 1);
-    __shared__ NsLDS<NN, NP> L;
-    const int lane = threadIdx.x & 63, grp = lane >> 4, t = lane & 15;
+    constexpr uint64_t kLane0 = G == 16 ? 0x0001000100010001ull : 0x0000000100000001ull;  // lane 0 of each group
+    constexpr uint32_t kGroup = (uint32_t)((1ull << G) - 1);
+    __shared__ NsLDS<NN, NP, G> L;
+    const int lane = threadIdx.x & 63, grp = lane / G, t = lane % G;
     double *const U = L.u[grp];
+    const int n = GEN ? a.n : NN, n2 = n - NP;
     const bool grouped = a.grp_x != nullptr;
     long ntasks = a.ntasks;
     if (a.ntasks_dev) ntasks = min(ntasks, (long)*a.ntasks_dev);
-    const long task0 = (long)blockIdx.x * 4;
+    const long task0 = (long)blockIdx.x * T::S;
     if (task0 >= ntasks) return;  // whole wavefront
     // a group without a task works on a copy of the first and stores nothing
     const bool live = task0 + grp < ntasks;
@@ -751,39 +845,39 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
     const bool m3 = a.method == 3;
 
     // ---- stencil frame (src/scalestencil.jl:10-21, src/generate_operator.jl:100-134)
-    double C[NODES][NP];  // this lane's rows of P: nodes t + 16 r
+    double C[NODES][NP];  // this lane's rows of P: nodes t + G r
     uint32_t alive[NODES];
     double sx = 1.0, sy = 1.0, cx, cy;
     double nx[NODES], nyy[NODES];
     int gid[NODES], rk[NODES];
     {
 #pragma clang fp contract(off)
-        const int c = max(a.stencils[xs * NN], 0);  // a failed search leaves -1: every read stays in X
+        const int c = max(a.stencils[xs * n], 0);  // a failed search leaves -1: every read stays in X
         cx = a.X[2 * (long)c];
         cy = a.X[2 * (long)c + 1];
         double mx = 0.0, my = 0.0;
         int *gl = reinterpret_cast<int *>(U);
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
-            const int i = t + 16 * r;
-            gid[r] = i < NN ? max(a.stencils[xs * NN + i], 0) : c;
-            if (i < NN) gl[i] = gid[r];
+            const int i = t + G * r;
+            gid[r] = i < n ? max(a.stencils[xs * n + i], 0) : c;
+            if (i < NN) gl[i] = i < n ? gid[r] : 0x7FFFFFFF;
             nx[r] = a.X[2 * (long)gid[r]] - cx;
             nyy[r] = a.X[2 * (long)gid[r] + 1] - cy;
             mx = fmax(mx, __builtin_fabs(nx[r]));
             my = fmax(my, __builtin_fabs(nyy[r]));
         }
         if (!m3) {
-            mx = group_max_nonneg_f64<16>(mx);
-            my = group_max_nonneg_f64<16>(my);
+            mx = group_max_nonneg_f64<G>(mx);
+            my = group_max_nonneg_f64<G>(my);
             sx = 1.0 / mx;
             sy = 1.0 / my;
         }
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
             // method 3 leaves the frame unscaled, its centre at (eps, eps) (src/generate_operator.jl:393-410)
-            nx[r] = m3 ? (t + 16 * r == 0 ? kEps : nx[r]) : nx[r] * sx;
-            nyy[r] = m3 ? (t + 16 * r == 0 ? kEps : nyy[r]) : nyy[r] * sy;
+            nx[r] = m3 ? (t + G * r == 0 ? kEps : nx[r]) : nx[r] * sx;
+            nyy[r] = m3 ? (t + G * r == 0 ? kEps : nyy[r]) : nyy[r] * sy;
         }
         __builtin_amdgcn_wave_barrier();
         // the output column of each node: the rank of its global index inside the stencil
@@ -797,7 +891,6 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         }
         __builtin_amdgcn_wave_barrier();
     }
-
     if (t == 0) {
         L.frame[grp][0] = cx;
         L.frame[grp][1] = cy;
@@ -814,7 +907,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         px[0] = py[0] = 1.0;
 #pragma unroll
         for (int d = 1; d <= DEG; ++d) { px[d] = px[d - 1] * nx[r]; py[d] = py[d - 1] * nyy[r]; }
-        alive[r] = t + 16 * r < NN ? 0xFFFFFFFFu : 0u;
+        alive[r] = t + G * r < n ? 0xFFFFFFFFu : 0u;
 #pragma unroll
         for (int q = 0; q < NP; ++q) C[r][q] = px[mono_ea(q)] * py[mono_eb(q)];
     }
@@ -833,7 +926,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
             const uint32_t kr = ((__float_as_uint((float)C[r][k]) & 0x7FFFFF00u) |
-                                 (0x80u | (uint32_t)(127 - (t + 16 * r)))) & alive[r];
+                                 (0x80u | (uint32_t)(127 - (t + G * r)))) & alive[r];
             if (r == 0) {
                 key = kr;
             } else if (kr > key) {
@@ -842,14 +935,14 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
             }
         }
         const double crp = rcp_nr(cv);
-        key = group_max_u32<16>(key);
+        key = group_max_u32<G>(key);
         weakest = min(weakest, key);
         const int v = 127 - (int)(key & 127u);
-        const bool iam = t == (v & 15);
+        const bool iam = t == v % G;
         // the picked row goes to the group, its reciprocal pivot in the pivot's place
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
-            if (iam && (v >> 4) == r) {
+            if (iam && v / G == r) {
                 for_blocks<0, NP / 2>([&](auto jc) {
                     constexpr int j = 2 * decltype(jc)::value;
                     lds_write2<j, j + 1>(ua, j == k ? crp : C[r][j], j + 1 == k ? crp : C[r][j + 1]);
@@ -861,14 +954,14 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
             }
         }
         __builtin_amdgcn_wave_barrier();
-        double pr[NB1];
+        double pr[B1];
 #pragma unroll
-        for (int b = 0; b < NB1; ++b) pr[b] = U[t + 16 * b];
+        for (int b = 0; b < B1; ++b) pr[b] = U[t % 16 + 16 * b];
         const double rp = row_bcast64<k % 16>(pr[k / 16]);
         double l[NODES];
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
-            const bool me = iam && (v >> 4) == r;
+            const bool me = iam && v / G == r;
             // the picked row's multiplier: its high word zeroed leaves a value below 2^-1022, which the additions lose
             l[r] = hi_if(-(C[r][k] * rp), me, 0u);
             C[r][k] = me ? 1.0 : l[r];
@@ -887,14 +980,14 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         for (int r = 0; r < NODES; ++r) {
             const bool fr = alive[r] != 0u;
             const uint64_t bal = __builtin_amdgcn_ballot_w64(fr);
-            const uint32_t gm = (uint32_t)(bal >> (grp * 16)) & 0xFFFFu;
+            const uint32_t gm = (uint32_t)(bal >> (grp * G)) & kGroup;
             if (fr) pos[r] = base + __builtin_popcount(gm & ((1u << t) - 1u));
             base += __builtin_popcount(gm);
         }
     }
 #pragma unroll
     for (int r = 0; r < NODES; ++r) {
-        if (t + 16 * r < NN) {
+        if (t + G * r < n) {
 #pragma unroll
             for (int j = 0; j < NP; ++j) U[pos[r] * T::TS + j] = C[r][j] * fin[r];
             L.xi[grp][2 * pos[r]] = nx[r];
@@ -904,28 +997,23 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         }
     }
     __builtin_amdgcn_wave_barrier();
-    // this lane's rows from here on: picked nodes kb[s] = t + 16 s, others
-    // qa[s] = t + 16 s (lanes past the end repeat the last row and store nothing)
-    int kb[NB1], qa[NB2];
-    double xb[NB1], yb[NB1], xa[NB2], ya[NB2];
-    double nT[NB2][NP];   // -T, row qa
-    double nTt[NB1][N2];  // -T, column kb
-    double Pit[NB1][NP];  // P1^-1, column kb
+    // this lane's rows from here on: picked nodes kb[s] = t + G s, others
+    // qa[s] = t + G s (lanes past the end repeat the last row and store nothing)
+    int kb[S1], qa[S2];
+    double nT[S2][NP];   // -T, row qa
+    double nTt[S1][N2];  // -T, column kb
+    double Pit[S1][NP];  // P1^-1, column kb
 #pragma unroll
-    for (int s = 0; s < NB1; ++s) {
-        kb[s] = min(t + 16 * s, NP - 1);
-        xb[s] = L.xi[grp][2 * kb[s]];
-        yb[s] = L.xi[grp][2 * kb[s] + 1];
+    for (int s = 0; s < S1; ++s) {
+        kb[s] = min(t + G * s, NP - 1);
 #pragma unroll
         for (int k = 0; k < NP; ++k) Pit[s][k] = U[k * T::TS + kb[s]];
 #pragma unroll
-        for (int i = 0; i < N2; ++i) nTt[s][i] = U[(NP + i) * T::TS + kb[s]];
+        for (int i = 0; i < N2; ++i) nTt[s][i] = !GEN || i < n2 ? U[(NP + i) * T::TS + kb[s]] : 0.0;
     }
 #pragma unroll
-    for (int s = 0; s < NB2; ++s) {
-        qa[s] = min(t + 16 * s, N2 - 1);
-        xa[s] = L.xi[grp][2 * (NP + qa[s])];
-        ya[s] = L.xi[grp][2 * (NP + qa[s]) + 1];
+    for (int s = 0; s < S2; ++s) {
+        qa[s] = min(t + G * s, n2 - 1);
 #pragma unroll
         for (int k = 0; k < NP; ++k) nT[s][k] = U[(NP + qa[s]) * T::TS + k];
     }
@@ -933,6 +1021,10 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
 
     __builtin_amdgcn_sched_barrier(0);
     // ---- Phi by position, each pair once
+    if constexpr (GEN) {  // columns past the last node stay zero
+        for (int i = t; i < T::PHI; i += G) U[i] = 0.0;
+        __builtin_amdgcn_wave_barrier();
+    }
     {
         auto pairs = [&](auto mc) {
             constexpr int MC = decltype(mc)::value;
@@ -943,28 +1035,30 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
                 return upow(r2, mm >> 1) * ns_sqrt(r2);
             };
 #pragma unroll
-            for (int s = 0; s < NB2; ++s) {
-                if (t + 16 * s < N2) {
+            for (int s = 0; s < S2; ++s) {
+                if (t + G * s < n2) {
+                    const double x = L.xi[grp][2 * (NP + qa[s])], y = L.xi[grp][2 * (NP + qa[s]) + 1];
 #pragma unroll 3
-                    for (int k = 0; k < NP; ++k) U[T::F12 + k * T::WS + qa[s]] = phs(xa[s], ya[s], k);
+                    for (int k = 0; k < NP; ++k) U[T::F12 + k * T::WS + qa[s]] = phs(x, y, k);
                     U[T::F22 + T::tri(N2, qa[s]) + qa[s]] = 0.0;
 #pragma unroll 2
-                    for (int d = 1; d <= N2 / 2; ++d) {
+                    for (int d = 1; d <= n2 / 2; ++d) {
                         int j = qa[s] + d;
-                        if (j >= N2) j -= N2;
-                        U[T::F22 + T::tri(N2, min(qa[s], j)) + max(qa[s], j)] = phs(xa[s], ya[s], NP + j);
+                        if (j >= n2) j -= n2;
+                        U[T::F22 + T::tri(N2, min(qa[s], j)) + max(qa[s], j)] = phs(x, y, NP + j);
                     }
                 }
             }
 #pragma unroll
-            for (int s = 0; s < NB1; ++s) {
-                if (t + 16 * s < NP) {
+            for (int s = 0; s < S1; ++s) {
+                if (t + G * s < NP) {
+                    const double x = L.xi[grp][2 * kb[s]], y = L.xi[grp][2 * kb[s] + 1];
                     U[T::F11 + T::tri(NP, kb[s]) + kb[s]] = 0.0;
 #pragma unroll 2
                     for (int d = 1; d <= NP / 2; ++d) {
                         int j = kb[s] + d;
                         if (j >= NP) j -= NP;
-                        U[T::F11 + T::tri(NP, min(kb[s], j)) + max(kb[s], j)] = phs(xb[s], yb[s], j);
+                        U[T::F11 + T::tri(NP, min(kb[s], j)) + max(kb[s], j)] = phs(x, y, j);
                     }
                 }
             }
@@ -978,103 +1072,176 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         }
     }
     __builtin_amdgcn_wave_barrier();
-    // Phi(picked row kb, picked column c), Phi(kb, other j), Phi(other row qa, picked c), Phi(qa, other j)
-    // the two triangles: one addition and a select per entry, by lane masks known at compile time
-    auto f11 = [&](int k, auto sc, auto cc) {
-        constexpr int s = decltype(sc)::value, c = decltype(cc)::value;
+    // Phi(picked row k, picked column c), Phi(k, other j), Phi(other row q, picked c), Phi(q, other j);
+    // the two triangles: one addition and a select per entry, the mask by the row's slot (GG lanes apart)
+    auto f11 = [&](auto gg, int k, auto sc, auto cc) {
+        constexpr int GG = decltype(gg)::value, s = decltype(sc)::value, c = decltype(cc)::value;
         const int up = T::F11 + T::tri(NP, k), lo = k + (T::F11 + T::tri(NP, c) - c);
-        return U[(upto<s>(c) ? up : lo) + c];
+        return U[(upto<GG, s>(c) ? up : lo) + c];
     };
     auto f12 = [&](int k, int j) { return U[T::F12 + k * T::WS + j]; };
     auto f21 = [&](int q, int c) { return U[T::F12 + c * T::WS + q]; };
     auto f22 = [&](int q, auto sc, auto jc) {
         constexpr int s = decltype(sc)::value, j = decltype(jc)::value;
         const int up = T::F22 + T::tri(N2, q), lo = q + (T::F22 + T::tri(N2, j) - j);
-        return U[(upto<s>(j) ? up : lo) + j];
+        return U[(upto<G, s>(j) ? up : lo) + j];
     };
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- S = Phi22 - T Phi12 - (Phi21 - T Phi11) T^T, one row per lane slot
-    double S[NB2][N2];
-    {
-        double V[NB2][NP], B[NB1][NP];
-        for_blocks<0, NB1>([&](auto sc) {
-            constexpr int s = decltype(sc)::value;
-            for_blocks<0, NP>([&](auto cc) { B[s][decltype(cc)::value] = f11(kb[s], sc, cc); });
-        });
-#pragma unroll
-        for (int s = 0; s < NB2; ++s) {
-#pragma unroll
-            for (int c = 0; c < NP; ++c) V[s][c] = f21(qa[s], c);
-            for_blocks<0, NP>([&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                fb_cols<k % 16, 0, NP>(V[s], B[k / 16], nT[s][k]);
-            });
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        for_blocks<0, NB2>([&](auto sc) {
-            constexpr int s = decltype(sc)::value;
-            for_blocks<0, N2>([&](auto jc) { S[s][decltype(jc)::value] = f22(qa[s], sc, jc); });
-        });
-        // + V (-T)^T: column c of -T, over the lanes of the other nodes
-        for_blocks<0, NP>([&](auto cc) {
-            constexpr int c = decltype(cc)::value;
-            double tc[NB2];
-#pragma unroll
-            for (int s = 0; s < NB2; ++s) tc[s] = nT[s][c];
-#pragma unroll
-            for (int s = 0; s < NB2; ++s) fb_lanes<0, N2>(S[s], tc, V[s][c]);
-        });
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    {
-        double B[NB1][N2];
-#pragma unroll
-        for (int s = 0; s < NB1; ++s)
-#pragma unroll
-            for (int j = 0; j < N2; ++j) B[s][j] = f12(kb[s], j);
-#pragma unroll
-        for (int s = 0; s < NB2; ++s)
-            for_blocks<0, NP>([&](auto kc) {
-                constexpr int k = decltype(kc)::value;
-                fb_cols<k % 16, 0, N2>(S[s], B[k / 16], nT[s][k]);
-            });
-    }
+    using LanesG = std::integral_constant<int, G>;
+    using Lanes16 = std::integral_constant<int, 16>;
 
     __builtin_amdgcn_sched_barrier(0);
-    // ---- S^-1 in place without pivoting (S is definite); row q stays scaled
-    // by its pivot, whose reciprocal (rps) multiplies the products
-    for_blocks<0, N2>([&](auto kc) {
-        constexpr int k = decltype(kc)::value;
-        const double p = row_bcast64<k % 16>(S[k / 16][k]);
-        const double rp = rcp_nr(p);
-        U[T::RPS + k] = rp;  // the same value from every lane of the group
-        double l[NB2];
+    // ---- S = Phi22 - T Phi12 - (Phi21 - T Phi11) T^T, one row per lane slot.
+    // Columns go in blocks of 16, to bound the registers; the picked nodes' rows
+    // are loaded as broadcast sources (every DPP row of a group holds them all).
+    double S[S2][N2];
+    int ks[B1];
 #pragma unroll
-        for (int s = 0; s < NB2; ++s) {
-            const bool me = s == k / 16 && __builtin_amdgcn_inverse_ballot_w64(0x0001000100010001ull << (k % 16));
-            l[s] = hi_if(-(S[s][k] * rp), me, 0u);
-            S[s][k] = me ? 1.0 : l[s];
-        }
-#pragma unroll
-        for (int s = 0; s < NB2; ++s)
-            if constexpr (k + 1 < N2) fb_cols<k % 16, k + 1, 1>(S[s], S[k / 16], l[s]);
-#pragma unroll
-        for (int s = 0; s < NB2; ++s)
-            fb_cols<k % 16, (k + 1 < N2 ? k + 2 : k + 1) % N2, N2 - 1 - (k + 1 < N2)>(S[s], S[k / 16], l[s]);
+    for (int b = 0; b < B1; ++b) ks[b] = min(t % 16 + 16 * b, NP - 1);
+    for_blocks<0, S2>([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        for_blocks<0, N2>([&](auto jc) { S[s][decltype(jc)::value] = f22(qa[s], sc, jc); });
     });
+    for_blocks<0, (NP + 15) / 16>([&](auto blk) {
+        constexpr int c0 = 16 * decltype(blk)::value, W = NP - c0 < 16 ? NP - c0 : 16;
+        double V[S2][W], B[B1][W];
+        for_blocks<0, B1>([&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            for_blocks<0, W>([&](auto cc) {
+                B[b][decltype(cc)::value] =
+                    f11(Lanes16{}, ks[b], bc, std::integral_constant<int, c0 + decltype(cc)::value>{});
+            });
+        });
+#pragma unroll
+        for (int s = 0; s < S2; ++s) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) V[s][c] = f21(qa[s], c0 + c);
+            for_blocks<0, NP>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                fb_sub<k % 16, 0, 0, W>(V[s], B[k / 16], nT[s][k]);
+            });
+        }
+        // + V (-T)^T: column c of -T, over the lanes of the other nodes
+        for_blocks<0, W>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            double own[S2], tc[B2];
+#pragma unroll
+            for (int s = 0; s < S2; ++s) own[s] = nT[s][c0 + c];
+            spread<G>(own, tc);
+#pragma unroll
+            for (int s = 0; s < S2; ++s) fb_lanes<0, N2>(S[s], tc, V[s][c]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    for_blocks<0, (N2 + 15) / 16>([&](auto blk) {
+        constexpr int j0 = 16 * decltype(blk)::value, W = N2 - j0 < 16 ? N2 - j0 : 16;
+        double B[B1][W];
+#pragma unroll
+        for (int b = 0; b < B1; ++b)
+#pragma unroll
+            for (int j = 0; j < W; ++j) B[b][j] = f12(ks[b], j0 + j);
+#pragma unroll
+        for (int s = 0; s < S2; ++s)
+            for_blocks<0, NP>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                fb_sub<k % 16, j0, 0, W>(S[s], B[k / 16], nT[s][k]);
+            });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (GEN) {
+#pragma unroll
+        for (int s = 0; s < S2; ++s)
+#pragma unroll
+            for (int j = 0; j < N2; ++j) S[s][j] = j < n2 ? S[s][j] : 0.0;
+    }
+
+    // ---- S^-1 in place without pivoting (S is definite); row q stays scaled by
+    // its pivot, whose reciprocal (rps) multiplies the products
+    if constexpr (G == 16) {
+        for_blocks<0, N2>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            if (GEN && k >= n2) return;  // uniform
+            const double rp = rcp_nr(row_bcast64<k % 16>(S[k / 16][k]));
+            U[T::RPS + k] = rp;  // the same value from every lane of the group
+            double l[S2];
+#pragma unroll
+            for (int s = 0; s < S2; ++s) {
+                const bool me = s == k / 16 && __builtin_amdgcn_inverse_ballot_w64(kLane0 << (k % 16));
+                l[s] = hi_if(-(S[s][k] * rp), me, 0u);
+                S[s][k] = me ? 1.0 : l[s];
+            }
+#pragma unroll
+            for (int s = 0; s < S2; ++s)
+                if constexpr (k + 1 < N2) fb_cols<k % 16, k + 1, 1>(S[s], S[k / 16], l[s]);
+#pragma unroll
+            for (int s = 0; s < S2; ++s)
+                fb_cols<k % 16, (k + 1 < N2 ? k + 2 : k + 1) % N2, N2 - 1 - (k + 1 < N2)>(S[s], S[k / 16], l[s]);
+        });
+    } else {
+        // 32 lanes: a lane holds row t, and a pivot row would have to cross the
+        // group's two DPP rows entry by entry.  One lane swap per register pair
+        // turns that into two rows a lane, t % 16 and t % 16 + 16, with one half
+        // of the columns in each DPP row: the pivot row then broadcasts inside
+        // each, and only the multipliers cross (the pivot row's transpose, one
+        // value a lane, would cross as cheaply and do in exact arithmetic, but on
+        // uniform random nodes at n = 57 it left weights 1e-2 off).
+        constexpr int H = (N2 + 1) / 2;
+        double R[2][H];
+#pragma unroll
+        for (int j = 0; j < H; ++j) swap_rows(S[0][j], H + j < N2 ? S[0][H + j] : 0.0, R[0][j], R[1][j]);
+        for_blocks<0, N2>([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            if (GEN && k >= n2) return;              // uniform
+            constexpr int hk = k / H, kk = k % H;    // its column's DPP row and register
+            constexpr uint64_t half = 0x0000FFFF0000FFFFull << (16 * hk);
+            double c[2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const double own[1] = {R[s][kk]};
+                double both[2];
+                spread<G>(own, both);
+                c[s] = both[hk];
+            }
+            const double rp = rcp_nr(row_bcast64<k % 16>(c[k / 16]));
+            U[T::RPS + k] = rp;
+            // the column becomes -c rp (1 in the pivot row): zero plus the
+            // multiplier times the pivot row's entry, set to 1
+            double l[2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const bool me = s == k / 16 && __builtin_amdgcn_inverse_ballot_w64(0x0001000100010001ull << (k % 16));
+                const bool col = __builtin_amdgcn_inverse_ballot_w64(half);
+                l[s] = hi_if(-(c[s] * rp), me, 0u);
+                R[s][kk] = col ? 0.0 : R[s][kk];
+                if (s == k / 16)
+                    R[s][kk] = hi_if(R[s][kk], __builtin_amdgcn_inverse_ballot_w64(
+                                                   half & (0x0001000100010001ull << (k % 16))), 0x3FF00000u);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) fb_cols<k % 16, (kk + 1) % H, 1>(R[s], R[k / 16], l[s]);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) fb_cols<k % 16, (kk + 2) % H, H - 1>(R[s], R[k / 16], l[s]);
+        });
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+            double a, b;
+            swap_rows(R[0][j], R[1][j], a, b);
+            S[0][j] = a;
+            if (H + j < N2) S[0][H + j] = b;
+        }
+    }
     // pivots: the reciprocals' extremes over the group
-    double rps[NB2], rmin = 1e300, rmax = -1e300;
+    double rps[S2], rmin = 1e300, rmax = -1e300;
     const double sgn = ((m + 1) >> 1) & 1 ? -1.0 : 1.0;  // sign of the definite form, (-1)^((m+1)/2)
 #pragma unroll
-    for (int s = 0; s < NB2; ++s) {
+    for (int s = 0; s < S2; ++s) {
         rps[s] = U[T::RPS + qa[s]];
         rmin = fmin(rmin, sgn * rps[s]);
         rmax = fmax(rmax, sgn * rps[s]);
     }
     // a wrong sign makes rmin negative, a NaN fails the finiteness check of the weights
     const bool definite = !(rmin <= 0.0);
-    rmax = group_max_nonneg_f64<16>(fmax(rmax, 0.0));
-    const double imax = group_max_nonneg_f64<16>(definite ? 1.0 / rmin : 1e300);
+    rmax = group_max_nonneg_f64<G>(fmax(rmax, 0.0));
+    const double imax = group_max_nonneg_f64<G>(definite ? 1.0 / rmin : 1e300);
     __builtin_amdgcn_sched_barrier(0);
     // the smallest pivot is 1 / rmax, the largest imax
     bool bad = (weakest & 0x7FFFFF00u) == 0u || !definite || !(kNsPivotTol * imax * rmax < 1.0);
@@ -1111,7 +1278,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
             if (!m3 && uy == 0.0) uy = kEps;
         };
         for (int o0 = 0; o0 < ap->nops; o0 += RC) {
-            double ba[NB2][RC], bb[NB1][RC], np[NB1][RC];
+            double ba[S2][RC], bb[S1][RC], np[S1][RC];
             // kept inside the row loop: hoisted out of it, what depends on the
             // operators costs more registers than it saves work
             int kind[RC], ord[RC];
@@ -1128,125 +1295,138 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
                 u_at(L.xi[grp][2 * p], L.xi[grp][2 * p + 1], ux, uy);
                 const NsPhsAt q = ns_phs_at(mh, ux, uy);
 #pragma unroll
-                for (int o = 0; o < RC; ++o) {
+                for (int o = 0; o < RC; ++o)
                     b[o] = ns_op_phs(kind[o], ord[o], mh, ap->xk_c[min(o0 + o, ap->nops - 1)], ux, uy, hx, hy, q);
-                }
                 __builtin_amdgcn_sched_barrier(0);
             };
 #pragma unroll
-            for (int s = 0; s < NB2; ++s) rhs_at(NP + qa[s], ba[s]);
+            for (int s = 0; s < S2; ++s) rhs_at(NP + qa[s], ba[s]);
 #pragma unroll
-            for (int s = 0; s < NB1; ++s) {
+            for (int s = 0; s < S1; ++s) {
                 rhs_at(kb[s], bb[s]);
                 int q = kb[s];  // the exponents of monomial kb
                 asm volatile("" : "+v"(q));
                 const int d = (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15) + (q >= 21);
                 const int ea = q - d * (d + 1) / 2, eb = d - ea;
 #pragma unroll
-                for (int o = 0; o < RC; ++o) {
-                    np[s][o] = -ns_op_mono(kind[o], ord[o], ea, eb, px, py, hx, hy);
-                }
+                for (int o = 0; o < RC; ++o) np[s][o] = -ns_op_mono(kind[o], ord[o], ea, eb, px, py, hx, hy);
             }
             __builtin_amdgcn_sched_barrier(0);
             // the negated weights: w1n = -w0 first, w2n = 0
-            double w1n[NB1][RC], w2n[NB2][RC];
+            double w1n[S1][RC], w2n[S2][RC];
+            {
+                double src[B1][RC];
+                spread<G>(np, src);
 #pragma unroll
-            for (int s = 0; s < NB1; ++s) {
+                for (int s = 0; s < S1; ++s) {
 #pragma unroll
-                for (int o = 0; o < RC; ++o) w1n[s][o] = 0.0;
-                fb_sum<0, NP>(w1n[s], np, Pit[s]);
+                    for (int o = 0; o < RC; ++o) w1n[s][o] = 0.0;
+                    fb_sum<0, NP>(w1n[s], src, Pit[s]);
+                }
             }
 #pragma unroll
-            for (int s = 0; s < NB2; ++s)
+            for (int s = 0; s < S2; ++s)
 #pragma unroll
                 for (int o = 0; o < RC; ++o) w2n[s][o] = 0.0;
             // the solve, then one step of refinement: residual b - Phi w,
             // projected on the null space, through S^-1
 #pragma nounroll
             for (int it = 0; it < 2; ++it) {
-                double ra[NB2][RC], rb[NB1][RC];
-                int kh[NB1], qh[NB2];  // addresses formed here each time, not held in registers
+                double ra[S2][RC], rb[S1][RC];
+                int kh[S1], qh[S2];  // addresses formed here each time, not held in registers
 #pragma unroll
-                for (int s = 0; s < NB1; ++s) {
+                for (int s = 0; s < S1; ++s) {
                     kh[s] = kb[s];
                     asm volatile("" : "+v"(kh[s]));
                 }
 #pragma unroll
-                for (int s = 0; s < NB2; ++s) {
+                for (int s = 0; s < S2; ++s) {
                     qh[s] = qa[s];
                     asm volatile("" : "+v"(qh[s]));
                 }
+                {
+                    double src[B1][RC];
+                    spread<G>(w1n, src);
 #pragma unroll
-                for (int s = 0; s < NB2; ++s) {
-                    double f[NP];
+                    for (int s = 0; s < S2; ++s) {
+                        double f[NP];
 #pragma unroll
-                    for (int c = 0; c < NP; ++c) f[c] = f21(qh[s], c);
+                        for (int c = 0; c < NP; ++c) f[c] = f21(qh[s], c);
 #pragma unroll
-                    for (int o = 0; o < RC; ++o) ra[s][o] = ba[s][o];
-                    fb_sum<0, NP>(ra[s], w1n, f);
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (int o = 0; o < RC; ++o) ra[s][o] = ba[s][o];
+                        fb_sum2<NP>(ra[s], src, f);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    for_blocks<0, S1>([&](auto sc) {
+                        constexpr int s = decltype(sc)::value;
+                        double f[NP];
+                        for_blocks<0, NP>([&](auto cc) { f[decltype(cc)::value] = f11(LanesG{}, kh[s], sc, cc); });
+#pragma unroll
+                        for (int o = 0; o < RC; ++o) rb[s][o] = bb[s][o];
+                        fb_sum2<NP>(rb[s], src, f);
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
                 }
-                for_blocks<0, NB1>([&](auto sc) {
-                    constexpr int s = decltype(sc)::value;
-                    double f[NP];
-                    for_blocks<0, NP>([&](auto cc) { f[decltype(cc)::value] = f11(kh[s], sc, cc); });
-#pragma unroll
-                    for (int o = 0; o < RC; ++o) rb[s][o] = bb[s][o];
-                    fb_sum<0, NP>(rb[s], w1n, f);
-                    __builtin_amdgcn_sched_barrier(0);
-                });
                 if (it) {
-                    for_blocks<0, NB2>([&](auto sc) {
+                    double src[B2][RC];
+                    spread<G>(w2n, src);
+                    for_blocks<0, S2>([&](auto sc) {
                         constexpr int s = decltype(sc)::value;
                         double f[N2];
                         for_blocks<0, N2>([&](auto jc) { f[decltype(jc)::value] = f22(qh[s], sc, jc); });
-                        fb_sum<0, N2>(ra[s], w2n, f);
+                        fb_sum2<N2>(ra[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     });
 #pragma unroll
-                    for (int s = 0; s < NB1; ++s) {
+                    for (int s = 0; s < S1; ++s) {
                         double f[N2];
 #pragma unroll
                         for (int j = 0; j < N2; ++j) f[j] = f12(kh[s], j);
-                        fb_sum<0, N2>(rb[s], w2n, f);
+                        fb_sum2<N2>(rb[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
+                {
+                    double src[B1][RC];
+                    spread<G>(rb, src);
 #pragma unroll
-                for (int s = 0; s < NB2; ++s) fb_sum<0, NP>(ra[s], rb, nT[s]);
-                double dn[NB2][RC];
+                    for (int s = 0; s < S2; ++s) fb_sum2<NP>(ra[s], src, nT[s]);
+                }
+                double dn[S2][RC], src[B2][RC];
+                spread<G>(ra, src);
 #pragma unroll
-                for (int s = 0; s < NB2; ++s) {
+                for (int s = 0; s < S2; ++s) {
                     double y[RC];
 #pragma unroll
                     for (int o = 0; o < RC; ++o) y[o] = 0.0;
-                    fb_sum<0, N2>(y, ra, S[s]);
+                    fb_sum<0, N2>(y, src, S[s]);
 #pragma unroll
                     for (int o = 0; o < RC; ++o) {
                         dn[s][o] = -rps[s] * y[o];
                         w2n[s][o] += dn[s][o];
                     }
                 }
+                spread<G>(dn, src);
 #pragma unroll
-                for (int s = 0; s < NB1; ++s) fb_sum<0, N2>(w1n[s], dn, nTt[s]);
+                for (int s = 0; s < S1; ++s) fb_sum<0, N2>(w1n[s], src, nTt[s]);
             }
             // ---- CSR output, columns sorted by global index
 #pragma unroll
             for (int o = 0; o < RC; ++o) {
                 if (o0 + o < ap->nops) {
                     const double f = m3 ? -1.0 : -op_post_scale(kind[o], ord[o], hx, hy);
-                    double *out = ap->vals[o0 + o] + row * NN;
+                    double *out = ap->vals[o0 + o] + row * n;
 #pragma unroll
-                    for (int s = 0; s < NB2; ++s) {
-                        if (t + 16 * s < N2) {
+                    for (int s = 0; s < S2; ++s) {
+                        if (t + G * s < n2) {
                             const double wv = f * w2n[s][o];
                             bad |= !__builtin_isfinite(wv);
                             if (on) out[L.rank[grp][NP + qa[s]]] = wv;
                         }
                     }
 #pragma unroll
-                    for (int s = 0; s < NB1; ++s) {
-                        if (t + 16 * s < NP) {
+                    for (int s = 0; s < S1; ++s) {
+                        if (t + G * s < NP) {
                             const double wv = f * w1n[s][o];
                             bad |= !__builtin_isfinite(wv);
                             if (on) out[L.rank[grp][kb[s]]] = wv;
@@ -1257,30 +1437,42 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP>())) void solve_ns_kernel(
         }
         if (ap->colidx && on) {
 #pragma unroll
-            for (int s = 0; s < NB2; ++s)
-                if (t + 16 * s < N2) ap->colidx[row * NN + L.rank[grp][NP + qa[s]]] = L.g[grp][NP + qa[s]];
+            for (int s = 0; s < S2; ++s)
+                if (t + G * s < n2) ap->colidx[row * n + L.rank[grp][NP + qa[s]]] = L.g[grp][NP + qa[s]];
 #pragma unroll
-            for (int s = 0; s < NB1; ++s)
-                if (t + 16 * s < NP) ap->colidx[row * NN + L.rank[grp][kb[s]]] = L.g[grp][kb[s]];
+            for (int s = 0; s < S1; ++s)
+                if (t + G * s < NP) ap->colidx[row * n + L.rank[grp][kb[s]]] = L.g[grp][kb[s]];
         }
         if (ap->status && on && t == 0 && !ap->status_accumulate) ap->status[row] = 0;
     }
     // rows for the pivoting kernel
-    const uint64_t bb = __builtin_amdgcn_ballot_w64(bad);
-    if (((bb >> (grp * 16)) & 0xFFFFu) && live) {
-        for (int q = t; q < ny; q += 16)
-            a.redo[1 + atomicAdd(a.redo, 1)] = grouped ? a.ylist[ybase + q] : yk;
+    const uint64_t bm = __builtin_amdgcn_ballot_w64(bad);
+    if (((bm >> (grp * G)) & kGroup) && live) {
+        for (int q = t; q < ny; q += G) a.redo[1 + atomicAdd(a.redo, 1)] = grouped ? a.ylist[ybase + q] : yk;
     }
 }
 
-// One wavefront (four stencils) per block.
+// Lanes per stencil: 16 while the stencil's own rows fit one slot per lane,
+// else 32 (with two slots of 16 lanes, four stencils a wavefront hold 36 KB of
+// LDS and all 512 registers at n = 43, one wavefront per SIMD: 3.70 ms per
+// 262,144 stencils).
+constexpr int ns_lanes(int nn, int np) { return np <= 16 && nn - np <= 16 ? 16 : 32; }
+
+// One wavefront per block.
+template <int NN, int NP, int RC, bool GEN>
+void launch_ns_rc(const NsArgs &a, hipStream_t s)
+{
+    constexpr int G = ns_lanes(NN, NP);
+    const unsigned nb = (unsigned)((a.ntasks + 64 / G - 1) / (64 / G));
+    solve_ns_kernel<NN, NP, G, RC, GEN><<<nb, 64, 0, s>>>(a);
+}
+
 template <int NN, int NP>
 void launch_ns_shape(const NsArgs &a, hipStream_t s)
 {
-    const unsigned nb = (unsigned)((a.ntasks + 3) / 4);
-    if (a.nops == 1) solve_ns_kernel<NN, NP, 1><<<nb, 64, 0, s>>>(a);
-    else if (a.nops == 2) solve_ns_kernel<NN, NP, 2><<<nb, 64, 0, s>>>(a);
-    else solve_ns_kernel<NN, NP, 3><<<nb, 64, 0, s>>>(a);
+    if (a.nops == 1) launch_ns_rc<NN, NP, 1, false>(a, s);
+    else if (a.nops == 2) launch_ns_rc<NN, NP, 2, false>(a, s);
+    else launch_ns_rc<NN, NP, 3, false>(a, s);
 }
 
 }  // namespace rbffd

@@ -15,7 +15,7 @@ from rbffd_amd.nodes import jittered_grid
 pytestmark = pytest.mark.gpu
 
 # (PHS power, polynomial degree, stencil size)
-SHAPES = [(3, 3, 20), (5, 3, 21), (7, 3, 21), (7, 4, 31), (9, 4, 31)]
+SHAPES = [(3, 3, 20), (5, 3, 21), (7, 3, 21), (7, 4, 31), (9, 4, 31), (5, 5, 42), (7, 5, 43), (9, 6, 57)]
 OPS = ["E", "Dx", "Dyy", "Dxy", "Lap", "Dxk", "Dyk"]
 
 
@@ -63,7 +63,7 @@ def test_against_the_oracle(ctx, O, p, polydeg, n, kind):
         assert np.median(e) <= max(1e-13, 2 * np.median(lu))
 
 
-@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31)])
+@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31), (5, 5, 42), (9, 6, 57)])
 @pytest.mark.parametrize("nops", [1, 2, 7])
 def test_handed_back_rows(ctx, O, p, polydeg, n, nops, monkeypatch):
     """Rows whose stencil holds a duplicated or nearly duplicated node or a NaN
