@@ -102,7 +102,7 @@ enum Slot {
     S_BBOX_PART, S_BBOX, S_FLAG, S_XGROUP, S_QGROUP, S_STENCILS, S_Y2X, S_STATUS, S_ROWS, S_CSC_COUNTS,
     S_CSC_PTR, S_CSC_FILL, S_CSC_PERM, S_CSC_ROW, S_H_X, S_H_Y, S_H_COL, S_H_VALS, S_H_CVALS,
     S_H_PTR64, S_H_ROW64, S_SCAN_TMP2, S_BATCH_FLAGS, S_MORTON_KEY, S_MORTON_IDX, S_CSC_PERM_IN, S_LSQ_ROWOF, S_LSQ_TCOL, S_LSQ_TPTR, S_LSQ_F64,
-    S_LSQ_COUNT, S_LSQ_DENSE, S_LSQ_INFO, S_CLOSURE_T,
+    S_LSQ_DENSE, S_LSQ_INFO, S_CLOSURE_T,
     S_CLOSURE_PART, S_GRP_COUNTS, S_GRP_YSTART, S_GRP_FILL, S_GRP_NTASK, S_GRP_TSTART, S_GRP_YLIST, S_GRP_TASKS,
     S_GRP_TMP, S_GEN_SCRATCH, S_NS_REDO, S_NSLOT
 };
@@ -982,21 +982,44 @@ struct LsqState {
     const int64_t *tptr;
     const int *tcol;
     const double *tval;  // (D C)^T
-    double *scale, *z, *p, *s, *r, *q;
-    double *g;           // g[0], g[1]: gamma by iteration parity; g[2]: |q|^2
-    double *partial;
-    unsigned *count;
+    double *scale, *z, *r0;
+    double2 *sp[2];      // by iteration parity: s and the p before it
+    double2 *rq[2];      // r and q
+    double *g;           // g[0], g[1]: gamma by iteration parity; g[2]: the last gamma, for the host
+    double *sum_q, *sum_s;
 };
 
-// CGLS iteration k (its gamma is g[k & 1]; the next one goes to g[(k + 1) & 1])
+// The second product of iteration k: the step along p and s = (D C)^T r.  init:
+// s and its list from rq[1] alone (its q, p and the list of |q|^2 are zero).
+void lsq_second(const LsqState &S, long k, bool init, hipStream_t st)
+{
+    const int now = init ? 1 : (int)(k & 1), next = now ^ 1;
+    rbffd::LsqProduct b{};
+    b.rows = S.N; b.rowptr = S.tptr; b.col = S.tcol; b.val = S.tval;
+    b.uw = S.rq[now]; b.vnew = &S.rq[next]->x; b.y = &S.sp[next]->x; b.nv = S.M;
+    b.p = &S.sp[next]->y; b.z = S.z; b.nz = S.N;
+    b.sum_in = S.sum_q; b.nsum_in = rbffd::lsq_blocks(S.M, S.nnz); b.sum_out = S.sum_s;
+    b.gam = S.g + now;
+    rbffd::launch_lsq_product(b, S.nnz, false, st);
+}
+
+// CGLS iteration k (its gamma goes to g[k & 1])
 void lsq_iteration(const LsqState &S, long k, hipStream_t st)
 {
-    const double *gam = S.g + (k & 1);
-    double *gam_new = S.g + ((k + 1) & 1);
-    rbffd::launch_lsq_spmv(S.M, S.nnz, S.rowptr, S.col, S.dval, S.p, S.q, {S.partial, S.count, S.g + 2}, st);
-    rbffd::launch_lsq_update(S.N, S.M, gam, S.g + 2, S.p, S.q, S.z, S.r, st);
-    rbffd::launch_lsq_spmv(S.N, S.nnz, S.tptr, S.tcol, S.tval, S.r, S.s, {S.partial, S.count, gam_new}, st);
-    rbffd::launch_lsq_direction(S.N, gam, gam_new, S.s, S.p, st);
+    const int now = (int)(k & 1), next = now ^ 1;
+    rbffd::LsqProduct a{};
+    a.rows = S.M; a.rowptr = S.rowptr; a.col = S.col; a.val = S.dval;
+    a.uw = S.sp[now]; a.vnew = &S.sp[next]->y; a.y = &S.rq[now]->y; a.nv = S.N;
+    a.sum_in = S.sum_s; a.nsum_in = rbffd::lsq_blocks(S.N, S.nnz); a.sum_out = S.sum_q;
+    a.gam = S.g + now; a.gam_old = S.g + next;
+    rbffd::launch_lsq_product(a, S.nnz, true, st);
+    lsq_second(S, k, false, st);
+}
+
+// gamma of the next iteration, for the host's stopping test
+void lsq_gamma(const LsqState &S, hipStream_t st)
+{
+    rbffd::launch_lsq_sum(S.sum_s, rbffd::lsq_blocks(S.N, S.nnz), S.g + 2, st);
 }
 
 // Largest dense copy (entries) the automatic choice sends to the direct method.
@@ -1037,20 +1060,20 @@ void lsq_impl(rbffd_context *c, long M, long N, const int64_t *rowptr, const int
     int *entry = (int *)ws(c, S_CSC_ROW, sizeof(int) * nnz);
     int *tcol = (int *)ws(c, S_LSQ_TCOL, sizeof(int) * nnz);
     int64_t *tptr = (int64_t *)ws(c, S_LSQ_TPTR, sizeof(int64_t) * (N + 1));
-    const size_t nf = 2 * (size_t)nnz + 4 * (size_t)N + 2 * (size_t)M + rbffd::kLsqBlocks + 4;
+    const size_t nf = 2 * (size_t)nnz + 6 * (size_t)N + 5 * (size_t)M + 2 * rbffd::kLsqBlocks + 4;
     double *f = (double *)ws(c, S_LSQ_F64, sizeof(double) * nf);
-    unsigned *count = (unsigned *)ws(c, S_LSQ_COUNT, sizeof(unsigned) * 4);
     LsqState S;
     S.M = M; S.N = N; S.nnz = nnz; S.rowptr = rowptr; S.col = col;
-    double *dval = f, *tval = dval + nnz;
-    S.scale = tval + nnz; S.z = S.scale + N; S.p = S.z + N; S.s = S.p + N;
-    S.r = S.s + N; S.q = S.r + M; S.partial = S.q + M; S.g = S.partial + rbffd::kLsqBlocks;
-    S.dval = dval; S.tptr = tptr; S.tcol = tcol; S.tval = tval; S.count = count;
+    // the pairs come first (16-byte aligned); they, z, the list of |q|^2 and g start at zero
+    S.sp[0] = (double2 *)f; S.sp[1] = S.sp[0] + N; S.rq[0] = S.sp[1] + N; S.rq[1] = S.rq[0] + M;
+    S.z = (double *)(S.rq[1] + M); S.sum_q = S.z + N; S.g = S.sum_q + rbffd::kLsqBlocks;
+    S.sum_s = S.g + 4; S.scale = S.sum_s + rbffd::kLsqBlocks; S.r0 = S.scale + N;
+    double *dval = S.r0 + M, *tval = dval + nnz;
+    S.dval = dval; S.tptr = tptr; S.tcol = tcol; S.tval = tval;
 
     rbffd::launch_row_of(rowptr, M, row_of, st);
     rbffd::launch_fill_i32(counts, N + 1, 0, st);
     rbffd::launch_fill_i32(fill, N, 0, st);
-    rbffd::launch_fill_i32((int *)count, 4, 0, st);
     rbffd::launch_csc_count(col, nnz, counts, st);
     const size_t tb = rbffd::scan_tmp_bytes(N + 1);
     void *tmp = ws(c, S_SCAN_TMP2, tb);
@@ -1064,16 +1087,16 @@ void lsq_impl(rbffd_context *c, long M, long N, const int64_t *rowptr, const int
     rbffd::launch_scale_cols(col, nnz, S.scale, vals, dval, st);
     rbffd::launch_gather_f64(dval, perm, nnz, tval, st);       // (D C)^T
 
-    // r = b - D x0, z = 0, s = (D C)^T r, gamma0 = |s|^2, p = s
-    rbffd::launch_copy_f64(b, M, S.r, st);
-    rbffd::launch_spmv(M, rowptr, col, vals, 0, 1, x, S.r, -1.0, 1.0, 0, nullptr, st);
-    rbffd::launch_fill_f64(S.z, N, 0.0, st);
-    rbffd::launch_fill_f64(S.g, 4, 0.0, st);
-    rbffd::launch_lsq_spmv(N, nnz, tptr, tcol, tval, S.r, S.s, {S.partial, count, S.g}, st);
-    rbffd::launch_copy_f64(S.s, N, S.p, st);
+    // r = b - D x0, z = 0, s = (D C)^T r, gamma0 = |s|^2
+    rbffd::launch_copy_f64(b, M, S.r0, st);
+    rbffd::launch_spmv(M, rowptr, col, vals, 0, 1, x, S.r0, -1.0, 1.0, 0, nullptr, st);
+    rbffd::launch_fill_f64(f, 5 * N + 4 * M + rbffd::kLsqBlocks + 4, 0.0, st);
+    rbffd::launch_lsq_pair(S.r0, M, S.rq[1], st);
+    lsq_second(S, 0, true, st);
+    lsq_gamma(S, st);
     RBFFD_HIP(hipGetLastError());
     double g0 = 0.0;
-    RBFFD_HIP(hipMemcpyAsync(&g0, S.g, sizeof(double), hipMemcpyDeviceToHost, st));
+    RBFFD_HIP(hipMemcpyAsync(&g0, S.g + 2, sizeof(double), hipMemcpyDeviceToHost, st));
     RBFFD_HIP(hipStreamSynchronize(st));
     if (!std::isfinite(g0)) throw Error{RBFFD_ERR_NONFINITE, "lsq: non-finite values in D, b or x"};
 
@@ -1089,6 +1112,7 @@ void lsq_impl(rbffd_context *c, long M, long N, const int64_t *rowptr, const int
             RBFFD_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
                 for (long k = 0; k < kLsqChunk; ++k) lsq_iteration(S, k, st);
+                lsq_gamma(S, st);
                 RBFFD_HIP(hipGetLastError());
             } catch (...) {
                 // leave the stream out of capture mode
@@ -1108,11 +1132,13 @@ void lsq_impl(rbffd_context *c, long M, long N, const int64_t *rowptr, const int
                 const long k = std::min(kLsqChunk, max_iters - done);
                 if (exec && k == kLsqChunk)
                     RBFFD_HIP(hipGraphLaunch(exec, st));
-                else
+                else {
                     for (long j = 0; j < k; ++j) lsq_iteration(S, done + j, st);
+                    lsq_gamma(S, st);
+                }
                 done += k;
                 double g = 0.0;
-                RBFFD_HIP(hipMemcpyAsync(&g, S.g + (done & 1), sizeof(double), hipMemcpyDeviceToHost, st));
+                RBFFD_HIP(hipMemcpyAsync(&g, S.g + 2, sizeof(double), hipMemcpyDeviceToHost, st));
                 RBFFD_HIP(hipStreamSynchronize(st));
                 if (!std::isfinite(g)) throw Error{RBFFD_ERR_NONFINITE, "lsq: non-finite iterate"};
                 rel = std::sqrt(g / g0);

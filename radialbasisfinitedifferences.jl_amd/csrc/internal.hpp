@@ -285,23 +285,32 @@ struct CombineTerms {
 void launch_combine(long nnz, const CombineTerms &t, double *out, float *out32, hipStream_t s);
 
 // --------------------------------------------------- sparse solve (CGLS)
-// Grid-wide sum target: block sums go to partial[kLsqBlocks], the counter is
-// zero between launches, the total lands in *out.
-constexpr int kLsqBlocks = 1024;
-struct LsqReduce {
-    double *partial;
-    unsigned *count;
-    double *out;
+// One of the two products of a CGLS iteration (lsq.hip): y = A (u + c w) over
+// CSR rows and pairs (u, w), the vector stored in vnew, block sums of y^2 in
+// sum_out; c from the sum of a previous product's list sum_in and the gammas.
+// vnew, y and p are halves of pairs (stride 2).
+constexpr int kLsqBlocks = 1024;  // longest list: every CU full, and two loads a thread to add up
+struct LsqProduct {
+    long rows;
+    const int64_t *rowptr;
+    const int *col;
+    const double *val;
+    const double2 *uw;
+    double *vnew, *y;
+    long nv;
+    const double *p;      // second product: z -= c p
+    double *z;
+    long nz;
+    const double *sum_in;
+    int nsum_in;
+    double *sum_out;
+    double *gam;
+    const double *gam_old;
 };
-// y = A x (CSR, int64 rowptr) and |y|^2 -> *red.out
-void launch_lsq_spmv(long M, long nnz, const int64_t *rowptr, const int *col, const double *val, const double *x,
-                     double *y, const LsqReduce &red, hipStream_t s);
-// z += a p, r -= a q with a = *gam / *qq
-void launch_lsq_update(long N, long M, const double *gam, const double *qq, const double *p, const double *q,
-                       double *z, double *r, hipStream_t s);
-// p = s + (*gam_new / *gam) p
-void launch_lsq_direction(long N, const double *gam, const double *gam_new, const double *sv, double *p,
-                          hipStream_t s);
+int lsq_blocks(long rows, long nnz);  // length of a product's list
+void launch_lsq_product(const LsqProduct &a, long nnz, bool first, hipStream_t s);
+void launch_lsq_pair(const double *x, long n, double2 *out, hipStream_t s);
+void launch_lsq_sum(const double *partial, int n, double *out, hipStream_t s);
 void launch_row_of(const int64_t *rowptr, long M, int *row_of, hipStream_t s);
 void launch_gather_i32(const int *src, const int *idx, long n, int *dst, hipStream_t s);
 void launch_col_scale(const int64_t *tptr, long N, const double *tval, double *scale, hipStream_t s);

@@ -5,16 +5,20 @@
 //
 // The solver is CGLS (conjugate gradients on the normal equations,
 // Hestenes-Stiefel form) on the column-equilibrated matrix D~ = D C,
-// C = diag(1 / ||D e_j||), with x = x0 + C z.  One iteration is four kernels:
-//   1. q = D~ p                     and |q|^2
-//   2. z += a p, r -= a q           a = gamma / |q|^2
-//   3. s = D~^T r                   and gamma' = |s|^2
-//   4. p = s + (gamma' / gamma) p
+// C = diag(1 / ||D e_j||), with x = x0 + C z.  One iteration is two kernels:
+//   1. p = s + (gamma / gamma_old) p,  q = D~ p,              |q|^2
+//   2. a = gamma / |q|^2,  z += a p,  r -= a q,  s = D~^T r,  gamma' = |s|^2
+// Each product forms the vector it gathers from (p, r) entry by entry as it
+// reads it, with the rounding of the stored copy that the kernel also writes.
 // D~^T is stored as a CSR of its own, so both products are row gathers with
-// no atomics.  Squared norms use a two-level sum in a fixed order (block sums,
-// then the last block to finish adds them in block order), so a solve is
-// bitwise reproducible.  The scalars stay in device memory: no iteration
-// waits for the host.
+// no atomics.  The systems are small (3.8 MB of D at 10,201 x 2,601): an
+// iteration is bound by its dependent launches, not by bytes.  A kernel leaves
+// its block sums of a squared norm in a list that every block of the next one
+// adds up in the same order (at most 1,024 values: two loads a thread), so there
+// is no fence, counter or last block, the scalars never leave the device and a
+// solve is bitwise reproducible.  Four kernels an iteration with a last-block
+// sum in the two products took 12 + 5 + 12 + 5 us, 31 us an iteration; the two
+// take 4.4 + 4.8 us, 10.3 us an iteration (10,201 x 2,601, 204,020 entries).
 //
 // For systems whose dense copy fits the device, the direct method writes D
 // into a column-major dense array and calls rocSOLVER's QR least-squares
@@ -40,121 +44,146 @@ __device__ __forceinline__ double wave_sum_f64(double v)
     return v;
 }
 
-// Sum of v over the grid (256 threads a block).  Each block stores its sum in
-// partial[blockIdx.x]; the last block to arrive adds the block sums in block
-// order, writes the total to *out and re-arms the counter.
-__device__ void grid_sum_finish(double v, const LsqReduce &r)
+constexpr int kLsqThreads = 512;
+
+// Sum of v over the block, in every thread (fixed order)
+__device__ __forceinline__ double block_sum(double v)
 {
-    __shared__ double wsum[4];
-    __shared__ int last;
-    const int w = threadIdx.x >> 6;
+    __shared__ double wsum[kLsqThreads / 64];
     v = wave_sum_f64(v);
-    if ((threadIdx.x & 63) == 0) wsum[w] = v;
+    __syncthreads();  // wsum may still be read from an earlier sum
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        r.partial[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-        __threadfence();
-        const unsigned t = atomicAdd(r.count, 1u);
-        last = t == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
     double s = 0.0;
-    for (unsigned i = threadIdx.x; i < gridDim.x; i += blockDim.x)
-        s += __hip_atomic_load(&r.partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s = wave_sum_f64(s);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) wsum[w] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        *r.out = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-        atomicExch(r.count, 0u);
-    }
+#pragma unroll
+    for (int w = 0; w < kLsqThreads / 64; ++w) s += wsum[w];
+    return s;
 }
 
-// y = A x over CSR rows, G lanes a row, and |y|^2 into *red.out.  Waves walk
-// the rows in passes of 64 / G rows (a wave-uniform loop, so the lane-group
-// sums always run with the whole wave).
-template <int G>
-__global__ __launch_bounds__(256) void lsq_spmv_kernel(long M, const int64_t *__restrict__ rowptr,
-                                                       const int *__restrict__ col, const double *__restrict__ val,
-                                                       const double *__restrict__ x, double *__restrict__ y,
-                                                       LsqReduce red)
+__device__ __forceinline__ double list_sum(const double *partial, int n)
 {
-    constexpr int RPW = 64 / G;
+    double v = 0.0;
+    for (int i = threadIdx.x; i < n; i += kLsqThreads) v += partial[i];
+    return block_sum(v);
+}
+
+// One product of an iteration over CSR rows, G lanes a row: with
+// v = x + c y of the pairs uw formed where they are read (one 16-byte load an
+// entry: two loads took 203 against 196 us an iteration at 640,000 x 160,000),
+// A v and the block sums of its squares to sum_out; v itself is stored too.
+//   FIRST: pairs (s, p), v the new p, A v = q, c = gamma / gamma_old (gamma: the
+//     sum of sum_in, also kept in *gam; *gam_old is 0 for the first step);
+//   else:  pairs (r, q), v the new r, A v = s, c = -gamma / |q|^2 (|q|^2: the sum
+//     of sum_in), and z -= c p.
+// The outputs are halves of pairs as well: stride 2.
+// A wave walks its rows in passes of 64 / G (a wave-uniform loop, so the
+// lane-group sums always run with the whole wave).
+template <int G, bool FIRST>
+__global__ __launch_bounds__(kLsqThreads) void lsq_product_kernel(LsqProduct a)
+{
+    constexpr int RPW = 64 / G, PRE = 2;
+    const long tid = blockIdx.x * (long)kLsqThreads + threadIdx.x, nthreads = (long)gridDim.x * kLsqThreads;
     const int lane = threadIdx.x & 63, sub = lane % G;
-    const long wave = (blockIdx.x * (long)blockDim.x + threadIdx.x) >> 6;
-    const long stride = (long)gridDim.x * (blockDim.x >> 6) * RPW;
+    const long base0 = (tid >> 6) * RPW, stride = (nthreads >> 6) * RPW;
+    // the first row's first entries do not need c: their chain of loads
+    // (row pointer, column, vector) runs beside the sum's (0.5 us of 5.4)
+    long p0 = 0, p1 = 0;
+    double fv[PRE];
+    double2 fx[PRE];
+    if (base0 + lane / G < a.rows) { p0 = a.rowptr[base0 + lane / G]; p1 = a.rowptr[base0 + lane / G + 1]; }
+#pragma unroll
+    for (int e = 0; e < PRE; ++e) {
+        const long p = p0 + sub + G * e;
+        fv[e] = 0.0;
+        fx[e] = double2{0.0, 0.0};
+        if (p < p1) {
+            fv[e] = a.val[p];
+            fx[e] = a.uw[a.col[p]];
+        }
+    }
+    const double total = list_sum(a.sum_in, a.nsum_in);
+    double c;
+    if constexpr (FIRST) {
+        const double old = *a.gam_old;
+        c = old > 0.0 ? total / old : 0.0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.gam = total;
+    } else {
+        c = total > 0.0 ? -(*a.gam / total) : 0.0;
+    }
+    for (long i = tid; i < a.nv; i += nthreads) {
+        const double2 x = a.uw[i];
+        a.vnew[2 * i] = __builtin_fma(c, x.y, x.x);
+    }
+    if constexpr (!FIRST)
+        for (long i = tid; i < a.nz; i += nthreads) a.z[i] = __builtin_fma(-c, a.p[2 * i], a.z[i]);
     double sq = 0.0;
-    for (long base = wave * RPW; base < M; base += stride) {
+    for (long base = base0; base < a.rows; base += stride) {
         const long row = base + lane / G;
-        const bool live = row < M;
-        long p0 = 0, p1 = 0;
-        if (live) { p0 = rowptr[row]; p1 = rowptr[row + 1]; }
+        const bool live = row < a.rows;
         double acc = 0.0;
-        for (long p = p0 + sub; p < p1; p += G) acc = __builtin_fma(val[p], x[col[p]], acc);
-        acc = group_sum_f64<G>(acc);
+        long p = 0, end = 0;
+        if (base == base0) {
+#pragma unroll
+            for (int e = 0; e < PRE; ++e)
+                if (p0 + sub + G * e < p1) acc = __builtin_fma(fv[e], __builtin_fma(c, fx[e].y, fx[e].x), acc);
+            p = p0 + sub + G * PRE;
+            end = p1;
+        } else if (live) {
+            p = a.rowptr[row] + sub;
+            end = a.rowptr[row + 1];
+        }
+        for (; p < end; p += G) {
+            const double2 x = a.uw[a.col[p]];
+            acc = __builtin_fma(a.val[p], __builtin_fma(c, x.y, x.x), acc);
+        }
+        acc = G == 64 ? wave_sum_f64(acc) : group_sum_f64<G == 64 ? 32 : G>(acc);
         if (live && sub == 0) {
-            y[row] = acc;
+            a.y[2 * row] = acc;
             sq = __builtin_fma(acc, acc, sq);
         }
     }
-    grid_sum_finish(sq, red);
+    sq = block_sum(sq);
+    if (threadIdx.x == 0) a.sum_out[blockIdx.x] = sq;
 }
 
-static int lsq_lanes(long rows, long nnz) { return (rows > 0 && nnz / rows < 12) ? 8 : 16; }
-
-static unsigned lsq_spmv_blocks(long M, int G)
+// *out = the sum of a list of block sums
+__global__ __launch_bounds__(kLsqThreads) void lsq_sum_kernel(const double *partial, int n, double *out)
 {
-    const long b = (M * G + 255) / 256;
-    return (unsigned)std::max<long>(1, std::min<long>(kLsqBlocks, b));
+    const double s = list_sum(partial, n);
+    if (threadIdx.x == 0) *out = s;
 }
 
-void launch_lsq_spmv(long M, long nnz, const int64_t *rowptr, const int *col, const double *val, const double *x,
-                     double *y, const LsqReduce &red, hipStream_t s)
+void launch_lsq_sum(const double *partial, int n, double *out, hipStream_t s)
 {
-    // M == 0 still launches one block so that *red.out is written (0)
-    if (lsq_lanes(M, nnz) == 8)
-        lsq_spmv_kernel<8><<<lsq_spmv_blocks(M, 8), 256, 0, s>>>(M, rowptr, col, val, x, y, red);
-    else
-        lsq_spmv_kernel<16><<<lsq_spmv_blocks(M, 16), 256, 0, s>>>(M, rowptr, col, val, x, y, red);
+    lsq_sum_kernel<<<1, kLsqThreads, 0, s>>>(partial, n, out);
 }
 
-static unsigned blocks_of(long n) { return (unsigned)std::max<long>(1, std::min<long>(65535L * 16, (n + 255) / 256)); }
-
-// z += a p (N entries), r -= a q (M entries), a = gamma / |q|^2
-__global__ void lsq_update_kernel(long N, long M, const double *__restrict__ gam, const double *__restrict__ qq,
-                                  const double *__restrict__ p, const double *__restrict__ q, double *__restrict__ z,
-                                  double *__restrict__ r)
+// Lanes per row: two passes or so over an average row.
+static int lsq_lanes(long rows, long nnz)
 {
-    const double a = *qq > 0.0 ? *gam / *qq : 0.0;
-    const long n = N > M ? N : M;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        if (i < N) z[i] = __builtin_fma(a, p[i], z[i]);
-        if (i < M) r[i] = __builtin_fma(-a, q[i], r[i]);
+    const long avg = rows > 0 ? nnz / rows : 0;
+    return avg < 12 ? 8 : (avg < 64 ? 16 : 64);
+}
+
+int lsq_blocks(long rows, long nnz)
+{
+    const long b = (rows * lsq_lanes(rows, nnz) + kLsqThreads - 1) / kLsqThreads;
+    return (int)std::max<long>(1, std::min<long>(kLsqBlocks, b));
+}
+
+void launch_lsq_product(const LsqProduct &a, long nnz, bool first, hipStream_t s)
+{
+    const unsigned nb = (unsigned)lsq_blocks(a.rows, nnz);
+    const int g = lsq_lanes(a.rows, nnz);
+    if (first) {
+        if (g == 8) lsq_product_kernel<8, true><<<nb, kLsqThreads, 0, s>>>(a);
+        else if (g == 16) lsq_product_kernel<16, true><<<nb, kLsqThreads, 0, s>>>(a);
+        else lsq_product_kernel<64, true><<<nb, kLsqThreads, 0, s>>>(a);
+    } else {
+        if (g == 8) lsq_product_kernel<8, false><<<nb, kLsqThreads, 0, s>>>(a);
+        else if (g == 16) lsq_product_kernel<16, false><<<nb, kLsqThreads, 0, s>>>(a);
+        else lsq_product_kernel<64, false><<<nb, kLsqThreads, 0, s>>>(a);
     }
-}
-
-void launch_lsq_update(long N, long M, const double *gam, const double *qq, const double *p, const double *q,
-                       double *z, double *r, hipStream_t s)
-{
-    lsq_update_kernel<<<blocks_of(std::max(N, M)), 256, 0, s>>>(N, M, gam, qq, p, q, z, r);
-}
-
-// p = s + (gamma' / gamma) p
-__global__ void lsq_direction_kernel(long N, const double *__restrict__ gam, const double *__restrict__ gam_new,
-                                     const double *__restrict__ sv, double *__restrict__ p)
-{
-    const double b = *gam > 0.0 ? *gam_new / *gam : 0.0;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x)
-        p[i] = __builtin_fma(b, p[i], sv[i]);
-}
-
-void launch_lsq_direction(long N, const double *gam, const double *gam_new, const double *sv, double *p,
-                          hipStream_t s)
-{
-    if (N > 0) lsq_direction_kernel<<<blocks_of(N), 256, 0, s>>>(N, gam, gam_new, sv, p);
 }
 
 // ---- set-up and finish
@@ -208,6 +237,18 @@ __global__ void scale_cols_kernel(const int *col, long nnz, const double *scale,
 void launch_scale_cols(const int *col, long nnz, const double *scale, const double *v, double *out, hipStream_t s)
 {
     if (nnz > 0) scale_cols_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, s>>>(col, nnz, scale, v, out);
+}
+
+// out = (x, 0) pairs
+__global__ void lsq_pair_kernel(const double *x, long n, double2 *out)
+{
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i < n) out[i] = double2{x[i], 0.0};
+}
+
+void launch_lsq_pair(const double *x, long n, double2 *out, hipStream_t s)
+{
+    if (n > 0) lsq_pair_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(x, n, out);
 }
 
 // y = x (n entries)

@@ -146,3 +146,49 @@ def test_rank_deficient_and_bad_arguments(ctx):
         rbffd_amd.solve(sp.random(5, 9, density=0.5, format="csr"), np.ones(5), ctx=ctx)   # M < N
     with pytest.raises(rbffd_amd.NonFiniteError):
         rbffd_amd.solve(sp.eye(6, format="csr") * np.nan, np.ones(6), method="cgls", ctx=ctx)
+
+
+@pytest.mark.parametrize("M,N,per_row", [(1, 1, 1), (7, 3, 2), (600, 500, 5), (520, 33, 20), (9000, 400, 11)])
+@pytest.mark.parametrize("iters", [3, 33, 400])
+def test_cgls_iterates(ctx, M, N, per_row, iters):
+    """The CGLS kernels at every lane count (8, 16 and 64 lanes a row: rows and
+    columns of 1 to a few hundred entries), with rows past a block's first
+    pass, empty rows, and iteration counts that are no multiple of the
+    recorded chunk: the iterate equals CGLS in numpy.  Bar: both run the same
+    recurrence in FP64 on systems with condition numbers below 50, so their
+    iterates stay within a small multiple of 50^2 times rounding: 1e-11."""
+    import rbffd_amd
+
+    rng = np.random.default_rng(M + iters)
+    D = sp.random(M, N, density=min(1.0, per_row / N), random_state=rng, format="csr", data_rvs=rng.standard_normal)
+    D = (D * 0.3 + sp.eye(M, N)).tocsr()
+    if M > 8:
+        D = sp.vstack([D, sp.csr_matrix((5, N))]).tocsr()
+    b = rng.standard_normal(D.shape[0])
+    A = D.toarray()
+    C = 1.0 / np.linalg.norm(A, axis=0)
+    A = A * C
+    print(f"CGLS {D.shape}, {D.nnz} entries, {iters} iterations, cond {np.linalg.cond(A):.1f}", flush=True)
+    r = b.copy()
+    z = np.zeros(N)
+    s = A.T @ r
+    p, gam = s.copy(), s @ s
+    g0, done = gam, 0
+    while done < iters and gam > 0 and np.sqrt(gam / g0) > 1e-14:
+        for _ in range(min(32, iters - done)):
+            if gam <= 1e-30 * g0:  # converged to rounding: later steps are 0 / 0 here
+                done += 1
+                continue
+            q = A @ p
+            a = gam / (q @ q) if q @ q > 0 else 0.0
+            z += a * p
+            r -= a * q
+            s = A.T @ r
+            new = s @ s
+            p = s + (new / gam if gam > 0 else 0.0) * p
+            gam = new
+            done += 1
+    x, (its, rel) = rbffd_amd.solve(D, b, method="cgls", tol=1e-14, max_iters=iters, ctx=ctx, info=True)
+    assert its <= iters
+    assert np.linalg.cond(A) < 50
+    assert _rel(x, C * z) <= 1e-11
