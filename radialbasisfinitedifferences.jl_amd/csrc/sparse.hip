@@ -19,6 +19,7 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "spmm_rows.hpp"
 
 namespace rbffd {
 
@@ -242,6 +243,74 @@ static void spmm_split_launch_t(long M, const int64_t *rowptr, const int *col, c
         spmm_split_kernel<TV, F, FL, false><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, x, y, alpha, beta);
 }
 
+// 8 fields, 16 lanes a row (row_times_8).  MODE 0: y = alpha A x + beta y;
+// MODE 1: one Shu-Osher stage y = a u + b x + c (A x), rows with fixed[r] != 0
+// keeping u (y may be u: the same lane reads and writes a value).
+struct RowsOut {
+    double *y;
+    double alpha, beta;
+    const double *u;
+    const uint8_t *fixed;
+    double a, b, c;
+};
+
+template <typename TV, bool UNIFORM, int MODE>
+__global__ __launch_bounds__(256) void spmm_rows_kernel(long M, const int64_t *__restrict__ rowptr,
+                                                        const int *__restrict__ col, const TV *__restrict__ val,
+                                                        int n_uniform, const int *__restrict__ order,
+                                                        const double *__restrict__ x, RowsOut o)
+{
+    constexpr int F = 8;
+    const int sub = threadIdx.x & 15, f0 = 2 * (sub & 3);
+    const long g = blockIdx.x * 16L + (threadIdx.x >> 4);
+    // rows past the end still take part in the broadcasts
+    const bool live = g < M;
+    const long row = !live ? 0 : (order ? (long)order[g] : g);
+    long p0 = 0;
+    int len = 0, most;
+    bool full;
+    if (UNIFORM) {
+        p0 = row * (long)n_uniform;
+        len = live ? n_uniform : 0;
+        most = n_uniform;
+        full = __builtin_amdgcn_ballot_w64(live) == ~0ull;
+    } else {
+        if (live) {
+            p0 = rowptr[row];
+            len = (int)(rowptr[row + 1] - p0);
+        }
+        rows_extent(len, most, full);
+    }
+    double acc[2];
+    row_times_8(acc, val + p0, col + p0, len, most, full, x);
+    if (live && sub < 4) {
+        const long e = row * F + f0;
+        const bool hold = MODE == 1 && o.fixed && o.fixed[row];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            if constexpr (MODE == 0) {
+                double r = o.alpha * acc[f];
+                if (o.beta != 0.0) r = __builtin_fma(o.beta, o.y[e + f], r);
+                o.y[e + f] = r;
+            } else {
+                const double ui = o.u[e + f];
+                o.y[e + f] = hold ? ui : o.a * ui + o.b * x[e + f] + o.c * acc[f];
+            }
+        }
+    }
+}
+
+template <typename TV, int MODE>
+static void spmm_rows_t(long M, const int64_t *rowptr, const int *col, const TV *val, int nu, const int *order,
+                        const double *x, const RowsOut &o, hipStream_t s)
+{
+    const unsigned blocks = (unsigned)((M + 15) / 16);
+    if (nu > 0)
+        spmm_rows_kernel<TV, true, MODE><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, x, o);
+    else
+        spmm_rows_kernel<TV, false, MODE><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, x, o);
+}
+
 template <typename TV, int G, int F>
 static void spmv_launch_t(long M, const int64_t *rowptr, const int *col, const TV *val, int nu, const int *order,
                           const double *x, double *y, double alpha, double beta, hipStream_t s)
@@ -281,14 +350,24 @@ static void spmv_dispatch(long M, const int64_t *rowptr, const int *col, const T
 {
     static const int g1 = lanes_env("RBFFD_SPMV_LANES", 16);
     static const int gf = lanes_env("RBFFD_SPMM_LANES", 16);
-    // lanes sharing a nonzero: RBFFD_SPMM_FL = 1 | 2 | 4 | 8; by default 2
-    // from 4 fields up (8 fields over 1M nodes, n = 31: 189 us against 212 us with
-    // every field in every lane; 4 and 8 lanes were slower)
+    // lanes sharing a nonzero: RBFFD_SPMM_FL = 1 | 2 | 4 | 8; by default 2 at 4
+    // fields, and at 8 fields the quads of spmm_rows_kernel (1M nodes, n = 31: 145
+    // us against 181 with 2 lanes, 212 with every field in every lane; 4 and 8
+    // lanes were slower.  Quads at 4 fields: 140 against 142 us, but 130 against 111
+    // with FP32 values, where a load of one field a lane is mostly address)
     static const int fl_env = [] {
         const char *e = std::getenv("RBFFD_SPMM_FL");
         const int v = e ? std::atoi(e) : 0;
         return (v == 1 || v == 2 || v == 4 || v == 8) ? v : 0;
     }();
+    if (F == 8 && gf == 16 && fl_env == 0) {
+        RowsOut o{};
+        o.y = y;
+        o.alpha = alpha;
+        o.beta = beta;
+        spmm_rows_t<TV, 0>(M, rowptr, col, val, nu, order, x, o, s);
+        return;
+    }
     const int fl = fl_env ? fl_env : (F >= 4 ? 2 : 1);
     if (F >= 2 && gf == 16 && fl > 1 && fl <= F) {
         auto go = [&](auto fc, auto flc) {
@@ -369,6 +448,7 @@ void launch_morton_order(const double *X, long N, const double *box, uint32_t *k
 // One Shu-Osher stage: out = a u + b w + c (L w) for F fields, L in CSR with
 // G lanes per row (as spmv_kernel).  Rows with fixed[r] != 0 keep u.  out may
 // be u (each value is read and written by the same lane); out must not be w.
+// (1 to 4 fields; 8 run spmm_rows_kernel.)
 template <typename TV, int G, int F, int FL, bool UNIFORM>
 __global__ __launch_bounds__(256) void rk_stage_kernel(long M, const int64_t *__restrict__ rowptr,
                                                        const int *__restrict__ col, const TV *__restrict__ val,
@@ -436,16 +516,28 @@ static void rk_stage_t(long M, const int64_t *rowptr, const int *col, const TV *
                        const double *w, const double *u, double *out, const uint8_t *fixed, double a, double b,
                        double c, hipStream_t s)
 {
-    constexpr int G = 16;
-    // two lanes per nonzero from 4 fields up, as the SpMM
-    constexpr int FL = F >= 4 ? 2 : 1;
-    const unsigned blocks = (unsigned)((M * G + 255) / 256);
-    if (nu > 0)
-        rk_stage_kernel<TV, G, F, FL, true><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, w, u, out, fixed,
-                                                                   a, b, c);
-    else
-        rk_stage_kernel<TV, G, F, FL, false><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, w, u, out,
-                                                                    fixed, a, b, c);
+    if constexpr (F == 8) {
+        RowsOut o{};
+        o.y = out;
+        o.u = u;
+        o.fixed = fixed;
+        o.a = a;
+        o.b = b;
+        o.c = c;
+        spmm_rows_t<TV, 1>(M, rowptr, col, val, nu, order, w, o, s);
+        return;
+    } else {
+        constexpr int G = 16;
+        // two lanes per nonzero at 4 fields, as the SpMM
+        constexpr int FL = F == 4 ? 2 : 1;
+        const unsigned blocks = (unsigned)((M * G + 255) / 256);
+        if (nu > 0)
+            rk_stage_kernel<TV, G, F, FL, true><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, w, u, out, fixed,
+                                                                       a, b, c);
+        else
+            rk_stage_kernel<TV, G, F, FL, false><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, w, u, out,
+                                                                        fixed, a, b, c);
+    }
 }
 
 template <typename TV>

@@ -1,9 +1,11 @@
 // spmv_plan.hip -- K4 for repeated products with one operator: an
 // application plan that stages each workgroup's x rows in LDS.
 //
-// The plain kernels (sparse.hip) gather a node's F fields from HBM/L2 once
-// per nonzero, so a product with 8 fields issues about 4 vector-memory loads
-// per nonzero and is bound by the texture address path of the L1, not by HBM.
+// The plain kernels (sparse.hip) gather a node's fields from L1/L2 once per
+// nonzero and are bound by the L1's address path, not by HBM.  Up to 4 fields a
+// plan takes x from LDS instead; 8 fields run in the plan's order of rows with x
+// gathered as the plain product does (plan_rows_kernel).
+//
 // A plan cuts the rows, in a locality order (Morton order of the rows' nodes
 // for RBF-FD operators), into blocks of kPlanRows consecutive rows and lists
 // each block's distinct columns (its halo, sorted).  Its nonzeros then refer to
@@ -12,9 +14,10 @@
 // consecutive nodes on structured node sets) and reads x from LDS per nonzero.
 //
 // Each row's nonzeros keep their order, and lanes take them and reduce across
-// DPP exactly as spmv_kernel / spmm_split_kernel / rk_stage_kernel do, so a
-// plan product is bitwise equal to the plain one with the default lane layout
-// (16 lanes a row; two lanes a nonzero from 4 fields up).
+// DPP exactly as spmv_kernel / spmm_split_kernel / spmm_rows_kernel /
+// rk_stage_kernel do, so a plan product is bitwise equal to the plain one with
+// the default lane layout (16 lanes a row; two lanes a nonzero at 4 fields, a
+// quad at 8).
 //
 // Replaces SparseMatrixCSC * Vector of the reference's harnesses
 // (test/poisson_test.jl:121, examples/adv_diff_test.jl:151-152) where one
@@ -27,6 +30,7 @@
 
 #include "device_common.hpp"
 #include "internal.hpp"
+#include "spmm_rows.hpp"
 
 namespace rbffd {
 
@@ -174,7 +178,7 @@ struct PlanOut {
 
 // LDS stride of a staged x row, in doubles: F + 2 from 2 fields up, so rows
 // that a wavefront reads at once spread over the banks (at a stride of F
-// doubles, 8 fields, its 32 rows hit only 4 bank offsets) and stay 16-byte
+// doubles, 4 fields, its 32 rows hit only 8 bank offsets) and stay 16-byte
 // aligned for the staging stores
 template <int F>
 constexpr int plan_lds_stride() { return F == 1 ? 1 : F + 2; }
@@ -324,23 +328,81 @@ __global__ __launch_bounds__(NT) void plan_apply_kernel(long M, int nu, const in
     }
 }
 
+// 8 fields: the rows by row_times_8, x gathered through the columns as the plain
+// product does.  Over a million rows of 31 in turn with two lanes a nonzero and
+// x in LDS (a halo of about 450 nodes staged for 256 rows, then one barrier): 144
+// us against 158, FP32 values 140 against 149; 57 entries a row, FP32, 230 against
+// 229.  The same sum from LDS took 203, and through 16-bit slots of the halo's
+// list 187.  Three RK stages of four million rows: 2.18 ms against 2.90, FP32 2.14
+// against 2.71.
+template <typename TV, bool UNIFORM, int MODE>
+__global__ __launch_bounds__(256) void plan_rows_kernel(long M, int nu, const int *__restrict__ prow,
+                                                        const int64_t *__restrict__ pptr,
+                                                        const int *__restrict__ pcol, const TV *__restrict__ pval,
+                                                        const double *__restrict__ x, PlanOut o)
+{
+    constexpr int F = 8;
+    const int sub = threadIdx.x & 15, f0 = 2 * (sub & 3);
+    const long i = blockIdx.x * 16L + (threadIdx.x >> 4);
+    const bool live = i < M;
+    long p0 = 0, row = 0;
+    int len = 0, most;
+    bool full;
+    if (live) {
+        p0 = UNIFORM ? i * (long)nu : pptr[i];
+        len = UNIFORM ? nu : (int)(pptr[i + 1] - p0);
+        row = prow[i];
+    }
+    if (UNIFORM) {
+        most = nu;
+        full = __builtin_amdgcn_ballot_w64(live) == ~0ull;
+    } else {
+        rows_extent(len, most, full);
+    }
+    double acc[2];
+    row_times_8(acc, pval + p0, pcol + p0, len, most, full, x);
+    if (live && sub < 4) {
+        const long e = row * F + f0;
+        const bool hold = MODE == 1 && o.fixed && o.fixed[row];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            if constexpr (MODE == 0) {
+                double t = o.alpha * acc[f];
+                if (o.beta != 0.0) t = __builtin_fma(o.beta, o.y[e + f], t);
+                o.y[e + f] = t;
+            } else {
+                const double ui = o.u[e + f];
+                o.y[e + f] = hold ? ui : o.a * ui + o.b * x[e + f] + o.c * acc[f];
+            }
+        }
+    }
+}
+
 template <typename TV, int F, int MODE>
 void plan_apply_t(const SpmvPlan &P, const double *x, const PlanOut &o, hipStream_t s)
 {
-    constexpr int FL = F >= 4 ? 2 : 1, SX = plan_lds_stride<F>();
-    // LDS for the largest listed halo, at most 64 KiB a workgroup
-    const int cap = std::min(P.hmax, (int)(65536 / (sizeof(double) * SX)));
-    const size_t lds = sizeof(double) * SX * (size_t)std::max(cap, 1);
-    const bool x16 = ((uintptr_t)x & 15) == 0;
-    // 1024 lanes a block from 4 fields up (at 8 fields 161-168 us per product
-    // over 1M rows, against 318 us with 256 lanes a block), 256 below
-    constexpr int NT = F >= 4 ? 1024 : 256;
-    // rows a lane group takes per pass: two up to 2 fields (one field: 85-86 us
-    // against 95), one from 4 fields up (two rows: 8 fields no faster, and an
-    // FP32 SSP-RK3 run 17% slower)
-    constexpr int RPP = F >= 4 ? 1 : 2;
-    plan_apply_kernel<TV, F, FL, MODE, NT, RPP><<<P.nblocks, NT, lds, s>>>(
-        P.M, P.uniform, P.prow, P.pptr, P.plc, P.pcol, (const TV *)P.pval, P.halo, P.hcount, cap, x16, x, o);
+    if constexpr (F == 8) {
+        const unsigned blocks = (unsigned)((P.M + 15) / 16);
+        auto go = [&](auto un) {
+            plan_rows_kernel<TV, decltype(un)::value, MODE>
+                <<<blocks, 256, 0, s>>>(P.M, P.uniform, P.prow, P.pptr, P.pcol, (const TV *)P.pval, x, o);
+        };
+        if (P.uniform > 0) go(std::true_type{});
+        else go(std::false_type{});
+    } else {
+        constexpr int FL = F == 4 ? 2 : 1, SX = plan_lds_stride<F>();
+        // LDS for the largest listed halo, at most 64 KiB a workgroup
+        const int cap = std::min(P.hmax, (int)(65536 / (sizeof(double) * SX)));
+        const size_t lds = sizeof(double) * SX * (size_t)std::max(cap, 1);
+        const bool x16 = ((uintptr_t)x & 15) == 0;
+        // 1024 lanes a block at 4 fields, 256 below
+        constexpr int NT = F == 4 ? 1024 : 256;
+        // rows a lane group takes per pass: two up to 2 fields (one field: 85-86
+        // us against 95), one at 4
+        constexpr int RPP = F == 4 ? 1 : 2;
+        plan_apply_kernel<TV, F, FL, MODE, NT, RPP><<<P.nblocks, NT, lds, s>>>(
+            P.M, P.uniform, P.prow, P.pptr, P.plc, P.pcol, (const TV *)P.pval, P.halo, P.hcount, cap, x16, x, o);
+    }
 }
 
 template <int MODE>
@@ -426,10 +488,6 @@ void spmv_plan_build(SpmvPlan &P, long M, long N, const int64_t *rowptr, const i
         RBFFD_HIP(hipStreamSynchronize(s));
         P.hmax = h[0];
         P.overflow_blocks = h[1];
-        if (P.overflow_blocks == 0) {  // every block reads x through its halo list
-            (void)hipFree(P.pcol);
-            P.pcol = nullptr;
-        }
     } catch (...) {
         spmv_plan_free(P);
         throw;

@@ -53,6 +53,43 @@ def test_spmv_matches_oracle(ctx, O, F, vtype):
     assert np.array_equal(y3.get(), y)
 
 
+@pytest.mark.parametrize("M", [1, 15, 17, 70])
+@pytest.mark.parametrize("vtype", ["f64", "f32"])
+@pytest.mark.parametrize("lens", ["ragged", 1, 4, 31, 32, 33, 64, 67])
+def test_eight_fields_row_lengths(ctx, M, vtype, lens):
+    # rows of every length around the 4 entries of a step and the 32 of a pass,
+    # in plain products and plans; node 0, which padded entries read,
+    # holds a NaN and is no row's column.  An entry's product is rounded once in
+    # its sum, and sums of at most 70 terms lie within 70 ulps of sum |v x|.
+    import rbffd_amd
+
+    print(f"8 fields M={M} {vtype} lens={lens}", flush=True)
+    rng = np.random.default_rng(M)
+    N = 200
+    n = np.resize([0, 1, 3, 4, 5, 31, 32, 33, 36, 63, 64, 65, 70], M) if lens == "ragged" else np.full(M, lens)
+    rowptr = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    col = rng.integers(1, N, rowptr[-1]).astype(np.int32)
+    v = rng.standard_normal(rowptr[-1]).astype(np.float32 if vtype == "f32" else np.float64)
+    x = rng.standard_normal((N, 8))
+    # copied: abs() sums duplicates in place
+    A = sp.csr_matrix((v.astype(np.float64), col, rowptr), shape=(M, N), copy=True)
+    ref, mag = A @ np.where(np.arange(N)[:, None] == 0, 0.0, x), abs(A) @ abs(x)
+    x[0] = np.nan
+    eng = rbffd_amd.Engine(ctx)
+    how = dict(rowptr=ctx.to_device(rowptr)) if lens == "ragged" else dict(uniform_n=int(lens))
+    cd, vd, xd = ctx.to_device(col), ctx.to_device(v), ctx.to_device(x)
+    order = ctx.to_device(rng.permutation(M).astype(np.int32))
+    y = [ctx.empty((M, 8), np.float64) for _ in range(3)]
+    eng.spmv(cd, vd, xd, y[0], **how)
+    eng.spmv(cd, vd, xd, y[1], order=order, **how)
+    plan = eng.spmv_plan(cd, vd, M, N, order=order, **how)
+    plan.apply(xd, y[2])
+    out = [a.get() for a in y]
+    plan.close()
+    assert (np.abs(out[0] - ref) <= 70 * 2.0**-52 * mag).all()
+    assert np.array_equal(out[1], out[0]) and np.array_equal(out[2], out[0])
+
+
 def test_csr_to_csc_matches_sparse(ctx, O):
     X = jittered_grid(60, 50, 0.25, seed=7)
     N, n = len(X), 31
