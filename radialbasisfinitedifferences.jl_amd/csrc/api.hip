@@ -219,9 +219,10 @@ struct Workspace {
     size_t cap = 0, used = 0;
     bool may_alloc = true;
 
+    static size_t padded(size_t bytes) { return ((bytes ? bytes : 16) + 255) & ~(size_t)255; }
     void *take(size_t bytes)
     {
-        const size_t b = ((bytes ? bytes : 16) + 255) & ~(size_t)255;
+        const size_t b = padded(bytes);
         if (b > cap - used)
             throw Error{RBFFD_ERR_ARG, "the call needs more device workspace than the " +
                                            std::to_string(cap >> 20) + " MiB static array holds"};
@@ -544,14 +545,25 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
                     rbffd_buf &redo_buf, const int **ntasks_dev = nullptr)
 {
     const int P = n_monomials(polydeg);
-    const bool ns = precision == RBFFD_PREC_FP64 && rbffd::ns_applies(n, polydeg, p, nops, ops);
+    bool ns = precision == RBFFD_PREC_FP64 && rbffd::ns_applies(n, polydeg, p, nops, ops);
+    const bool may_group = y2x && !rows && precision == RBFFD_PREC_FP64 && M > 1 && grouping_enabled();
+    // its grouping and its list of stencils handed back take workspace that
+    // the pivoting kernels may do without: a static array that does not hold
+    // them keeps those kernels
+    if (ns && w.arena) {
+        size_t need = w.padded(sizeof(int) * (1 + (rows ? nrows : M)));
+        if (may_group)
+            need += 4 * w.padded(sizeof(int) * (N + 1)) + w.padded(sizeof(int) * N) + w.padded(sizeof(int) * 8) +
+                    w.padded(sizeof(int) * M) + w.padded(sizeof(int) * 3 * M) + w.padded(rbffd::group_tmp_bytes(N));
+        if (need > w.room()) ns = false;
+    }
     const int cmax = std::min(rbffd::kMaxRhs, nops);
     if (ntasks_dev) *ntasks_dev = nullptr;
     // ---- group the Y rows by their X node
     int ky = 1;
     int *counts = nullptr, *fill = nullptr;
     bool grp_tuned = tuned_groups(n, P, precision);
-    if (y2x && !rows && precision == RBFFD_PREC_FP64 && M > 1 && grouping_enabled()) {
+    if (may_group) {
         counts = (int *)w.get(S_GRP_COUNTS, sizeof(int) * (N + 1));
         fill = (int *)w.get(S_GRP_FILL, sizeof(int) * N);
         int *flag = (int *)w.get(S_FLAG, sizeof(int) * 8);

@@ -72,6 +72,32 @@ def test_noalloc_matches_weights_device(ctx, O, p, polydeg, n, colloc, size1, si
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("own", [False, True])
+def test_noalloc_null_space_past_the_array(ctx, O, own):
+    # n = 20, degree 3: the null-space solve's workspace is about 40 bytes a row
+    # with y2x (1.9M rows: 76 MB) and 4 without (17M: 68 MB), past the 64 MiB
+    # array; the pivoting kernels need 8 (the largest group is one row) and none.
+    # Every row solves the same stencil: X is a cloud repeated by offset.
+    from rbffd_amd import _lib
+
+    L = _lib.load()
+    na = _fn(L)
+    X0 = jittered_grid(4, 5, 0.25, seed=3)
+    M = 1_900_000 if own else 17_000_000
+    print(f"no-alloc null-space rows={M} y2x={own}", flush=True)
+    if own:
+        X = np.resize(X0, (M, 2))
+        st = np.repeat((np.arange(M) // 20 * 20)[:, None], 20, axis=1) + np.arange(20)
+        Y, y2x = X, np.arange(M)
+    else:
+        X, st = X0, np.tile(np.arange(20, dtype=np.int32), (M, 1))
+        Y, y2x = np.resize(X0, (M, 2)), None
+    col, (v,), status = _call(ctx, na, X, Y, st.astype(np.int32), y2x, 3, 3, ["Lap"])
+    assert not status.any() and np.array_equal(col[-1], st[-1])
+    c1, (v1,), s1 = _call(ctx, L.rbffd_weights_device, X0, X0, st[:20].astype(np.int32) % 20, None, 3, 3, ["Lap"])
+    assert np.abs(v.reshape(-1, 20, 20) - v1).max() <= 1e-9 * np.abs(v1).max()
+
+
 def test_noalloc_refuses_more_than_the_array(ctx, O):
     from rbffd_amd import _lib
 
