@@ -674,7 +674,7 @@ long solves_enqueue(rbffd_context *c, Workspace &w, long N, const double *X, con
                 for (int o = 0; o < cnt; ++o)
                     if (a.op_kind[o] == RBFFD_OP_XK || a.op_kind[o] == RBFFD_OP_YK)
                         rbffd::ns_deriv_constants(p, a.op_k[o], b.xk_c[o]);
-                if (o0 == 0) c->last_group = 16;
+                if (o0 == 0) c->last_group = rbffd::ns_lanes(n, P);
                 rbffd::launch_fill_i32(redo, 1, 0, s);
                 rbffd::launch_ns(b, s);
                 // what it handed back, one row per task

@@ -137,6 +137,12 @@ void ns_deriv_constants(int m, int k, double *c);
 #define RBFFD_DECLARE_NS(nn, pp) void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s);
 RBFFD_NS_SHAPES(RBFFD_DECLARE_NS)
 #undef RBFFD_DECLARE_NS
+// Kernels for the sizes between: P monomials and up to as many nodes as the
+// first number (ns_upto holds the rule).
+#define RBFFD_NS_UPTO_SHAPES(X) X(22, 6) X(26, 10) X(42, 10) X(31, 15) X(47, 15) X(53, 21)
+#define RBFFD_DECLARE_NS_UPTO(nn, pp) void launch_ns_upto_##nn##_##pp(const NsArgs &a, hipStream_t s);
+RBFFD_NS_UPTO_SHAPES(RBFFD_DECLARE_NS_UPTO)
+#undef RBFFD_DECLARE_NS_UPTO
 constexpr bool ns_shape(int n, int P)
 {
 #define RBFFD_CASE(nn, pp) \
@@ -147,6 +153,11 @@ constexpr bool ns_shape(int n, int P)
 }
 // blocks of the pivoting kernel's pass over the rows handed back
 constexpr unsigned kRedoBlocks = 1024;
+// Lanes per stencil: 16 while the stencil's own rows fit one slot per lane,
+// else 32 (with two slots of 16 lanes, four stencils a wavefront hold 36 KB of
+// LDS and all 512 registers at n = 43, one wavefront per SIMD: 3.70 ms per
+// 262,144 stencils).
+constexpr int ns_lanes(int nn, int np) { return np <= 16 && nn - np <= 16 ? 16 : 32; }
 // rows per grouped task of the null-space kernel
 constexpr int kNsRows = 16;
 // Compiled lane-group sizes for a shape: groups[0] default, groups[1..kMaxGroups-1]

@@ -46,6 +46,29 @@ bool solve_tuned(int n, int P, int precision)
     return false;
 }
 
+// Sizes for which no kernel is compiled by itself.  Against the padded
+// eliminations over 160,000 stencils, three operators: 0.35 against 0.75 ms at n =
+// 18 with 6 monomials, 0.48 against 2.84 at 25 with 10, 1.64 against 2.99 at 35
+// with 10, 2.47 against 4.44 at 39 with 15, 3.25 against 20.3 at 51 with 21.
+// Systems of at most 16 equations stay with those (n = 9: 0.25 against 0.43), and
+// with 21 monomials, where 32 lanes share a stencil, those of at most 48 (n = 24:
+// 3.11 against 3.28).  So do m = 3 and polynomials more than one degree above what
+// definiteness asks for: their systems are so well conditioned that the
+// elimination rounds less than this kernel's residual (errors of second
+// derivatives against 64 more bits, m = 3: degree 2 1.28 and degree 3 1.35 times
+// the elimination's; the sizes here: 0.92 to 1.19, mean 1.05, and 0.05 to 0.5 with so
+// few nodes over P that P is nearly singular).
+static bool ns_upto(int n, int P, int polydeg, int m)
+{
+    if (solve_tuned(n, P, 0) || n - P < 3 || n + P <= (P == 21 ? 48 : 16)) return false;
+    if (m < 5 || polydeg > (m + 1) / 2) return false;
+#define RBFFD_CASE(nn, pp) \
+    if (n <= nn && P == pp) return true;
+    RBFFD_NS_UPTO_SHAPES(RBFFD_CASE)
+#undef RBFFD_CASE
+    return false;
+}
+
 // The null-space kernel needs the form definite on the polynomials' complement:
 // odd PHS powers with polynomials of at least degree (m - 1) / 2.  Laplacian^k
 // (per-axis scales inside a double sum) stays with the pivoting kernels, and
@@ -65,7 +88,7 @@ bool ns_applies(int n, int polydeg, int m, int nops, const int *ops)
     if (n == nn && P == pp) return true;
     RBFFD_NS_SHAPES(RBFFD_CASE)
 #undef RBFFD_CASE
-    return false;
+    return ns_upto(n, P, polydeg, m);
 }
 
 void launch_ns(const NsArgs &a, hipStream_t s)
@@ -74,6 +97,10 @@ void launch_ns(const NsArgs &a, hipStream_t s)
 #define RBFFD_CASE(nn, pp) \
     if (a.n == nn && a.P == pp) { launch_ns_##nn##_##pp(a, s); return; }
     RBFFD_NS_SHAPES(RBFFD_CASE)
+#undef RBFFD_CASE
+#define RBFFD_CASE(nn, pp) \
+    if (a.n > pp && a.n <= nn && a.P == pp) { launch_ns_upto_##nn##_##pp(a, s); return; }
+    RBFFD_NS_UPTO_SHAPES(RBFFD_CASE)  // the smallest first
 #undef RBFFD_CASE
     throw Error{3, "null-space solve: no kernel for this shape"};
 }

@@ -36,6 +36,10 @@
 // 1.16 against 1.17 ms with three operators, 1.66 against 1.33 ms with six (its
 // seven unpicked nodes fill less than half of the 16 lanes).
 //
+// GEN: n at run time, up to the compiled size, with the missing nodes' rows of
+// S zero and its pivots not taken; against the eliminations padded to 16, 32, 48
+// .. equations 1.4 to 6.5 times as fast (ns_upto in stencil.hip).
+//
 // What it cannot solve it hands back: a stencil with a zero panel pivot, a
 // pivot of S of the wrong sign or below kNsPivotTol of the largest, or
 // weights that are not finite goes to a list that the pivoting Gauss-Jordan
@@ -558,18 +562,28 @@ __device__ __forceinline__ void fb_sum(double (&a)[RC], const double (&s)[NB][RC
     }
 }
 
-// The same sum in two chains of half the length, added to a at the end: the
-// residual's rounding is what is left of the solve's error
-template <int K1, int RC, int NB, int W>
-__device__ __forceinline__ void fb_sum2(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
+// The same sum in CH chains, added pairwise and then to a: the residual's
+// rounding is what is left of the solve's error
+template <int CH, int K1, int RC, int NB, int W>
+__device__ __forceinline__ void fb_sums(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
 {
-    double h0[RC], h1[RC];
+    double h[CH][RC];
 #pragma unroll
-    for (int o = 0; o < RC; ++o) h0[o] = h1[o] = 0.0;
-    fb_sum<0, K1 / 2>(h0, s, m);
-    fb_sum<K1 / 2, K1>(h1, s, m);
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
-    for (int o = 0; o < RC; ++o) a[o] += h0[o] + h1[o];
+        for (int o = 0; o < RC; ++o) h[c][o] = 0.0;
+    for_blocks<0, CH>([&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+        fb_sum<K1 * c / CH, K1 *(c + 1) / CH>(h[c], s, m);
+    });
+#pragma unroll
+    for (int w = 1; w < CH; w *= 2)
+#pragma unroll
+        for (int c = 0; c + w < CH; c += 2 * w)
+#pragma unroll
+            for (int o = 0; o < RC; ++o) h[c][o] += h[c + w][o];
+#pragma unroll
+    for (int o = 0; o < RC; ++o) a[o] += h[0][o];
 }
 
 __device__ __forceinline__ uint32_t lds_address(const void *p)
@@ -816,6 +830,10 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
     using T = NsShape<NN, NP, G>;
     constexpr int N2 = T::N2, S1 = T::S1, S2 = T::S2, B1 = T::B1, B2 = T::B2, NODES = T::NODES;
     constexpr int DEG = mono_deg(NP - 1);
+    // chains of the residual's sums: the weights' error against an LU solve of
+    // the whole system falls from 1.11 to 1.07 (n = 41, degree 3, m = 5) for 3%
+    // of the time; at the fixed sizes two chains are at or below it
+    constexpr int CH = GEN ? 8 : 2;
     constexpr uint64_t kLane0 = G == 16 ? 0x0001000100010001ull : 0x0000000100000001ull;  // lane 0 of each group
     constexpr uint32_t kGroup = (uint32_t)((1ull << G) - 1);
     __shared__ NsLDS<NN, NP, G> L;
@@ -1354,7 +1372,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         for (int c = 0; c < NP; ++c) f[c] = f21(qh[s], c);
 #pragma unroll
                         for (int o = 0; o < RC; ++o) ra[s][o] = ba[s][o];
-                        fb_sum2<NP>(ra[s], src, f);
+                        fb_sums<CH, NP>(ra[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     for_blocks<0, S1>([&](auto sc) {
@@ -1363,7 +1381,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         for_blocks<0, NP>([&](auto cc) { f[decltype(cc)::value] = f11(LanesG{}, kh[s], sc, cc); });
 #pragma unroll
                         for (int o = 0; o < RC; ++o) rb[s][o] = bb[s][o];
-                        fb_sum2<NP>(rb[s], src, f);
+                        fb_sums<CH, NP>(rb[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 }
@@ -1374,7 +1392,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         constexpr int s = decltype(sc)::value;
                         double f[N2];
                         for_blocks<0, N2>([&](auto jc) { f[decltype(jc)::value] = f22(qh[s], sc, jc); });
-                        fb_sum2<N2>(ra[s], src, f);
+                        fb_sums<CH, N2>(ra[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     });
 #pragma unroll
@@ -1382,7 +1400,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         double f[N2];
 #pragma unroll
                         for (int j = 0; j < N2; ++j) f[j] = f12(kh[s], j);
-                        fb_sum2<N2>(rb[s], src, f);
+                        fb_sums<CH, N2>(rb[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -1390,7 +1408,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                     double src[B1][RC];
                     spread<G>(rb, src);
 #pragma unroll
-                    for (int s = 0; s < S2; ++s) fb_sum2<NP>(ra[s], src, nT[s]);
+                    for (int s = 0; s < S2; ++s) fb_sums<CH, NP>(ra[s], src, nT[s]);
                 }
                 double dn[S2][RC], src[B2][RC];
                 spread<G>(ra, src);
@@ -1452,12 +1470,6 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
     }
 }
 
-// Lanes per stencil: 16 while the stencil's own rows fit one slot per lane,
-// else 32 (with two slots of 16 lanes, four stencils a wavefront hold 36 KB of
-// LDS and all 512 registers at n = 43, one wavefront per SIMD: 3.70 ms per
-// 262,144 stencils).
-constexpr int ns_lanes(int nn, int np) { return np <= 16 && nn - np <= 16 ? 16 : 32; }
-
 // One wavefront per block.
 template <int NN, int NP, int RC, bool GEN>
 void launch_ns_rc(const NsArgs &a, hipStream_t s)
@@ -1475,8 +1487,21 @@ void launch_ns_shape(const NsArgs &a, hipStream_t s)
     else launch_ns_rc<NN, NP, 3, false>(a, s);
 }
 
+// Any n from NP + 1 to NN.
+template <int NN, int NP>
+void launch_ns_upto(const NsArgs &a, hipStream_t s)
+{
+    if (a.nops == 1) launch_ns_rc<NN, NP, 1, true>(a, s);
+    else if (a.nops == 2) launch_ns_rc<NN, NP, 2, true>(a, s);
+    else launch_ns_rc<NN, NP, 3, true>(a, s);
+}
+
 }  // namespace rbffd
 
+#define RBFFD_DEFINE_NS_UPTO(nn, pp) \
+    namespace rbffd {                \
+    void launch_ns_upto_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_upto<nn, pp>(a, s); } \
+    }
 #define RBFFD_DEFINE_NS(nn, pp) \
     namespace rbffd {           \
     void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_shape<nn, pp>(a, s); } \

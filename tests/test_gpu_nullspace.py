@@ -93,3 +93,68 @@ def test_handed_back_rows(ctx, O, p, polydeg, n, nops, monkeypatch):
         assert d.max() <= 1e-9
         bad = status0 != 0
         assert np.array_equal(a[bad], b[bad], equal_nan=True)
+
+
+# sizes between the compiled ones: the edges of each kernel (11..22 nodes with 6
+# monomials, 13..26 and 27..42 with 10, 18..31 and 32..47 with 15, 28..53 with 21)
+BETWEEN = [(5, 2, 11), (5, 2, 22), (5, 3, 13), (5, 3, 26), (5, 3, 27), (7, 3, 42), (7, 4, 18), (7, 4, 30), (7, 4, 32),
+           (9, 4, 47), (9, 5, 28), (9, 5, 53)]
+
+
+@pytest.mark.parametrize("p,polydeg,n", BETWEEN)
+@pytest.mark.parametrize("kind", ["grid", "clustered"])
+def test_sizes_between_against_the_oracle(ctx, O, p, polydeg, n, kind):
+    test_against_the_oracle(ctx, O, p, polydeg, n, kind)
+
+
+# 48, 64 and 96 padded equations in the kernel that takes the rows handed back
+@pytest.mark.parametrize("p,polydeg,n", [(5, 2, 17), (5, 3, 25), (5, 3, 38), (7, 4, 47), (9, 5, 53)])
+@pytest.mark.parametrize("nops", [1, 2, 7])
+def test_sizes_between_handed_back_rows(ctx, O, p, polydeg, n, nops, monkeypatch):
+    test_handed_back_rows(ctx, O, p, polydeg, n, nops, monkeypatch)
+
+
+@pytest.mark.parametrize("p,polydeg,n", [(5, 2, 17), (5, 3, 25), (5, 3, 35), (9, 5, 31)])
+def test_sizes_between_grouped_rows(ctx, O, p, polydeg, n, monkeypatch):
+    """Output rows that share stencils, up to 40 to one (more than a task
+    holds), against the pivoting kernels; one call of single rows gives the bits
+    of the grouped ones."""
+    import rbffd_amd
+
+    X = jittered_grid(17, 15, 0.25, seed=n)
+    rng = np.random.default_rng(n)
+    y2x = np.concatenate([np.full(40, 7), rng.integers(0, len(X), 500)]).astype(np.int32)
+    Y = X[y2x] + rng.uniform(-0.02, 0.02, (len(y2x), 2))
+    st, _ = O.knn(X, X, n)
+    print(f"grouped rows p={p} deg={polydeg} n={n}", flush=True)
+    eng = rbffd_amd.Engine(ctx)
+    Xd, Yd, std = (ctx.to_device(a) for a in (X, Y, st.astype(np.int32)))
+
+    def run():
+        col, vals, status = eng.weights(Xd, Yd, std, ctx.to_device(y2x), p, polydeg, ["Dx", "Lap"], k=0)
+        return col.get(), [v.get() for v in vals], status.get()
+
+    col, vals, status = run()
+    sd, Y1 = ctx.to_device(st[y2x].astype(np.int32)), Yd
+    _, single, _ = eng.weights(Xd, Y1, sd, None, p, polydeg, ["Dx", "Lap"], k=0)
+    single = [v.get() for v in single]
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = run()
+    assert np.array_equal(col, col0) and not status.any() and not status0.any()
+    for a, b, c in zip(vals, vals0, single):
+        assert (np.abs(a - b).max(axis=1) <= 1e-9 * np.abs(b).max(axis=1)).all()
+        assert np.array_equal(a, c)
+
+
+# outside of it: fewer nodes or more than a kernel takes, a degree further above (m - 1) / 2, m = 3, even m
+@pytest.mark.parametrize("p,polydeg,n", [(5, 2, 10), (5, 3, 43), (3, 2, 18), (3, 3, 25), (5, 4, 25), (6, 3, 25), (9, 5, 27), (3, 1, 10)])
+def test_sizes_that_stay(ctx, O, p, polydeg, n, monkeypatch):
+    X = jittered_grid(16, 15, 0.25, seed=n)
+    st, _ = O.knn(X, X, n)
+    print(f"sizes that stay p={p} deg={polydeg} n={n}", flush=True)
+    col, vals, status = _weights(ctx, X, st, p, polydeg, ["Dx", "Lap"], 0)
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = _weights(ctx, X, st, p, polydeg, ["Dx", "Lap"], 0)
+    assert np.array_equal(col, col0) and np.array_equal(status, status0)
+    for a, b in zip(vals, vals0):
+        assert np.array_equal(a, b)
