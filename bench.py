@@ -76,6 +76,16 @@ def read_traffic(name):
     return None
 
 
+def solve_flops(n, P, nops):
+    """Multiply-adds (2 flops each) of one stencil's null-space solve: the panel's
+    elimination, S and its inverse, and per operator the solve and one step of
+    refinement."""
+    n2 = n - P
+    factor = n * P * P + n2 * P * P + 2 * n2 * n2 * P + n2**3
+    per_op = P * P + n * P + n * n + 2 * (2 * n2 * P + n2 * n2)
+    return 2.0 * (factor + nops * per_op)
+
+
 def row_errors(got, ref):
     """max and p99 of the per-row relative error max_j |got - ref| / max_j |ref|."""
     e = np.abs(got - ref).max(axis=1) / np.maximum(np.abs(ref).max(axis=1), 1e-300)
@@ -118,8 +128,7 @@ def main():
     N = len(X)
     Xd = ctx.to_device(X)
     P = (polydeg + 1) * (polydeg + 2) // 2
-    nsys = n + P
-    flops_per_stencil = (2.0 / 3.0) * nsys**3 + 2.0 * nsys**2 * len(OPS)
+    flops_per_stencil = solve_flops(n, P, len(OPS))
 
     def run(precision, steps, warmup, tag, col, vals, st_d):
         stats = None
@@ -340,10 +349,11 @@ def main():
         "config": {"workload": "gen1m: 1,048,576 jittered nodes (1024x1024, +-0.25h, seed 2), PHS r^7, "
                                "degree-4 monomials, n=31, operators Dx, Dy, Lap as FP64 CSR",
                    "nodes": N, "stencil": n, "polydeg": polydeg, "phs_power": p, "ops": OPS},
-        "roofline": {"bound": "valu-fp64", "kernel": f"solve_lu_kernel<31,15,3,{G}>",
+        "roofline": {"bound": "valu-fp64", "kernel": f"solve_ns_kernel<31,15,{G},3>",
+                     "flops_per_stencil": flops_per_stencil,
                      "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64_TFLOPS,
-                     "traffic": read_traffic("solve_lu_gen1m_pmc.txt")},
+                     "traffic": read_traffic("solve_ns_gen1m_pmc.txt")},
         "kernel_only_stencils_per_s": N / (r64["ms_solve"] * 1e-3),
         "ms_knn": r64["ms_knn"], "ms_solve": r64["ms_solve"], "lanes_per_stencil": G,
         "end_to_end": e2e, "accuracy": accuracy,
@@ -405,7 +415,8 @@ def extra_hyper4m(rbffd_amd, ctx, eng, no_cpu):
                                    stencils_out=st)
         ms = ctx.timer_stop()
         nsys = n + 28
-        flops = (2.0 / 3.0) * nsys**3 + 2.0 * nsys**2 * len(ops)
+        # Laplacian^k runs the pivoting elimination, the derivatives the null-space solve
+        flops = (2.0 / 3.0) * nsys**3 + 2.0 * nsys**2 * len(ops) if "Lapk" in ops else solve_flops(n, 28, len(ops))
         res[tag] = {"ms": ms, "stencils_per_s": N / (ms * 1e-3), "ms_solve": stats["ms_solve"],
                     "ms_knn": stats["ms_knn"], "lanes_per_stencil": stats["lanes_per_stencil"],
                     "solve_tflops": N * flops / (stats["ms_solve"] * 1e-3) / 1e12}
@@ -541,10 +552,10 @@ def extra_advdiff(rbffd_amd, ctx, eng, no_cpu):
 def extra_ydistinct(rbffd_amd, ctx, eng, no_cpu):
     """Y distinct from X: X the 1024^2 workload nodes (r^7, degree 4, n = 31),
     Y a 2047^2 jittered grid (4,190,209 rows, about 4 per X node), operators
-    Dx, Dy, Lap: the library's own choice (timed on the first large call),
-    rows grouped by X node (each task's rows solved against one factorisation
-    of its system; an X node with more rows than a task holds takes several),
-    and one factorisation per row."""
+    Dx, Dy, Lap: rows grouped by X node (the default: each task's rows solved
+    against one factorisation; an X node with more rows than a task holds takes
+    several), the same in the pivoting elimination, and one factorisation per
+    row."""
     from rbffd_amd.nodes import config_nodes, jittered_grid
 
     log("extra: Y distinct from X, 1M X nodes, 4.2M Y rows")
@@ -559,7 +570,7 @@ def extra_ydistinct(rbffd_amd, ctx, eng, no_cpu):
     old = os.environ.get("RBFFD_GROUP_ROWS")
     try:
         outs = {}
-        for tag, flag in (("default_choice", None), ("grouped_by_x_node", "1"),
+        for tag, flag in (("grouped_by_x_node", None), ("grouped_pivoting_elimination", "1"),
                           ("one_factorisation_per_row", "0")):
             if flag is None:
                 os.environ.pop("RBFFD_GROUP_ROWS", None)

@@ -56,7 +56,7 @@ extern "C" {
 #define RBFFD_MAX_OPS 10
 
 /* precision of the local solves */
-#define RBFFD_PREC_FP64 0   /* FP64 Gauss-Jordan elimination with partial pivoting */
+#define RBFFD_PREC_FP64 0   /* FP64: null-space solve where it applies, else Gauss-Jordan with partial pivoting */
 #define RBFFD_PREC_MIXED 1  /* experimental: FP32 Gauss-Jordan inverse + FP64 refinement, FP64 re-solve
                                where it does not converge; built for the specialised shapes with
                                n + P <= 64, every other shape solves in FP64 */
@@ -142,8 +142,8 @@ int rbffd_knn_device(rbffd_context *ctx, const double *X, int64_t N, const doubl
  * generate_operator (src/generate_operator.jl:55-166, method 3 :388-467) and
  * hyperviscosity_operator (src/hyperviscosity_operator.jl:66-161).
  * Any stencil size 1 <= n <= 128 and polynomial degree with n + P <= 512
- * (P = (polydeg+1)(polydeg+2)/2); shapes without a specialised kernel run a
- * generic one.  With y2x, the rows that share an X node's stencil are solved
+ * (P = (polydeg+1)(polydeg+2)/2); shapes without a specialised kernel run one
+ * of the next size.  With y2x, the rows that share an X node's stencil are solved
  * against one factorisation of it, as the reference factors each X node once
  * (src/generate_operator.jl:55-65,158); RBFFD_GROUP_ROWS=0 turns this off.
  * method: 1 (also method 2, same numerics) or 3.  ops/opk: nops operator kinds
@@ -168,7 +168,8 @@ int rbffd_weights_device(rbffd_context *ctx, const double *X, int64_t N, const d
  * equations) comes from one fixed 64 MiB array in each GPU's memory, held
  * until the process ends; no layout autotuning runs.  RBFFD_ERR_ARG when a
  * call needs more than the array holds (grouping takes about 20 bytes per X
- * node and 16 per Y row).  Every call on a GPU shares that GPU's array: calls
+ * node and 16 per Y row; where the null-space solve's list, 4 bytes a row, or
+ * its grouping does not fit, the pivoting kernels run instead).  Every call on a GPU shares that GPU's array: calls
  * that overlap on one GPU (two contexts, two threads) race.  Synchronises for
  * the index checks, like rbffd_weights_device. */
 int rbffd_weights_device_noalloc(rbffd_context *ctx, const double *X, int64_t N, const double *Y, int64_t M,
@@ -227,13 +228,13 @@ int rbffd_read_sum_device(rbffd_context *ctx, const double *x, int64_t n, double
  * copies the CSR into blocks of 256 consecutive rows of row_order (NULL: the
  * natural order; a locality order from rbffd_locality_order_device keeps each
  * block a compact patch), lists each block's distinct columns and refers to
- * them by 16-bit local index.  A product then loads a block's x rows into LDS
- * with coalesced loads and reads them there per nonzero, instead of gathering
- * every nonzero's x row from memory.  Arguments as rbffd_spmv_device; results
- * are bitwise equal to it (default lane layout).  The plan takes about 10 B
- * per nonzero with FP64 values (6 with FP32), plus 4 more when a block has
- * over 2048 distinct columns, plus 8 KiB per block, and keeps no pointer to
- * the caller's arrays.  No reference counterpart: the reference's harnesses
+ * them by 16-bit local index.  A product of 1, 2 or 4 fields then loads a
+ * block's x rows into LDS with coalesced loads and reads them there per
+ * nonzero, instead of gathering every nonzero's x row from memory; 8 fields
+ * gather them in the plan's order of rows.  Arguments as rbffd_spmv_device;
+ * results are bitwise equal to it (default lane layout).  The plan takes about
+ * 14 B per nonzero with FP64 values (10 with FP32), plus 8 KiB per block, and
+ * keeps no pointer to the caller's arrays.  No reference counterpart: the reference's harnesses
  * apply one operator many times (examples/adv_diff_test.jl:151-152), and the
  * plan moves the cost of that reuse to one set-up.  Creation synchronises;
  * products are asynchronous.  info (may be NULL) receives the row blocks,
@@ -305,8 +306,7 @@ int rbffd_ssprk3_device(rbffd_context *ctx, int64_t N, const int64_t *rowptr, co
                         double *work, const uint8_t *fixed, double dt, int64_t steps);
 
 /* rbffd_ssprk3_device over an application plan of L (N x N): the stages
- * stage each block's rows of the stage input in LDS as rbffd_spmv_plan_apply
- * does.  Results are bitwise equal to rbffd_ssprk3_device with the plan's
+ * read the stage input as rbffd_spmv_plan_apply does.  Results are bitwise equal to rbffd_ssprk3_device with the plan's
  * operator and row order.  Asynchronous. */
 int rbffd_ssprk3_plan_device(rbffd_context *ctx, const rbffd_spmv_plan *plan, int32_t F, double *u, double *work,
                              const uint8_t *fixed, double dt, int64_t steps);

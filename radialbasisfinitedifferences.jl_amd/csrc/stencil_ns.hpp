@@ -1,5 +1,5 @@
 // stencil_ns.hpp -- K2, FP64 null-space path: batched local RBF-FD solves for
-// conditionally positive definite splines, 16 lanes per stencil.
+// conditionally positive definite splines, 16 or 32 lanes per stencil.
 //
 // Replaces the same hot loops as stencil_lu.hpp (src/generate_operator.jl:55-65,
 // :89-166, method 3 at :388-467; src/hyperviscosity_operator.jl:66-161).
