@@ -40,10 +40,11 @@
 // S zero and its pivots not taken; against the eliminations padded to 16, 32, 48
 // .. equations 1.4 to 6.5 times as fast (ns_upto in stencil.hip).
 //
-// What it cannot solve it hands back: a stencil with a zero panel pivot, a
-// pivot of S of the wrong sign or below kNsPivotTol of the largest, or
-// weights that are not finite goes to a list that the pivoting Gauss-Jordan
-// kernel solves afterwards (which also reports singular systems).
+// What it cannot solve it hands back: a stencil with a panel pivot below
+// kNsPanelTol of its column's size (nodes on which the monomials are dependent
+// up to rounding), a pivot of S of the wrong sign or below kNsPivotTol of the
+// largest, or weights that are not finite goes to a list that the pivoting
+// Gauss-Jordan kernel solves afterwards (which also reports singular systems).
 //
 // A task is one stencil with the output rows that use it (one row, or the
 // grouped rows of an X node): after the factorisation each row's right-hand
@@ -62,6 +63,17 @@ namespace rbffd {
 // error by 1e-2 or better down to 1e-9 and no longer at 1e-10.  Jittered grids
 // reach down to 1e-4 (n = 57) and 7e-3 (n = 13), uniform random nodes to 2e-7.
 constexpr double kNsPivotTol = 9.313225746154785e-10;  // 2^-30
+
+// A panel pivot below this share of the bounding box's value of its monomial
+// sends the stencil to the pivoting kernel.  Monomials that are dependent on a
+// stencil's nodes (as many straight rows of nodes as the degree, along an axis
+// or a diagonal) leave a pivot of rounding instead of zero, at most 3.6e-14 over
+// degrees 2 to 6; T is noise then, and Dx, which such nodes do determine, comes
+// out 8% off in the worst tenth of the rows (four rows of nodes, n = 39, degree
+// 4) where the elimination keeps 4e-11.  From pivots of 1e-13 on the weights are
+// closer to a 113-bit solve than an LU solve's of the whole system (1e-3 against
+// 0.2 there, 1e-6 against 0.1 at 1e-10, level at 1e-3).
+constexpr double kNsPanelTol = 9.094947017729282e-13;  // 2^-40
 
 // ---- multiply-adds with a fused broadcast: lane L of each 16-lane DPP row.
 // A DPP read needs two wait states after a VALU write of its source; the
@@ -755,6 +767,12 @@ __device__ __forceinline__ double lpow(double x, int e)
     return e & 4 ? p * x : p;
 }
 
+// degree of monomial q < 28, per lane (mono_deg's order)
+__device__ __forceinline__ int mono_degree(int q)
+{
+    return (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15) + (q >= 21);
+}
+
 // d^a/dx^a d^b/dy^b of x^ea y^eb (a, b uniform, the exponents per lane)
 __device__ __forceinline__ double ns_mono(int ea, int eb, int a, int b, double x, double y)
 {
@@ -933,7 +951,6 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
     double fin[NODES];
 #pragma unroll
     for (int r = 0; r < NODES; ++r) { pos[r] = 0; fin[r] = 1.0; }
-    uint32_t weakest = 0xFFFFFFFFu;
     const uint32_t ua = lds_address(U);
     for_blocks<0, NP>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
@@ -954,7 +971,6 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
         }
         const double crp = rcp_nr(cv);
         key = group_max_u32<G>(key);
-        weakest = min(weakest, key);
         const int v = 127 - (int)(key & 127u);
         const bool iam = t == v % G;
         // the picked row goes to the group, its reciprocal pivot in the pivot's place
@@ -991,6 +1007,29 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
             fb_lanes<(k + 1 < NP ? k + 2 : k + 1) % NP, NP - 1 - (k + 1 < NP)>(C[r], pr, l[r]);
         __builtin_amdgcn_wave_barrier();
     });
+    // a panel pivot at the rounding of its column (rows not picked hold 1 and pass):
+    // a monomial's value on the bounding box is 1 where the frame is scaled
+    bool bad = false;
+    if (!m3) {  // uniform
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) bad |= !(__builtin_fabs(fin[r]) * kNsPanelTol < 1.0);
+    } else {
+        double mx = 0.0, my = 0.0;
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            mx = fmax(mx, __builtin_fabs(nx[r]));
+            my = fmax(my, __builtin_fabs(nyy[r]));
+        }
+        mx = group_max_nonneg_f64<G>(mx);
+        my = group_max_nonneg_f64<G>(my);
+#pragma unroll
+        for (int r = 0; r < NODES; ++r) {
+            const int d = mono_degree(pos[r]), ea = pos[r] - d * (d + 1) / 2;
+            const double f = __builtin_fabs(fin[r]);
+            // below 2^-120 the float keys of the pivot search lose bits
+            bad |= !(f * (lpow(mx, ea) * lpow(my, d - ea)) * kNsPanelTol < 1.0) || !(f < 0x1p120);
+        }
+    }
     // positions of the rows that were not picked: slot by slot, lane by lane
     {
         int base = NP;
@@ -1262,7 +1301,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
     const double imax = group_max_nonneg_f64<G>(definite ? 1.0 / rmin : 1e300);
     __builtin_amdgcn_sched_barrier(0);
     // the smallest pivot is 1 / rmax, the largest imax
-    bool bad = (weakest & 0x7FFFFF00u) == 0u || !definite || !(kNsPivotTol * imax * rmax < 1.0);
+    bad |= !definite || !(kNsPivotTol * imax * rmax < 1.0);
 
     // ---- the rows' right-hand sides, RC operators at a time
     double gx = a.Y[2 * (long)yk], gy = a.Y[2 * (long)yk + 1];
@@ -1324,8 +1363,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                 rhs_at(kb[s], bb[s]);
                 int q = kb[s];  // the exponents of monomial kb
                 asm volatile("" : "+v"(q));
-                const int d = (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15) + (q >= 21);
-                const int ea = q - d * (d + 1) / 2, eb = d - ea;
+                const int d = mono_degree(q), ea = q - d * (d + 1) / 2, eb = d - ea;
 #pragma unroll
                 for (int o = 0; o < RC; ++o) np[s][o] = -ns_op_mono(kind[o], ord[o], ea, eb, px, py, hx, hy);
             }

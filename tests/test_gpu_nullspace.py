@@ -158,3 +158,42 @@ def test_sizes_that_stay(ctx, O, p, polydeg, n, monkeypatch):
     assert np.array_equal(col, col0) and np.array_equal(status, status0)
     for a, b in zip(vals, vals0):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("p,polydeg,n,lines", [(3, 3, 20, 3), (5, 3, 21, 3), (5, 3, 25, 3), (7, 4, 31, 4), (7, 4, 39, 4),
+                                               (7, 5, 43, 5), (9, 6, 57, 6), (9, 6, 57, 5)])
+@pytest.mark.parametrize("method", [1, 3])
+@pytest.mark.parametrize("diagonal", [False, True])
+def test_dependent_monomials(O, p, polydeg, n, lines, method, diagonal, monkeypatch):
+    """Nodes on at most as many straight lines as the degree (coordinates exact in
+    binary): a polynomial of the basis vanishes on every stencil, so the monomial
+    block is rank deficient up to rounding and each row is the pivoting kernel's,
+    bit for bit.  Dx along the lines is determined all the same.  The eliminations
+    of the sizes between keep it to 2e-11 in the median (the bar: 1e-9; a panel
+    pivot of rounding left 1e-1 in the worst tenth of the rows); those of the
+    compiled sizes, which take the monomials first, do not."""
+    import rbffd_amd
+
+    rng = np.random.default_rng(n + lines)
+    nx = 2 * n
+    x = np.round((np.arange(nx) + rng.uniform(-0.25, 0.25, (lines, nx))) * 2.0**14) / 2.0**20
+    X = np.stack([x, np.broadcast_to(np.arange(lines)[:, None] / 64.0, x.shape)], -1).reshape(-1, 2)
+    if diagonal:
+        X = np.stack([X[:, 0] + X[:, 1], X[:, 1] - X[:, 0]], -1)
+    st, _ = O.knn(X, X, n)
+    ops = ["Dx", "Dxx", "Lap"]
+    print(f"dependent monomials p={p} deg={polydeg} n={n} method={method} diagonal={diagonal}", flush=True)
+    c = rbffd_amd.Context(0)  # no layout chosen by earlier, larger calls
+    col, vals, status = _weights(c, X, st, p, polydeg, ops, 0, method=method)
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = _weights(c, X, st, p, polydeg, ops, 0, method=method)
+    c.close()
+    assert np.array_equal(col, col0) and np.array_equal(status, status0)
+    for a, b in zip(vals, vals0):
+        assert np.array_equal(a, b, equal_nan=True)
+    if method == 1 and not diagonal and n in (25, 39):
+        W, _, _ = O.weights(X, X, st, None, p, polydeg, [(O.OP_NAMES["Dx"], 0)], quad=True)
+        q = np.take_along_axis(W[:, 0], np.argsort(st, axis=1, kind="stable"), 1)
+        ok = (status == 0) & np.isfinite(q).all(axis=1)
+        e = np.abs(vals[0] - q)[ok].max(axis=1) / np.abs(q)[ok].max(axis=1)
+        assert np.quantile(e, 0.9) <= 1e-9
