@@ -47,17 +47,14 @@ bool solve_tuned(int n, int P, int precision)
 }
 
 // Sizes for which no kernel is compiled by itself.  Against the padded
-// eliminations over 160,000 stencils, three operators: 0.35 against 0.75 ms at n =
-// 18 with 6 monomials, 0.48 against 2.84 at 25 with 10, 1.64 against 2.99 at 35
-// with 10, 2.47 against 4.44 at 39 with 15, 3.25 against 20.3 at 51 with 21.
+// eliminations over 160,000 stencils, three operators: 0.37 against 0.74 ms at n =
+// 18 with 6 monomials, 0.50 against 2.78 at 25 with 10, 1.72 against 2.93 at 35
+// with 10, 2.68 against 4.44 at 39 with 15, 3.45 against 20.4 at 51 with 21.
 // Systems of at most 16 equations stay with those (n = 9: 0.25 against 0.43), and
 // with 21 monomials, where 32 lanes share a stencil, those of at most 48 (n = 24:
 // 3.11 against 3.28).  So do m = 3 and polynomials more than one degree above what
-// definiteness asks for: their systems are so well conditioned that the
-// elimination rounds less than this kernel's residual (errors of second
-// derivatives against 64 more bits, m = 3: degree 2 1.28 and degree 3 1.35 times
-// the elimination's; the sizes here: 0.92 to 1.19, mean 1.05, and 0.05 to 0.5 with so
-// few nodes over P that P is nearly singular).
+// definiteness asks for, where the elimination rounds least (1.28 and 1.35 times
+// its errors at m = 3 with the plain residual; not measured with the split one).
 static bool ns_upto(int n, int P, int polydeg, int m)
 {
     if (solve_tuned(n, P, 0) || n - P < 3 || n + P <= (P == 21 ? 48 : 16)) return false;
@@ -84,10 +81,10 @@ bool ns_applies(int n, int polydeg, int m, int nops, const int *ops)
         std::getenv("RBFFD_TUNED_GROUPS") || (g && g[0] == '1'))
         return false;
     const int P = (polydeg + 1) * (polydeg + 2) / 2;
-#define RBFFD_CASE(nn, pp) \
-    if (n == nn && P == pp) return true;
-    RBFFD_NS_SHAPES(RBFFD_CASE)
-#undef RBFFD_CASE
+    // compiled sizes: up to degree m + 2.  Above, rows near a boundary round more
+    // here (against a 113-bit solve 1.37 times the elimination's error at n = 57,
+    // m = 3, degree 6, and 1.34 at n = 31, m = 1, degree 4; 0.9 at m = 3, degree 5)
+    if (ns_shape(n, P)) return polydeg <= m + 2;
     return ns_upto(n, P, polydeg, m);
 }
 

@@ -16,7 +16,9 @@
 // follows; the weights are then as accurate as an LU solve of the whole
 // system (both sit at the rounding of Phi itself: median 7.6e-13 against
 // 7.6e-13 at n = 31, maximum 2.6e-11 against 2.7e-11, over 1,224 stencils
-// against a 113-bit solve; without the step 1.5 to 3 times that).
+// against a 113-bit solve; without the step 1.5 to 3 times that).  Where Phi is
+// so well conditioned that the residual's own rounding shows, its large part is
+// summed exactly (SPLIT).
 //
 // Why: the solve is bound by VALU issue.  Elimination of the whole system
 // takes n + NP dependent steps of pivot search, row publication through LDS
@@ -574,28 +576,63 @@ __device__ __forceinline__ void fb_sum(double (&a)[RC], const double (&s)[NB][RC
     }
 }
 
-// The same sum in CH chains, added pairwise and then to a: the residual's
-// rounding is what is left of the solve's error
-template <int CH, int K1, int RC, int NB, int W>
-__device__ __forceinline__ void fb_sums(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
+// The same sum in two chains: the residual's rounding shows in the weights
+template <int K1, int RC, int NB, int W>
+__device__ __forceinline__ void fb_sum2(double (&a)[RC], const double (&s)[NB][RC], const double (&m)[W])
 {
-    double h[CH][RC];
+    double h[2][RC];
 #pragma unroll
-    for (int c = 0; c < CH; ++c)
+    for (int o = 0; o < RC; ++o) h[0][o] = h[1][o] = 0.0;
+    fb_sum<0, K1 / 2>(h[0], s, m);
+    fb_sum<K1 / 2, K1>(h[1], s, m);
 #pragma unroll
-        for (int o = 0; o < RC; ++o) h[c][o] = 0.0;
-    for_blocks<0, CH>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        fb_sum<K1 * c / CH, K1 *(c + 1) / CH>(h[c], s, m);
-    });
+    for (int o = 0; o < RC; ++o) a[o] += h[0][o] + h[1][o];
+}
+
+// a[o] += sum over i < n of s[o](lane L + i) * m[i]
+template <int L, int RC, int n>
+__device__ __forceinline__ void fb_run(double (&a)[RC], const double (&s)[RC], const double (&m)[n])
+{
+    static_assert(n <= 8, "run");
+    if constexpr (n == 8) fb_dot<L>(a, s, m[0], m[1], m[2], m[3], m[4], m[5], m[6], m[7]);
+    else if constexpr (n == 7) fb_dot<L>(a, s, m[0], m[1], m[2], m[3], m[4], m[5], m[6]);
+    else if constexpr (n == 6) fb_dot<L>(a, s, m[0], m[1], m[2], m[3], m[4], m[5]);
+    else if constexpr (n == 5) fb_dot<L>(a, s, m[0], m[1], m[2], m[3], m[4]);
+    else if constexpr (n == 4) fb_dot<L>(a, s, m[0], m[1], m[2], m[3]);
+    else if constexpr (n == 3) fb_dot<L>(a, s, m[0], m[1], m[2]);
+    else if constexpr (n == 2) fb_dot<L>(a, s, m[0], m[1]);
+    else fb_dot<L>(a, s, m[0]);
+}
+
+// sum over k in K0..K1-1 of (sh + sl)[k / 16][o](lane k % 16) * load(k) in two
+// parts: the products of the upper halves, which a1 adds up without rounding,
+// and the others, 2^-23 of them, in a2.  c splits the loaded factors (split_at).
+template <int K0, int K1, int RC, int NB, class Load>
+__device__ __forceinline__ void fb_sum_split(double (&a1)[RC], double (&a2)[RC], const double (&sh)[NB][RC],
+                                             const double (&sl)[NB][RC], double c, Load &&load)
+{
+    if constexpr (K1 > K0) {
+        constexpr int l = K0 % 16, left = K1 - K0 < 16 - l ? K1 - K0 : 16 - l, n = left < 8 ? left : 8;
+        double f[n], h[n];
+        for_blocks<0, n>([&](auto ic) { f[decltype(ic)::value] = load(std::integral_constant<int, K0 + decltype(ic)::value>{}); });
+        fb_run<l>(a2, sl[K0 / 16], f);
 #pragma unroll
-    for (int w = 1; w < CH; w *= 2)
-#pragma unroll
-        for (int c = 0; c + w < CH; c += 2 * w)
-#pragma unroll
-            for (int o = 0; o < RC; ++o) h[c][o] += h[c + w][o];
-#pragma unroll
-    for (int o = 0; o < RC; ++o) a[o] += h[0][o];
+        for (int i = 0; i < n; ++i) {
+            h[i] = (f[i] + c) - c;
+            f[i] -= h[i];
+        }
+        fb_run<l>(a1, sh[K0 / 16], h);
+        fb_run<l>(a2, sh[K0 / 16], f);
+        fb_sum_split<K0 + n, K1>(a1, a2, sh, sl, c, load);
+    }
+}
+
+// (v + split_at(e)) - split_at(e) is v rounded to a multiple of 2^(e - 23), for
+// |v| <= 2^e.  Products of two such halves are multiples of 2^(e + e' - 46) of at
+// most 2^(e + e'), so sums of up to 64 of them are exact in 53 bits.
+__device__ __forceinline__ double split_at(int e)
+{
+    return __longlong_as_double((long long)((uint64_t)(uint32_t)(1023 + 29 + e) << 52 | 0x0008000000000000ull));
 }
 
 __device__ __forceinline__ uint32_t lds_address(const void *p)
@@ -674,6 +711,12 @@ __device__ __forceinline__ void spread(const double (&own)[S][RC], double (&src)
 #pragma unroll
         for (int i = 0; i < R; ++i) src[i][o] = b[i];
     }
+}
+
+// the high word of |v|
+__device__ __forceinline__ uint32_t high_abs(double v)
+{
+    return (uint32_t)((uint64_t)__double_as_longlong(v) >> 32) & 0x7FFFFFFFu;
 }
 
 // 1 / x to within an ulp (x finite and not zero): the instruction gives 23
@@ -801,6 +844,16 @@ __device__ __forceinline__ double ns_op_mono(int op, int k, int ea, int eb, doub
     return ns_mono(ea, eb, a, b, x, y);
 }
 
+// Fixed sizes that take the split residual (fb_sum_split): low powers with
+// polynomials more than one degree above what definiteness asks for.  Errors
+// against a 113-bit solve relative to the elimination's (geometric mean of a
+// row's, second derivatives): with the plain residual 1.2 at (m, degree) = (3, 4),
+// 1.1 at (3, 5), 1.05 at (5, 4) and (5, 5), at most 0.99 from m = 7 on and at
+// (5, 3); with the split one 0.87, 0.74 at m = 3.  It takes 4% (n = 57) to 29%
+// (n = 20) of the solve.  The kernels with n at run time always take it: 1.05
+// without, 0.97 with it, for 2 to 8% of their time.
+constexpr bool ns_split(int polydeg, int m) { return m <= 5 && polydeg > (m + 1) / 2; }
+
 template <int NN, int NP, int G>
 struct NsShape {
     static constexpr int N2 = NN - NP;
@@ -825,33 +878,34 @@ struct alignas(16) NsLDS {
     using T = NsShape<NN, NP, G>;
     double u[T::S][T::U];       // the panel's pivot row, then P1^-1 and T, then Phi
     double xi[T::S][2 * NN];    // scaled coordinates by position
-    double frame[T::S][4];      // centre and scales
+    double frame[T::S][5];      // centre and scales, the splitting constant of Phi (split_at)
     int g[T::S][NN], rank[T::S][NN];  // global index and output column by position
 };
 
 // Wavefronts per SIMD the kernel is compiled for.  n = 31: LDS (20 KB a
 // wavefront) and the row registers hold it to two.  n = 20 and 21: three, with
 // 30 registers spilled, take 2.00 ms per 1M stencils of n = 21 where two
-// without spills take 2.29 ms.
-template <int NN, int NP, int G>
+// without spills take 2.29 ms; with the split residual, which spills 102 there,
+// two take 0.40 against 0.48 ms per 160,000 stencils of n = 20.  n = 42 and 43:
+// two, with 75 registers spilled at three operators (127 split), one without
+// spills 2.79 against 2.06 ms split; the kernel for up to 42 nodes and 10
+// monomials spills 119 and takes 1.72 ms at n = 35 where one wavefront takes 2.29.
+template <int NN, int NP, int G, bool SPLIT>
 constexpr int ns_min_waves()
 {
     if (G == 32) return NN <= 43 ? 2 : 1;
-    return NN <= 21 ? 3 : 2;
+    return NN <= 21 && !SPLIT ? 3 : 2;
 }
 
 // NN nodes (GEN: at most NN, a.n of them), NP monomials, G lanes per stencil,
-// RC operators at a time
-template <int NN, int NP, int G, int RC, bool GEN>
-__global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kernel(const NsArgs a)
+// RC operators at a time, SPLIT: the refinement's residual without rounding in
+// its large part
+template <int NN, int NP, int G, int RC, bool GEN, bool SPLIT>
+__global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G, SPLIT>())) void solve_ns_kernel(const NsArgs a)
 {
     using T = NsShape<NN, NP, G>;
     constexpr int N2 = T::N2, S1 = T::S1, S2 = T::S2, B1 = T::B1, B2 = T::B2, NODES = T::NODES;
     constexpr int DEG = mono_deg(NP - 1);
-    // chains of the residual's sums: the weights' error against an LU solve of
-    // the whole system falls from 1.11 to 1.07 (n = 41, degree 3, m = 5) for 3%
-    // of the time; at the fixed sizes two chains are at or below it
-    constexpr int CH = GEN ? 8 : 2;
     constexpr uint64_t kLane0 = G == 16 ? 0x0001000100010001ull : 0x0000000100000001ull;  // lane 0 of each group
     constexpr uint32_t kGroup = (uint32_t)((1ull << G) - 1);
     __shared__ NsLDS<NN, NP, G> L;
@@ -1011,6 +1065,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
     // a monomial's value on the bounding box is 1 where the frame is scaled
     bool bad = false;
     if (!m3) {  // uniform
+        if (SPLIT && t == 0) L.frame[grp][4] = split_at((3 * m + 1) / 2);  // r^2 at most 8
 #pragma unroll
         for (int r = 0; r < NODES; ++r) bad |= !(__builtin_fabs(fin[r]) * kNsPanelTol < 1.0);
     } else {
@@ -1022,6 +1077,10 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
         }
         mx = group_max_nonneg_f64<G>(mx);
         my = group_max_nonneg_f64<G>(my);
+        if (SPLIT && t == 0) {
+            const int q = (int)((uint64_t)__double_as_longlong(4.0 * sq_sum(mx, my)) >> 52) - 1022;  // r^2 < 2^q
+            L.frame[grp][4] = split_at(min(max((q * m + 1) >> 1, -1000), 900));
+        }
 #pragma unroll
         for (int r = 0; r < NODES; ++r) {
             const int d = mono_degree(pos[r]), ea = pos[r] - d * (d + 1) / 2;
@@ -1400,7 +1459,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                     qh[s] = qa[s];
                     asm volatile("" : "+v"(qh[s]));
                 }
-                {
+                if (!SPLIT || !it) {
                     double src[B1][RC];
                     spread<G>(w1n, src);
 #pragma unroll
@@ -1410,7 +1469,7 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         for (int c = 0; c < NP; ++c) f[c] = f21(qh[s], c);
 #pragma unroll
                         for (int o = 0; o < RC; ++o) ra[s][o] = ba[s][o];
-                        fb_sums<CH, NP>(ra[s], src, f);
+                        fb_sum2<NP>(ra[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     for_blocks<0, S1>([&](auto sc) {
@@ -1419,34 +1478,108 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
                         for_blocks<0, NP>([&](auto cc) { f[decltype(cc)::value] = f11(LanesG{}, kh[s], sc, cc); });
 #pragma unroll
                         for (int o = 0; o < RC; ++o) rb[s][o] = bb[s][o];
-                        fb_sums<CH, NP>(rb[s], src, f);
+                        fb_sum2<NP>(rb[s], src, f);
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 }
-                if (it) {
-                    double src[B2][RC];
-                    spread<G>(w2n, src);
-                    for_blocks<0, S2>([&](auto sc) {
-                        constexpr int s = decltype(sc)::value;
-                        double f[N2];
-                        for_blocks<0, N2>([&](auto jc) { f[decltype(jc)::value] = f22(qh[s], sc, jc); });
-                        fb_sums<CH, N2>(ra[s], src, f);
-                        __builtin_amdgcn_sched_barrier(0);
-                    });
+                if constexpr (!SPLIT) {
+                    if (it) {
+                        double src[B2][RC];
+                        spread<G>(w2n, src);
+                        for_blocks<0, S2>([&](auto sc) {
+                            constexpr int s = decltype(sc)::value;
+                            double f[N2];
+                            for_blocks<0, N2>([&](auto jc) { f[decltype(jc)::value] = f22(qh[s], sc, jc); });
+                            fb_sum2<N2>(ra[s], src, f);
+                            __builtin_amdgcn_sched_barrier(0);
+                        });
 #pragma unroll
-                    for (int s = 0; s < S1; ++s) {
-                        double f[N2];
+                        for (int s = 0; s < S1; ++s) {
+                            double f[N2];
 #pragma unroll
-                        for (int j = 0; j < N2; ++j) f[j] = f12(kh[s], j);
-                        fb_sums<CH, N2>(rb[s], src, f);
-                        __builtin_amdgcn_sched_barrier(0);
+                            for (int j = 0; j < N2; ++j) f[j] = f12(kh[s], j);
+                            fb_sum2<N2>(rb[s], src, f);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                } else if (it) {
+                    // b - Phi w in halves: the upper ones' products sum exactly
+                    double a1[S2][RC], a2[S2][RC], b1[S1][RC], b2[S1][RC], cw[RC];
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) {
+                        uint32_t h = 0;
+#pragma unroll
+                        for (int s = 0; s < S1; ++s) h = max(h, high_abs(w1n[s][o]));
+#pragma unroll
+                        for (int s = 0; s < S2; ++s) h = max(h, high_abs(w2n[s][o]));
+                        h = group_max_u32<G>(h);
+                        // split_at of the largest weight's exponent
+                        cw[o] = __longlong_as_double((long long)((uint64_t)((h & 0x7FF00000u) + 0x01E80000u) << 32));
+#pragma unroll
+                        for (int s = 0; s < S2; ++s) a1[s][o] = a2[s][o] = 0.0;
+#pragma unroll
+                        for (int s = 0; s < S1; ++s) b1[s][o] = b2[s][o] = 0.0;
+                    }
+                    int fp = 0;
+                    asm volatile("" : "+v"(fp));
+                    const double cp = L.frame[grp][4 + fp];
+                    {
+                        double hi[S1][RC], lo[S1][RC], sh[B1][RC], sl[B1][RC];
+#pragma unroll
+                        for (int s = 0; s < S1; ++s)
+#pragma unroll
+                            for (int o = 0; o < RC; ++o) {
+                                hi[s][o] = (w1n[s][o] + cw[o]) - cw[o];
+                                lo[s][o] = w1n[s][o] - hi[s][o];
+                            }
+                        spread<G>(hi, sh);
+                        spread<G>(lo, sl);
+#pragma unroll
+                        for (int s = 0; s < S2; ++s) {
+                            fb_sum_split<0, NP>(a1[s], a2[s], sh, sl, cp, [&](auto cc) { return f21(qh[s], decltype(cc)::value); });
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        for_blocks<0, S1>([&](auto sc) {
+                            constexpr int s = decltype(sc)::value;
+                            fb_sum_split<0, NP>(b1[s], b2[s], sh, sl, cp, [&](auto cc) { return f11(LanesG{}, kh[s], sc, cc); });
+                            __builtin_amdgcn_sched_barrier(0);
+                        });
+                    }
+                    {
+                        double hi[S2][RC], lo[S2][RC], sh[B2][RC], sl[B2][RC];
+#pragma unroll
+                        for (int s = 0; s < S2; ++s)
+#pragma unroll
+                            for (int o = 0; o < RC; ++o) {
+                                hi[s][o] = (w2n[s][o] + cw[o]) - cw[o];
+                                lo[s][o] = w2n[s][o] - hi[s][o];
+                            }
+                        spread<G>(hi, sh);
+                        spread<G>(lo, sl);
+                        for_blocks<0, S2>([&](auto sc) {
+                            constexpr int s = decltype(sc)::value;
+                            fb_sum_split<0, N2>(a1[s], a2[s], sh, sl, cp, [&](auto jc) { return f22(qh[s], sc, jc); });
+                            __builtin_amdgcn_sched_barrier(0);
+                        });
+#pragma unroll
+                        for (int s = 0; s < S1; ++s) {
+                            fb_sum_split<0, N2>(b1[s], b2[s], sh, sl, cp, [&](auto jc) { return f12(kh[s], decltype(jc)::value); });
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+#pragma unroll
+                    for (int o = 0; o < RC; ++o) {
+#pragma unroll
+                        for (int s = 0; s < S2; ++s) ra[s][o] = (ba[s][o] + a1[s][o]) + a2[s][o];
+#pragma unroll
+                        for (int s = 0; s < S1; ++s) rb[s][o] = (bb[s][o] + b1[s][o]) + b2[s][o];
                     }
                 }
                 {
                     double src[B1][RC];
                     spread<G>(rb, src);
 #pragma unroll
-                    for (int s = 0; s < S2; ++s) fb_sums<CH, NP>(ra[s], src, nT[s]);
+                    for (int s = 0; s < S2; ++s) fb_sum2<NP>(ra[s], src, nT[s]);
                 }
                 double dn[S2][RC], src[B2][RC];
                 spread<G>(ra, src);
@@ -1509,38 +1642,33 @@ __global__ __launch_bounds__(64, (ns_min_waves<NN, NP, G>())) void solve_ns_kern
 }
 
 // One wavefront per block.
-template <int NN, int NP, int RC, bool GEN>
+template <int NN, int NP, int RC, bool GEN, bool SPLIT>
 void launch_ns_rc(const NsArgs &a, hipStream_t s)
 {
     constexpr int G = ns_lanes(NN, NP);
     const unsigned nb = (unsigned)((a.ntasks + 64 / G - 1) / (64 / G));
-    solve_ns_kernel<NN, NP, G, RC, GEN><<<nb, 64, 0, s>>>(a);
+    solve_ns_kernel<NN, NP, G, RC, GEN, SPLIT><<<nb, 64, 0, s>>>(a);
 }
 
-template <int NN, int NP>
+template <int NN, int NP, bool GEN, bool SPLIT>
 void launch_ns_shape(const NsArgs &a, hipStream_t s)
 {
-    if (a.nops == 1) launch_ns_rc<NN, NP, 1, false>(a, s);
-    else if (a.nops == 2) launch_ns_rc<NN, NP, 2, false>(a, s);
-    else launch_ns_rc<NN, NP, 3, false>(a, s);
-}
-
-// Any n from NP + 1 to NN.
-template <int NN, int NP>
-void launch_ns_upto(const NsArgs &a, hipStream_t s)
-{
-    if (a.nops == 1) launch_ns_rc<NN, NP, 1, true>(a, s);
-    else if (a.nops == 2) launch_ns_rc<NN, NP, 2, true>(a, s);
-    else launch_ns_rc<NN, NP, 3, true>(a, s);
+    if (a.nops == 1) launch_ns_rc<NN, NP, 1, GEN, SPLIT>(a, s);
+    else if (a.nops == 2) launch_ns_rc<NN, NP, 2, GEN, SPLIT>(a, s);
+    else launch_ns_rc<NN, NP, 3, GEN, SPLIT>(a, s);
 }
 
 }  // namespace rbffd
 
 #define RBFFD_DEFINE_NS_UPTO(nn, pp) \
     namespace rbffd {                \
-    void launch_ns_upto_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_upto<nn, pp>(a, s); } \
+    void launch_ns_upto_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_shape<nn, pp, true, true>(a, s); } \
     }
 #define RBFFD_DEFINE_NS(nn, pp) \
     namespace rbffd {           \
-    void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s) { launch_ns_shape<nn, pp>(a, s); } \
+    void launch_ns_##nn##_##pp(const NsArgs &a, hipStream_t s)              \
+    {                                                                       \
+        if (ns_split(mono_deg(pp - 1), a.m)) launch_ns_shape<nn, pp, false, true>(a, s); \
+        else launch_ns_shape<nn, pp, false, false>(a, s);                   \
+    }                                                                       \
     }
