@@ -670,6 +670,15 @@ __device__ __forceinline__ bool upto(int c)
     return __builtin_amdgcn_inverse_ballot_w64(m * (G == 16 ? 0x0001000100010001ull : 0x0000000100000001ull));
 }
 
+// A lane swap needs two wait states after a VALU write of its sources, which the
+// compiler provides for its own writes only: a value that may come from an asm
+// block passes through here first.
+__device__ __forceinline__ double settled(double v)
+{
+    asm("s_nop 1" : "+v"(v));
+    return v;
+}
+
 // Per-lane rows as broadcast sources: src[b] holds, in every 16-lane DPP row of
 // a group, rows 16 b .. 16 b + 15.  With 16 lanes these are the lane's own row
 // slots; with 32, v_permlane16_swap gives both halves to both DPP rows.
@@ -682,7 +691,7 @@ __device__ __forceinline__ void spread(const double (&own)[S], double (&src)[R])
         for (int b = 0; b < R; ++b) src[b] = own[b];
     } else {
         static_assert(S == 1 && R <= 2, "row slots");
-        const uint64_t v = (uint64_t)__double_as_longlong(own[0]);
+        const uint64_t v = (uint64_t)__double_as_longlong(settled(own[0]));
         const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
         const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
 #pragma unroll
@@ -693,6 +702,7 @@ __device__ __forceinline__ void spread(const double (&own)[S], double (&src)[R])
 // x's odd 16-lane rows exchanged with y's even ones (v_permlane16_swap)
 __device__ __forceinline__ void swap_rows(double x, double y, double &p, double &q)
 {
+    asm("s_nop 1" : "+v"(x), "+v"(y));  // as settled
     const uint64_t a = (uint64_t)__double_as_longlong(x), b = (uint64_t)__double_as_longlong(y);
     const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)a, (uint32_t)b, false, false);
     const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(a >> 32), (uint32_t)(b >> 32), false, false);
