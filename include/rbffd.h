@@ -233,8 +233,9 @@ int rbffd_read_sum_device(rbffd_context *ctx, const double *x, int64_t n, double
  * nonzero, instead of gathering every nonzero's x row from memory; 8 fields
  * gather them in the plan's order of rows.  Arguments as rbffd_spmv_device;
  * results are bitwise equal to it (default lane layout).  The plan takes about
- * 14 B per nonzero with FP64 values (10 with FP32), plus 8 KiB per block, and
- * keeps no pointer to the caller's arrays.  No reference counterpart: the reference's harnesses
+ * 10 B per nonzero with FP64 values (6 with FP32), plus 4 more when a block has
+ * over 2048 distinct columns, plus 8 KiB per block, and keeps no pointer to the
+ * caller's arrays.  No reference counterpart: the reference's harnesses
  * apply one operator many times (examples/adv_diff_test.jl:151-152), and the
  * plan moves the cost of that reuse to one set-up.  Creation synchronises;
  * products are asynchronous.  info (may be NULL) receives the row blocks,

@@ -256,7 +256,7 @@ struct SpmvPlan {
     int *prow = nullptr;      // plan row -> operator row
     int64_t *pptr = nullptr;  // M + 1, the rows in plan order
     uint16_t *plc = nullptr;  // nnz local column indices
-    int *pcol = nullptr;      // nnz columns (8 fields, and blocks past the cap)
+    int *pcol = nullptr;      // nnz columns; kept only when some block overflows
     void *pval = nullptr;     // nnz values (FP64 or FP32), plan order
     int *halo = nullptr;      // nblocks x kPlanHaloCap
     int *hcount = nullptr;    // nblocks (+ 2 scratch)

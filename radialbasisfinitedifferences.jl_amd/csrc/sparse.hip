@@ -243,25 +243,14 @@ static void spmm_split_launch_t(long M, const int64_t *rowptr, const int *col, c
         spmm_split_kernel<TV, F, FL, false><<<blocks, 256, 0, s>>>(M, rowptr, col, val, nu, order, x, y, alpha, beta);
 }
 
-// 8 fields, 16 lanes a row (row_times_8).  MODE 0: y = alpha A x + beta y;
-// MODE 1: one Shu-Osher stage y = a u + b x + c (A x), rows with fixed[r] != 0
-// keeping u (y may be u: the same lane reads and writes a value).
-struct RowsOut {
-    double *y;
-    double alpha, beta;
-    const double *u;
-    const uint8_t *fixed;
-    double a, b, c;
-};
-
+// 8 fields, 16 lanes a row (row_times_8).  MODE: as RowsOut.
 template <typename TV, bool UNIFORM, int MODE>
 __global__ __launch_bounds__(256) void spmm_rows_kernel(long M, const int64_t *__restrict__ rowptr,
                                                         const int *__restrict__ col, const TV *__restrict__ val,
                                                         int n_uniform, const int *__restrict__ order,
                                                         const double *__restrict__ x, RowsOut o)
 {
-    constexpr int F = 8;
-    const int sub = threadIdx.x & 15, f0 = 2 * (sub & 3);
+    const int sub = threadIdx.x & 15;
     const long g = blockIdx.x * 16L + (threadIdx.x >> 4);
     // rows past the end still take part in the broadcasts
     const bool live = g < M;
@@ -282,22 +271,8 @@ __global__ __launch_bounds__(256) void spmm_rows_kernel(long M, const int64_t *_
         rows_extent(len, most, full);
     }
     double acc[2];
-    row_times_8(acc, val + p0, col + p0, len, most, full, x);
-    if (live && sub < 4) {
-        const long e = row * F + f0;
-        const bool hold = MODE == 1 && o.fixed && o.fixed[row];
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-            if constexpr (MODE == 0) {
-                double r = o.alpha * acc[f];
-                if (o.beta != 0.0) r = __builtin_fma(o.beta, o.y[e + f], r);
-                o.y[e + f] = r;
-            } else {
-                const double ui = o.u[e + f];
-                o.y[e + f] = hold ? ui : o.a * ui + o.b * x[e + f] + o.c * acc[f];
-            }
-        }
-    }
+    row_times_8(acc, val + p0, col + p0, len, most, full, x, [](int c) { return c; });
+    if (live && sub < 4) put_row_8<MODE>(o, row, acc, x);
 }
 
 template <typename TV, int MODE>

@@ -43,16 +43,16 @@ __device__ __forceinline__ void for_steps(Fn &&f)
 }
 
 // A row's entries b .. b + 31, 16 a load, entry b + j in lane j % 16, register j /
-// 16; zeros past the row's end.  (Two entries a lane, in one load each of columns
-// and values, took 5 us more a million rows of 31: most of those loads start off
-// their width.)
+// 16; zeros past the row's end.  c: the column, or its place in a plan's list.
+// (Two entries a lane, in one load each of columns and values, took 5 us more a
+// million rows of 31: most of those loads start off their width.)
 struct RowEntries {
     int c[2];
     double v[2];
 };
 
-template <typename TV>
-__device__ __forceinline__ RowEntries row_entries(const TV *val, const int *col, int len, int b)
+template <typename TV, typename TC>
+__device__ __forceinline__ RowEntries row_entries(const TV *val, const TC *col, int len, int b)
 {
     RowEntries e;
 #pragma unroll
@@ -61,7 +61,7 @@ __device__ __forceinline__ RowEntries row_entries(const TV *val, const int *col,
         e.c[r] = 0;
         e.v[r] = 0.0;
         if (j < len) {
-            e.c[r] = col[j];
+            e.c[r] = (int)col[j];
             e.v[r] = (double)val[j];
         }
     }
@@ -76,11 +76,11 @@ __device__ __forceinline__ void rows_extent(int len, int &most, bool &full)
     full = __builtin_amdgcn_ballot_w64(len == most) == ~0ull;
 }
 
-// acc = the sum over j < len of val[j] x(col[j]) for this lane's two fields, 2
+// acc = the sum over j < len of val[j] x(at(col[j])) for this lane's two fields, 2
 // (lane % 4) and the next, in every quad of the row's 16 lanes.  val, col: the
 // row's entries; len: its length (0 for a group without a row); most, full: as
 // rows_extent (most may exceed every len); x: node 0's row.  Padded entries read
-// node 0 where the wavefront has any entry, and are dropped whatever it holds.
+// node at(0) where the wavefront has any entry, and are dropped whatever it holds.
 //
 // Loads are bound by the address unit, which takes a quad of lanes a cycle
 // whatever they carry (at 8 bytes a lane it was busy 92% of 196 us over a million
@@ -90,16 +90,18 @@ __device__ __forceinline__ void rows_extent(int len, int &most, bool &full)
 // bytes and a column and a value loaded by each.  All gathers of up to 32
 // entries are in flight together: two or four rows a lane group were slower.
 // Quad k sums entries k, k + 4, ... in order; the quads are added by rotations.
-template <typename TV>
-__device__ __forceinline__ void row_times_8(double (&acc)[2], const TV *val, const int *col, int len, int most,
-                                            bool full, const double *x)
+template <typename TV, typename TC, class At>
+__device__ __forceinline__ void row_times_8(double (&acc)[2], const TV *val, const TC *col, int len, int most,
+                                            bool full, const double *x, At &&at)
 {
     constexpr int STEPS = 8;
     const int quad = (threadIdx.x & 15) / 4;
     const double *const xf = x + 2 * (threadIdx.x & 3);
     acc[0] = acc[1] = 0.0;
     for (int b = 0; b < most; b += 32) {
-        const RowEntries e = row_entries(val, col, len, b);
+        RowEntries e = row_entries(val, col, len, b);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) e.c[r] = at(e.c[r]);
         // one path for the loads of padded entries and real ones: with two,
         // every gather would wait for the one before
         double xv[STEPS][2];
@@ -130,6 +132,36 @@ __device__ __forceinline__ void row_times_8(double (&acc)[2], const TV *val, con
     for (int f = 0; f < 2; ++f) {
         acc[f] += dpp_f64<0x120 | 4>(acc[f]);  // row_ror
         acc[f] += dpp_f64<0x120 | 8>(acc[f]);
+    }
+}
+
+// What becomes of a row's sum.  MODE 0: y = alpha A x + beta y; MODE 1: one
+// Shu-Osher stage y = a u + b x + c (A x), rows with fixed[r] != 0 keeping u (y may
+// be u: the same lane reads and writes a value).
+struct RowsOut {
+    double *y;
+    double alpha, beta;
+    const double *u;
+    const uint8_t *fixed;
+    double a, b, c;
+};
+
+// the two fields of a row of 8 that this lane holds (the first quad's lanes)
+template <int MODE>
+__device__ __forceinline__ void put_row_8(const RowsOut &o, long row, const double (&acc)[2], const double *x)
+{
+    const long e = row * 8 + 2 * (threadIdx.x & 3);
+    const bool hold = MODE == 1 && o.fixed && o.fixed[row];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        if constexpr (MODE == 0) {
+            double r = o.alpha * acc[f];
+            if (o.beta != 0.0) r = __builtin_fma(o.beta, o.y[e + f], r);
+            o.y[e + f] = r;
+        } else {
+            const double ui = o.u[e + f];
+            o.y[e + f] = hold ? ui : o.a * ui + o.b * x[e + f] + o.c * acc[f];
+        }
     }
 }
 

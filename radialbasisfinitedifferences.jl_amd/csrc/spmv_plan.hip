@@ -4,7 +4,8 @@
 // The plain kernels (sparse.hip) gather a node's fields from L1/L2 once per
 // nonzero and are bound by the L1's address path, not by HBM.  Up to 4 fields a
 // plan takes x from LDS instead; 8 fields run in the plan's order of rows with x
-// gathered as the plain product does (plan_rows_kernel).
+// gathered as the plain product does, by columns from the blocks' lists
+// (plan_rows_kernel).
 //
 // A plan cuts the rows, in a locality order (Morton order of the rows' nodes
 // for RBF-FD operators), into blocks of kPlanRows consecutive rows and lists
@@ -36,6 +37,8 @@ namespace rbffd {
 
 namespace {
 
+constexpr int kPlanListedRows = 64;           // rows of a workgroup that reads its block's column list
+static_assert(kPlanRows % kPlanListedRows == 0 && kPlanListedRows % 16 == 0, "whole passes");
 constexpr int kHashSlots = 2 * kPlanHaloCap;  // open addressing, load factor <= 1/2
 
 __global__ void plan_rowlen_kernel(long M, const int64_t *__restrict__ rowptr, int nu, const int *__restrict__ order,
@@ -166,15 +169,7 @@ __global__ void max_le_kernel(const int *__restrict__ v, int n, int cap, int *__
     if (i < n && v[i] > cap) atomicAdd(out + 1, 1);
 }
 
-// Epilogues: MODE 0 y = alpha acc (+ beta y); MODE 1 one SSP-RK stage,
-// out = a u + b w + c acc (rows with fixed != 0 keep u).
-struct PlanOut {
-    double *y;
-    double alpha, beta;
-    const double *u;
-    const uint8_t *fixed;
-    double a, b, c;
-};
+using PlanOut = RowsOut;  // what becomes of a row's sum (MODE 0: a product, 1: an SSP-RK stage)
 
 // LDS stride of a staged x row, in doubles: F + 2 from 2 fields up, so rows
 // that a wavefront reads at once spread over the banks (at a stride of F
@@ -328,53 +323,50 @@ __global__ __launch_bounds__(NT) void plan_apply_kernel(long M, int nu, const in
     }
 }
 
-// 8 fields: the rows by row_times_8, x gathered through the columns as the plain
-// product does.  Over a million rows of 31 in turn with two lanes a nonzero and
-// x in LDS (a halo of about 450 nodes staged for 256 rows, then one barrier): 144
-// us against 158, FP32 values 140 against 149; 57 entries a row, FP32, 230 against
-// 229.  The same sum from LDS took 203, and through 16-bit slots of the halo's
-// list 187.  Three RK stages of four million rows: 2.18 ms against 2.90, FP32 2.14
-// against 2.71.
-template <typename TV, bool UNIFORM, int MODE>
-__global__ __launch_bounds__(256) void plan_rows_kernel(long M, int nu, const int *__restrict__ prow,
-                                                        const int64_t *__restrict__ pptr,
-                                                        const int *__restrict__ pcol, const TV *__restrict__ pval,
-                                                        const double *__restrict__ x, PlanOut o)
+// 8 fields: the rows by row_times_8.  LISTED: a workgroup takes its block's column
+// list into LDS, and its rows' 16-bit places give the columns to gather x by; a
+// plan with a block past the lists gathers through its columns, as the plain
+// product does, at the same speed.  Over a million rows of 31 in turn with two
+// lanes a nonzero and x itself in LDS: 142 us against 158, FP32 values 136 against
+// 148; 13 entries 94 against 105, 57 entries, FP32, 232 against 230.  Three RK
+// stages of four million rows: 2.20 ms against 2.90.  64 rows and 256 lanes a
+// workgroup: 256 rows 153 (512 lanes 145), 32 rows 150, one pass of 512 lanes 147,
+// of 1024 lanes 173; the row sums from x in LDS 203, the places through the list in
+// memory 187.
+template <typename TV, bool UNIFORM, int MODE, bool LISTED>
+__global__ __launch_bounds__(256, 8) void plan_rows_kernel(long M, int nu, const int *__restrict__ prow,
+                                                           const int64_t *__restrict__ pptr,
+                                                           const std::conditional_t<LISTED, uint16_t, int> *__restrict__ idx,
+                                                           const TV *__restrict__ pval, const int *__restrict__ halo,
+                                                           const int *__restrict__ hcount,
+                                                           const double *__restrict__ x, PlanOut o)
 {
-    constexpr int F = 8;
-    const int sub = threadIdx.x & 15, f0 = 2 * (sub & 3);
-    const long i = blockIdx.x * 16L + (threadIdx.x >> 4);
-    const bool live = i < M;
-    long p0 = 0, row = 0;
-    int len = 0, most;
-    bool full;
-    if (live) {
-        p0 = UNIFORM ? i * (long)nu : pptr[i];
-        len = UNIFORM ? nu : (int)(pptr[i + 1] - p0);
-        row = prow[i];
+    constexpr int ROWS = LISTED ? kPlanListedRows : 16;  // of this workgroup
+    __shared__ int list[LISTED ? kPlanHaloCap : 1];
+    const int grp = threadIdx.x >> 4;
+    const long r0 = blockIdx.x * (long)ROWS;
+    if constexpr (LISTED) {
+        const long block = r0 / kPlanRows;
+        const int H = hcount[block];  // at most kPlanHaloCap: a plan with longer lists keeps its columns
+        for (int h = threadIdx.x; h < H; h += 256) list[h] = halo[block * kPlanHaloCap + h];
+        __syncthreads();
     }
-    if (UNIFORM) {
-        most = nu;
-        full = __builtin_amdgcn_ballot_w64(live) == ~0ull;
-    } else {
-        rows_extent(len, most, full);
-    }
-    double acc[2];
-    row_times_8(acc, pval + p0, pcol + p0, len, most, full, x);
-    if (live && sub < 4) {
-        const long e = row * F + f0;
-        const bool hold = MODE == 1 && o.fixed && o.fixed[row];
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-            if constexpr (MODE == 0) {
-                double t = o.alpha * acc[f];
-                if (o.beta != 0.0) t = __builtin_fma(o.beta, o.y[e + f], t);
-                o.y[e + f] = t;
-            } else {
-                const double ui = o.u[e + f];
-                o.y[e + f] = hold ? ui : o.a * ui + o.b * x[e + f] + o.c * acc[f];
-            }
+    for (int k = 0; k < ROWS; k += 16) {  // every group runs every pass
+        const long i = r0 + k + grp;
+        const bool live = i < M;
+        long p0 = 0, row = 0;
+        int len = 0, most = nu;
+        bool full;
+        if (live) {
+            p0 = UNIFORM ? i * (long)nu : pptr[i];
+            len = UNIFORM ? nu : (int)(pptr[i + 1] - p0);
+            row = prow[i];
         }
+        if (UNIFORM) full = __builtin_amdgcn_ballot_w64(live) == ~0ull;
+        else rows_extent(len, most, full);
+        double acc[2];
+        row_times_8(acc, pval + p0, idx + p0, len, most, full, x, [&](int c) { return LISTED ? list[c] : c; });
+        if (live && (threadIdx.x & 15) < 4) put_row_8<MODE>(o, row, acc, x);
     }
 }
 
@@ -382,13 +374,16 @@ template <typename TV, int F, int MODE>
 void plan_apply_t(const SpmvPlan &P, const double *x, const PlanOut &o, hipStream_t s)
 {
     if constexpr (F == 8) {
-        const unsigned blocks = (unsigned)((P.M + 15) / 16);
-        auto go = [&](auto un) {
-            plan_rows_kernel<TV, decltype(un)::value, MODE>
-                <<<blocks, 256, 0, s>>>(P.M, P.uniform, P.prow, P.pptr, P.pcol, (const TV *)P.pval, x, o);
+        auto go = [&](auto un, auto listed, const auto *idx) {
+            constexpr bool LISTED = decltype(listed)::value;
+            const long rows = LISTED ? kPlanListedRows : 16;
+            plan_rows_kernel<TV, decltype(un)::value, MODE, LISTED><<<(unsigned)((P.M + rows - 1) / rows), 256, 0, s>>>(
+                P.M, P.uniform, P.prow, P.pptr, idx, (const TV *)P.pval, P.halo, P.hcount, x, o);
         };
-        if (P.uniform > 0) go(std::true_type{});
-        else go(std::false_type{});
+        if (P.pcol && P.uniform > 0) go(std::true_type{}, std::false_type{}, P.pcol);
+        else if (P.pcol) go(std::false_type{}, std::false_type{}, P.pcol);
+        else if (P.uniform > 0) go(std::true_type{}, std::true_type{}, P.plc);
+        else go(std::false_type{}, std::true_type{}, P.plc);
     } else {
         constexpr int FL = F == 4 ? 2 : 1, SX = plan_lds_stride<F>();
         // LDS for the largest listed halo, at most 64 KiB a workgroup
@@ -488,6 +483,10 @@ void spmv_plan_build(SpmvPlan &P, long M, long N, const int64_t *rowptr, const i
         RBFFD_HIP(hipStreamSynchronize(s));
         P.hmax = h[0];
         P.overflow_blocks = h[1];
+        if (P.overflow_blocks == 0) {  // every block reads x through its halo list
+            (void)hipFree(P.pcol);
+            P.pcol = nullptr;
+        }
     } catch (...) {
         spmv_plan_free(P);
         throw;

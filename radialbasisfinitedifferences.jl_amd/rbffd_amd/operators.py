@@ -433,8 +433,8 @@ class SpmvPlan:
     """An application plan of one CSR operator (rbffd_spmv_plan_create): the
     rows in blocks of 256 of `order` (a locality order such as
     Engine.locality_order of the rows' nodes), each block's distinct columns
-    listed, so a product stages a block's x rows in LDS.  Products equal
-    Engine.spmv bit for bit.  `info`: row blocks, largest listed halo, blocks
+    listed, so a product of up to 4 fields stages a block's x rows in LDS.
+    Products equal Engine.spmv bit for bit.  `info`: row blocks, largest listed halo, blocks
     over 2048 distinct columns, nonzeros.  The plan keeps no reference to the
     arrays it was made from."""
 

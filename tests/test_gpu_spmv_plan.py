@@ -153,3 +153,34 @@ def test_plan_errors_and_empty(ctx):
     empty.close()
     plan.close()
     plan.close()
+
+
+@pytest.mark.parametrize("vtype,per_entry", [("f64", 10), ("f32", 6)])
+def test_plan_memory(ctx, vtype, per_entry):
+    """A plan whose blocks all fit their lists holds its values and 16-bit places
+    (10 or 6 bytes a nonzero), 8 KiB a block and 12 bytes a row: no 4-byte columns,
+    which would be 47 MiB more here.  Allocations come in pieces of 2 MiB."""
+    import ctypes
+
+    import rbffd_amd
+    from rbffd_amd import _lib
+
+    N, n = 400_000, 31
+    col = np.clip(np.arange(N)[:, None] + np.arange(n) - 15, 0, N - 1).astype(np.int32)
+    eng = rbffd_amd.Engine(ctx)
+    cd = ctx.to_device(col)
+    vd = ctx.to_device(np.ones((N, n), np.float64 if vtype == "f64" else np.float32))
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _lib.load().hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0  # of the HIP runtime it links
+        return f.value
+
+    ctx.synchronize()
+    before = free()
+    plan = eng.spmv_plan(cd, vd, N, N, uniform_n=n)
+    used = before - free()
+    print(f"plan memory {vtype}: {used / 2**20:.1f} MiB, {plan.info}", flush=True)
+    assert plan.info["overflow_blocks"] == 0
+    assert used <= per_entry * N * n + 8192 * plan.info["blocks"] + 12 * N + (14 << 20)
+    plan.close()
