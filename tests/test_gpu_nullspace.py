@@ -229,3 +229,45 @@ def test_rounding_against_the_elimination(ctx, O, p, polydeg, n, monkeypatch):
 
     print(f"p={p} deg={polydeg} n={n}: {err(vals):.2e}, elimination {err(vals0):.2e}", flush=True)
     assert err(vals) <= 1.015 * err(vals0)
+
+
+@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31), (3, 5, 42), (9, 6, 57), (5, 3, 25), (5, 3, 35), (9, 5, 47)])
+@pytest.mark.parametrize("gap", [1e-9, 1e-11, 3e-13])
+def test_near_duplicates_are_handed_back(O, p, polydeg, n, gap, monkeypatch):
+    """Two nodes a small part of the spacing apart leave a pivot of S of about
+    gap^m of the largest, far below the threshold: every row whose stencil holds
+    both gets the pivoting kernel's bits.  Elsewhere the null-space solve ran: its
+    rounding differs from that kernel's in nearly every row."""
+    import rbffd_amd
+
+    X = jittered_grid(24, 22, 0.25, seed=n)
+    at = [150, 300, 410]
+    X = np.concatenate([X, X[at] + gap / 23 * np.array([[1, 0], [0, 1], [0.6, -0.8]])])
+    st, _ = O.knn(X, X, n)
+    near = np.zeros(len(X), bool)
+    for i, k in enumerate(at):
+        near |= (st == k).any(axis=1) & (st == len(X) - 3 + i).any(axis=1)
+    print(f"near duplicates p={p} deg={polydeg} n={n} gap={gap}: {near.sum()} rows", flush=True)
+    c = rbffd_amd.Context(0)  # no layout chosen by earlier, larger calls
+    ops = ["Dx", "Dyy", "Lap"]
+    col, vals, status = _weights(c, X, st, p, polydeg, ops, 0)
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = _weights(c, X, st, p, polydeg, ops, 0)
+    c.close()
+    assert np.array_equal(col, col0) and np.array_equal(status, status0)
+    assert near.sum() >= n
+    for a, b in zip(vals, vals0):
+        assert np.array_equal(a[near], b[near], equal_nan=True)
+        assert (a != b).any(axis=1)[~near].mean() > 0.9
+
+
+# low powers with high degrees: the split residual
+@pytest.mark.parametrize("p,polydeg,n", [(1, 3, 20), (3, 4, 31), (5, 4, 31), (3, 5, 42), (3, 5, 43), (5, 6, 57)])
+@pytest.mark.parametrize("kind", ["grid", "uniform", "clustered"])
+def test_high_degrees_against_the_oracle(ctx, O, p, polydeg, n, kind):
+    test_against_the_oracle(ctx, O, p, polydeg, n, kind)
+
+
+@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31), (3, 5, 42), (7, 5, 43), (9, 6, 57)])
+def test_compiled_sizes_grouped_rows(ctx, O, p, polydeg, n, monkeypatch):
+    test_sizes_between_grouped_rows(ctx, O, p, polydeg, n, monkeypatch)
