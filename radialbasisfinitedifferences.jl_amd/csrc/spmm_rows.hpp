@@ -83,8 +83,8 @@ __device__ __forceinline__ void rows_extent(int len, int &most, bool &full)
 // node at(0) where the wavefront has any entry, and are dropped whatever it holds.
 //
 // Loads are bound by the address unit, which takes a quad of lanes a cycle
-// whatever they carry (at 8 bytes a lane it was busy 92% of 196 us over a million
-// rows, n = 31).  So an entry's 64 bytes of x go to one quad, 16 bytes a lane,
+// whatever they carry (with two lanes of 32 bytes it was busy 87% of 185 us over a
+// million rows, n = 31, and is 88% of 134 now).  So an entry's 64 bytes of x go to one quad, 16 bytes a lane,
 // and columns and values come in once, 16 entries a load, and DPP broadcasts
 // hand entry j to its quad: 1.5 cycles an entry against 2 with two lanes of 32
 // bytes and a column and a value loaded by each.  All gathers of up to 32

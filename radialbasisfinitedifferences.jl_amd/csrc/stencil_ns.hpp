@@ -28,15 +28,15 @@
 // row_newbcast: one instruction per multiply-add, no LDS), since lane k of a
 // group holds row k.  About half the multiply-adds remain.
 //
-// Measured, 1M stencils, three operators, against the Gauss-Jordan kernel:
-// n = 31 3.41 against 6.87 ms, n = 21 2.00 against 3.97 ms; six operators at
-// n = 20 2.54 against 4.42 ms; 262,144 stencils of n = 31 with 1M output rows
-// 1.95 against 4.36 ms.  A wavefront of four stencils issues 4,880 VALU
-// instructions at n = 31 (8,440 there), on 66% of its SIMD's cycles; the rest
-// are waits on the panel's LDS round trips and on dependent steps of S^-1 that
-// two wavefronts per SIMD do not cover.  n = 13 stays with the elimination:
-// 1.16 against 1.17 ms with three operators, 1.66 against 1.33 ms with six (its
-// seven unpicked nodes fill less than half of the 16 lanes).
+// Measured, whole weights calls on 1M stencils, three operators, against the
+// Gauss-Jordan kernel: n = 31 3.34 against 7.03 ms, n = 21 2.26 against 4.07 ms;
+// six operators at n = 20 2.69 against 4.52 ms (m = 3, SPLIT: 3.34); 262,144
+// stencils of n = 31 with 1M output rows 2.08 against 4.51 ms.  A wavefront of four
+// stencils issues 4,961 VALU instructions at n = 31 (8,440 there), on 70% of its
+// SIMD's cycles; the rest are waits on the panel's LDS round trips and on dependent
+// steps of S^-1 that two wavefronts per SIMD do not cover.  n = 13 stays with the
+// elimination: 1.16 against 1.17 ms with three operators, 1.66 against 1.33 ms with
+// six (its seven unpicked nodes fill less than half of the 16 lanes).
 //
 // GEN: n at run time, up to the compiled size, with the missing nodes' rows of
 // S zero and its pivots not taken; against the eliminations padded to 16, 32, 48
@@ -738,9 +738,10 @@ __device__ __forceinline__ double rcp_nr(double x)
     return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// sqrt(x) for x >= 2^-700 by the correction steps the compiler uses, without
-// its scaling of smaller arguments (7 instructions fewer); x = 0 gives NaN, so
-// a duplicated node fails the finiteness check
+// sqrt(x) for x >= 2^-700: Goldschmidt's coupled iteration from the 1 / sqrt(x)
+// estimate (g -> sqrt(x), h -> 1 / (2 sqrt(x))), then two steps on the residual
+// x - g^2.  Smaller arguments are not scaled first (7 instructions fewer); x = 0
+// gives NaN, so a duplicated node fails the finiteness check
 __device__ __forceinline__ double ns_sqrt(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -894,12 +895,14 @@ struct alignas(16) NsLDS {
 
 // Wavefronts per SIMD the kernel is compiled for.  n = 31: LDS (20 KB a
 // wavefront) and the row registers hold it to two.  n = 20 and 21: three, with
-// 30 registers spilled, take 2.00 ms per 1M stencils of n = 21 where two
+// 26 and 35 registers spilled, take 2.00 ms per 1M stencils of n = 21 where two
 // without spills take 2.29 ms; with the split residual, which spills 102 there,
 // two take 0.40 against 0.48 ms per 160,000 stencils of n = 20.  n = 42 and 43:
-// two, with 75 registers spilled at three operators (127 split), one without
-// spills 2.79 against 2.06 ms split; the kernel for up to 42 nodes and 10
-// monomials spills 119 and takes 1.72 ms at n = 35 where one wavefront takes 2.29.
+// two, with 75 and 70 registers spilled at three operators (127 and 134 split), one
+// without spills 2.79 against 2.06 ms split; the kernel for up to 42 nodes and 10
+// monomials spills 135 and takes 1.72 ms at n = 35 where one wavefront takes 2.29.
+// n = 31 spills 39 with the split residual, the kernels with n at run time for up to
+// 26 and 31 nodes 15 and 42; the others none.
 template <int NN, int NP, int G, bool SPLIT>
 constexpr int ns_min_waves()
 {
