@@ -271,3 +271,26 @@ def test_high_degrees_against_the_oracle(ctx, O, p, polydeg, n, kind):
 @pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31), (3, 5, 42), (7, 5, 43), (9, 6, 57)])
 def test_compiled_sizes_grouped_rows(ctx, O, p, polydeg, n, monkeypatch):
     test_sizes_between_grouped_rows(ctx, O, p, polydeg, n, monkeypatch)
+
+
+@pytest.mark.parametrize("p,polydeg,n", [(3, 3, 20), (7, 4, 31), (7, 5, 43), (9, 6, 57), (5, 3, 25), (5, 3, 35)])
+@pytest.mark.parametrize("unit", [2.0**-8, 1.0, 2.0**11])
+def test_unscaled_frames(O, p, polydeg, n, unit, monkeypatch):
+    """Method 3 solves in the nodes' own unit: the null-space solve runs whatever
+    that is (its bits are not the pivoting kernel's in nearly every row), and the
+    two agree to a few times the rounding of an FP64 solve at this conditioning
+    (9e-9 at n = 57)."""
+    import rbffd_amd
+
+    X = unit * jittered_grid(23, 21, 0.25, seed=n)
+    st, _ = O.knn(X, X, n)
+    print(f"unscaled frames p={p} deg={polydeg} n={n} unit={unit}", flush=True)
+    c = rbffd_amd.Context(0)  # no layout chosen by earlier, larger calls
+    col, vals, status = _weights(c, X, st, p, polydeg, ["Dx", "Lap"], 0, method=3)
+    monkeypatch.setenv("RBFFD_NULLSPACE", "0")
+    col0, vals0, status0 = _weights(c, X, st, p, polydeg, ["Dx", "Lap"], 0, method=3)
+    c.close()
+    assert np.array_equal(col, col0) and not status.any() and not status0.any()
+    for a, b in zip(vals, vals0):
+        assert (a != b).any(axis=1).mean() > 0.9
+        assert (np.abs(a - b).max(axis=1) <= (2e-8 if n == 57 else 1e-9) * np.abs(b).max(axis=1)).all()
